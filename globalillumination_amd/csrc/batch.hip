@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kClipThreads) void kb_clip(RasterTable t) {
         const int j = find_job(pre, t.njobs, item);
         const RasterJob& J = t.jobs[j];
         const uint32_t local = item - pre[j];
-        clip_body(J.mesh, mvp_of(J), J.cfg, J.b, (int)(local % kClipBlocks), kClipBlocks, (int)(local / kClipBlocks));
+        clip_body<0>(J.mesh, mvp_of(J), J.cfg, J.b, (int)(local % kClipBlocks), kClipBlocks, (int)(local / kClipBlocks));
     }
 }
 

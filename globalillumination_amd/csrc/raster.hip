@@ -64,7 +64,10 @@ int bin_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, const Rast
     dim3 gw(kWideBlocks, nmaps);
     if (mesh.nt > 0) {
         hipLaunchKernelGGL((k_bin<kTile, false>), gb, dim3(256), 0, s, mesh, mvps, cfg, b);
-        hipLaunchKernelGGL(k_clip, dim3(kClipBlocks, nmaps), dim3(kClipThreads), 0, s, mesh, mvps, cfg, b);
+        if (b.attrs)
+            hipLaunchKernelGGL(k_clip<6>, dim3(kClipBlocks, nmaps), dim3(kClipThreads), 0, s, mesh, mvps, cfg, b);
+        else
+            hipLaunchKernelGGL(k_clip<0>, dim3(kClipBlocks, nmaps), dim3(kClipThreads), 0, s, mesh, mvps, cfg, b);
         hipLaunchKernelGGL((k_bin_wide<kTile, false>), gw, dim3(256), 0, s, cfg, b);
     }
     hipLaunchKernelGGL(k_scan, dim3(nmaps), dim3(kScanThreads), 0, s, b, ntiles);
@@ -246,10 +249,14 @@ int gi_gbuffer_pass(const float* positions_dev, const float* normals_dev, int nv
     RasterCfg cfg{width, height, (width + kTile - 1) / kTile, (height + kTile - 1) / kTile, 0.0f, 0.0f};
     int rc = run_raster<true>(mesh, mvps, 1, cfg, ws, ws.vis, s);
     if (rc != GI_OK) return rc;
-    size_t npx = (size_t)width * height;
-    hipLaunchKernelGGL(k_gbuffer_resolve, dim3((unsigned)((npx + 255) / 256)), dim3(256), 0, s, mesh, mvps.single,
-                       cfg, reinterpret_cast<const unsigned long long*>(ws.vis), position_out_dev, normal_out_dev,
+    hipLaunchKernelGGL(k_gbuffer_resolve, dim3((unsigned)((width + 63) / 64), (unsigned)((height + 3) / 4)),
+                       dim3(256), 0, s, mesh, mvps.single, cfg, ws.bins,
+                       reinterpret_cast<const unsigned long long*>(ws.vis), position_out_dev, normal_out_dev,
                        facing_out_dev);
+    if ((uint32_t)ntris > ws.bins.acap)
+        hipLaunchKernelGGL(k_gbuffer_resolve_rest, dim3(256), dim3(256), 0, s, mesh, mvps.single, cfg, ws.bins,
+                           reinterpret_cast<const unsigned long long*>(ws.vis), position_out_dev, normal_out_dev,
+                           facing_out_dev);
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
 
