@@ -230,9 +230,9 @@ __global__ void kb_overflow_any(RasterTable t, uint32_t* __restrict__ flag) {
 }
 
 // (instance, map, tile) items from a work queue: tiles differ widely in cost.
-template <int TS>
-__global__ __launch_bounds__(kRasterThreads) void kb_raster(RasterTable t) {
-    __shared__ __align__(16) uint32_t tile[TS * TS];
+template <int TS, bool kBig>
+__global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_raster(RasterTable t) {
+    __shared__ __align__(16) uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     __shared__ uint32_t s_item;
@@ -249,13 +249,13 @@ __global__ __launch_bounds__(kRasterThreads) void kb_raster(RasterTable t) {
         const uint32_t local = item - pre[j];
         const int map = (int)(local / J.ntiles), tile_id = (int)(local % J.ntiles);
         if (J.b.overflow[map]) continue;  // left to kb_raster_fallback
-        raster_tile<TS, false, false>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec);
+        raster_tile<TS, false, false, kBig>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, false);
     }
 }
 
 template <int TS>
 __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable t) {
-    __shared__ uint32_t tile[TS * TS];
+    __shared__ uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     if (t.counter[1] == 0u) return;  // no map overflowed (kb_scan)
@@ -267,7 +267,8 @@ __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable
         const int tile_id = (int)(item - pre[j]);
         for (int map = 0; map < J.nmaps; ++map) {
             if (!J.b.overflow[map]) continue;
-            raster_tile<TS, false, true>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec);
+            raster_tile<TS, false, true, true>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec,
+                                               true);
             __syncthreads();
         }
     }
@@ -394,6 +395,7 @@ struct gi_batch {
     SoftGroup sg[kShapes][kNtGroups];
     uint32_t* counters;
     char* ws;  // the workspace: every job's binning buffers lie in it
+    bool big;  // some map is a big_view
 };
 
 struct gi_batch_graph {
@@ -423,6 +425,14 @@ void launch_scatter(const RasterVariant& R, const RasterTable& tab, char* ws, un
     }
 }
 
+template <int TS>
+void launch_raster(unsigned grid, const RasterTable& tab, bool big, hipStream_t s) {
+    if (big)
+        hipLaunchKernelGGL((kb_raster<TS, true>), dim3(grid), dim3(kRasterThreads), 0, s, tab);
+    else
+        hipLaunchKernelGGL((kb_raster<TS, false>), dim3(grid), dim3(kRasterThreads), 0, s, tab);
+}
+
 int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
     const int v = T.tile == 32 ? 0 : 1;
     const RasterVariant& R = b->rv[v];
@@ -442,7 +452,7 @@ int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
     if ((g = grid_of(R.total[kStWide], cap)))                                                                       \
         hipLaunchKernelGGL((kb_bin_wide<TS, true>), dim3(g), dim3(256), 0, s, tab);                                 \
     if ((g = grid_of(R.total[kStRaster], cap)))                                                                     \
-        hipLaunchKernelGGL((kb_raster<TS>), dim3(g), dim3(kRasterThreads), 0, s, tab);                              \
+        launch_raster<TS>(g, tab, b->big, s);                                                                       \
     if ((g = grid_of(R.total[kStFallback], cap)))                                                                   \
         hipLaunchKernelGGL((kb_raster_fallback<TS>), dim3(g), dim3(kRasterThreads), 0, s, tab);
     if (T.tile == 32) {
@@ -571,6 +581,7 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
     b->tuning = gi_batch_tuning{64, 4, 3, 4};
     b->counters = reinterpret_cast<uint32_t*>(base + L.counters);
     b->ws = base;
+    b->big = false;
     for (int v = 0; v < 2; ++v) {
         const int ts = kTiles[v];
         RasterJob* jobs = reinterpret_cast<RasterJob*>(img.data() + L.rjobs[v]);
@@ -585,6 +596,7 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
             J.mvps = I.light_mvps_dev;
             J.cfg = RasterCfg{I.sm_width, I.sm_height, (I.sm_width + ts - 1) / ts, (I.sm_height + ts - 1) / ts,
                               I.polygon_offset_factor, I.polygon_offset_units};
+            b->big = b->big || big_view(J.cfg);
             J.b = ws.bins;
             J.out = I.maps_dev;
             J.nzero = (uint32_t)zero_words(I.nsamples, J.cfg);

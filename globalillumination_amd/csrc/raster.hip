@@ -49,6 +49,9 @@ namespace gi {
 // ---------------------------------------------------------------------------
 namespace {
 
+// Tiles of a launch up to which every workgroup is resident at once.
+constexpr size_t kSpreadTiles = 2048;
+
 // Binning of every map (count, clip, scan, scatter) and the raster of the
 // maps whose lists overflowed the workspace.
 template <bool kVis>
@@ -96,8 +99,14 @@ int raster_stage(const MeshView& mesh, const MvpSource& mvps, int map_begin, int
                  hipEvent_t ev_end = nullptr) {
     const int ntiles = cfg.tiles_x * cfg.tiles_y;
     if (ev_begin && hipEventRecord(ev_begin, s) != hipSuccess) return GI_EDEVICE;
-    hipLaunchKernelGGL((k_raster<kTile, kVis>), dim3((unsigned)(ntiles * map_count)), dim3(kRasterThreads), 0, s, mesh,
-                       mvps, cfg, ws.bins, out, map_begin, map_count);
+    const dim3 grid((unsigned)(ntiles * map_count));
+    const bool spread = ntiles * (size_t)map_count <= kSpreadTiles;
+    if (big_view(cfg))
+        hipLaunchKernelGGL((k_raster<kTile, kVis, true>), grid, dim3(kRasterThreads), 0, s, mesh, mvps, cfg, ws.bins,
+                           out, map_begin, map_count, spread);
+    else
+        hipLaunchKernelGGL((k_raster<kTile, kVis, false>), grid, dim3(kRasterThreads), 0, s, mesh, mvps, cfg, ws.bins,
+                           out, map_begin, map_count, spread);
     if (ev_end && hipEventRecord(ev_end, s) != hipSuccess) return GI_EDEVICE;
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }

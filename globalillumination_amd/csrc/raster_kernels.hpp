@@ -24,19 +24,14 @@ constexpr int kTile = 64;
 constexpr int kRasterThreads = 256;
 constexpr float kGuard = 4.0f;
 constexpr int kMaxPoly = 9;
-// Launch-shape constants; a build may override them (-DGI_SELF_RASTER_MAX_PX=...).
-#ifndef GI_SELF_RASTER_MAX_PX
-#define GI_SELF_RASTER_MAX_PX 256
-#endif
-// 63 setup records (64 B each) beside the 16 KiB tile and the record count
-// keep a workgroup's LDS at 20,420 bytes, so 8 workgroups fit in a CU's
-// 160 KiB (64 records made it 20,484 bytes: 7 workgroups, k_raster 3% slower).
-#ifndef GI_REC_QUEUE
-#define GI_REC_QUEUE 63
-#endif
-constexpr int kSelfRasterMaxPx = GI_SELF_RASTER_MAX_PX;  // bbox∩tile area a lone thread rasterizes itself
+// 28 setup records (64 B each) beside the 18 KiB tile and the record count
+// keep a workgroup's LDS at 20,228 bytes, so 8 workgroups fit in a CU's
+// 160 KiB (7 of 20,484 bytes ran 3% slower).
+constexpr int kRecQueue = 28;  // LDS setup records that a workgroup puts aside
+constexpr int kShareList = 128;   // entries up to which a tile's list counts as short
+constexpr int kShareBlocks = 16;      // blocks over which a record of a short list is put aside
+constexpr int kShareBlocksLong = 44;  // and of a long one
 constexpr int kScanThreads = 1024;
-constexpr int kRecQueue = GI_REC_QUEUE;  // LDS setup records a workgroup rasterizes together per chunk
 
 struct MeshView {
     const float* __restrict__ pos;  // nverts x 3
@@ -336,45 +331,59 @@ __device__ __forceinline__ Setup to_setup(const Tri<NA>& t, uint32_t id) {
     return s;
 }
 
-// The count pass's record of a directly binned triangle, 48 bytes: the list
-// entry supplies the id, and the tie bits follow from the edges.  Pixel
-// bounds fit 16 bits (map edges are at most GI_MAX_EDGE).
+// The count pass's record of a directly binned triangle, 32 bytes: the list
+// entry supplies the id, the tie bits and the pixel box follow from the
+// vertices, and vertices 1 and 2 are kept as 16-bit offsets from vertex 0
+// (rec_fits; a triangle with a longer edge becomes a wide record).  The
+// records are the raster's and the count pass's largest traffic after the
+// maps themselves; with 48 bytes (32-bit coordinates, packed box) 289 maps of
+// a 50,002-triangle mesh took 206 us in the count pass and 450 us in the
+// raster, with 32 bytes 187 and 401 us (64 maps of 2048^2 and 100,822
+// triangles, whose count pass is bound by its arithmetic: raster 326 and 306).
 struct alignas(16) SetupRec {
-    int X[3], Y[3];
+    int X0, Y0;
+    uint32_t d1, d2;  // (X - X0) | (Y - Y0) << 16 of vertices 1 and 2
     float z0, A, B, zoff;
-    uint32_t bx, by;  // px0 | px1 << 16, py0 | py1 << 16
 };
-static_assert(sizeof(SetupRec) == 48, "three 16-byte loads");
-static_assert(GI_MAX_EDGE <= 65536, "pixel bounds are packed in 16 bits");
+static_assert(sizeof(SetupRec) == 32, "two 16-byte loads");
+// Workspace bytes reserved per directly binned triangle and map.
+constexpr size_t kRecStride = 48;
+static_assert(sizeof(SetupRec) <= kRecStride, "the workspace's record area");
+
+// Every vertex within 127 pixels of vertex 0.
+__device__ __forceinline__ bool rec_fits(const Tri<0>& t) {
+    const int dx1 = t.X[1] - t.X[0], dx2 = t.X[2] - t.X[0], dy1 = t.Y[1] - t.Y[0], dy2 = t.Y[2] - t.Y[0];
+    return max(max(abs(dx1), abs(dx2)), max(abs(dy1), abs(dy2))) < 32768;
+}
 
 __device__ __forceinline__ SetupRec to_rec(const Tri<0>& t) {
     SetupRec r;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        r.X[i] = t.X[i];
-        r.Y[i] = t.Y[i];
-    }
+    r.X0 = t.X[0];
+    r.Y0 = t.Y[0];
+    r.d1 = ((uint32_t)(t.X[1] - t.X[0]) & 0xFFFFu) | ((uint32_t)(t.Y[1] - t.Y[0]) << 16);
+    r.d2 = ((uint32_t)(t.X[2] - t.X[0]) & 0xFFFFu) | ((uint32_t)(t.Y[2] - t.Y[0]) << 16);
     r.z0 = t.z0; r.A = t.A; r.B = t.B; r.zoff = t.zoff;
-    r.bx = (uint32_t)t.px0 | ((uint32_t)t.px1 << 16);
-    r.by = (uint32_t)t.py0 | ((uint32_t)t.py1 << 16);
     return r;
 }
 
-// Same tie rule as setup_piece, on the same 24.8 coordinates.
-__device__ __forceinline__ Setup from_rec(const SetupRec& r, uint32_t id) {
+// Same box and tie rules as setup_piece, on the same 24.8 coordinates.
+__device__ __forceinline__ Setup from_rec(const SetupRec& r, uint32_t id, const RasterCfg& cfg) {
     Setup s;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) {
-        s.X[i] = r.X[i];
-        s.Y[i] = r.Y[i];
-    }
-    s.px0 = (int)(r.bx & 0xFFFFu); s.px1 = (int)(r.bx >> 16);
-    s.py0 = (int)(r.by & 0xFFFFu); s.py1 = (int)(r.by >> 16);
+    s.X[0] = r.X0;
+    s.Y[0] = r.Y0;
+    s.X[1] = r.X0 + (int)(int16_t)(r.d1 & 0xFFFFu);
+    s.Y[1] = r.Y0 + ((int)r.d1 >> 16);
+    s.X[2] = r.X0 + (int)(int16_t)(r.d2 & 0xFFFFu);
+    s.Y[2] = r.Y0 + ((int)r.d2 >> 16);
+    s.px0 = max((min(s.X[0], min(s.X[1], s.X[2])) + 127) >> 8, 0);
+    s.px1 = min((max(s.X[0], max(s.X[1], s.X[2])) - 128) >> 8, cfg.w - 1);
+    s.py0 = max((min(s.Y[0], min(s.Y[1], s.Y[2])) + 127) >> 8, 0);
+    s.py1 = min((max(s.Y[0], max(s.Y[1], s.Y[2])) - 128) >> 8, cfg.h - 1);
     s.tl = 0;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         int a = (i + 1) % 3, b = (i + 2) % 3;
-        const int dy = r.Y[b] - r.Y[a], dx = r.X[b] - r.X[a];
+        const int dy = s.Y[b] - s.Y[a], dx = s.X[b] - s.X[a];
         s.tl |= (dy < 0 || (dy == 0 && dx < 0)) ? (1 << i) : 0;
     }
     s.id = id;
@@ -568,7 +577,7 @@ __device__ __forceinline__ void bin_body(const MeshView& mesh, const MvpSource& 
             int tx0 = t.px0 / TS, tx1 = t.px1 / TS, ty0 = t.py0 / TS, ty1 = t.py1 / TS;
             int ntx = tx1 - tx0 + 1;
             int span = ntx * (ty1 - ty0 + 1);
-            if (span > kWideSpan) {
+            if (span > kWideSpan || (kCache && !rec_fits(t))) {
                 if (!kScatter) push_record(b, map, t, entry);
             } else {
                 uint32_t mask = 0;
@@ -945,52 +954,35 @@ struct KeyOf<true> {
     static constexpr unsigned long long clear = ~0ull;
 };
 
-// Edge functions of `s` at pixel centre (i, j) and their per-pixel steps.
-// Stepping adds exact integers, so every value equals eval_setup's.
-struct Edges {
-    long long e[3];
-    long long dx[3], dy[3];  // change per +1 pixel in x / y
-};
-
-__device__ __forceinline__ void edges_at(const Setup& s, int i, int j, Edges& E) {
-    const int Px = i * 256 + 128, Py = j * 256 + 128;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        const int a = (k + 1) % 3, b = (k + 2) % 3;
-        const int ex = s.X[b] - s.X[a], ey = s.Y[b] - s.Y[a];
-        E.e[k] = (long long)ex * (Py - s.Y[a]) - (long long)ey * (Px - s.X[a]);
-        E.dx[k] = (long long)ey * -256;
-        E.dy[k] = (long long)ex * 256;
-    }
-}
-
 // Depth of a covered pixel centre at fixed-point offset (dx, dy) from vertex 0.
-__device__ __forceinline__ uint32_t plane_bits(const Setup& s, int dx, int dy) {
-    float z = s.z0 + (s.A * (float)dx + s.B * (float)dy);
-    z = z + s.zoff;
+__device__ __forceinline__ uint32_t window_bits(float z, float zoff) {
+    z = z + zoff;
     if (!(z > 0.0f)) z = 0.0f;  // NaN and -0 become +0
     // z is +0 or positive here (never NaN), where min(z, 1) is `z > 1 ? 1 : z`
     return fbits(__builtin_fminf(z, 1.0f));
 }
+__device__ __forceinline__ uint32_t plane_bits(const Setup& s, int dx, int dy) {
+    return window_bits(s.z0 + (s.A * (float)dx + s.B * (float)dy), s.zoff);
+}
 
 template <bool kVis>
-__device__ __forceinline__ void store_min(const Setup& s, uint32_t zb, int slot, typename KeyOf<kVis>::T* tile) {
+__device__ __forceinline__ void store_min(uint32_t id, uint32_t zb, int slot, typename KeyOf<kVis>::T* tile) {
     if constexpr (kVis) {
-        atomicMin(&tile[slot], ((unsigned long long)zb << 32) | s.id);
+        atomicMin(&tile[slot], ((unsigned long long)zb << 32) | id);
     } else {
         atomicMin(&tile[slot], zb);
     }
 }
 
-template <bool kVis, typename E>
-__device__ __forceinline__ void plot(const Setup& s, const E e[3], int i, int j, int slot,
-                                     typename KeyOf<kVis>::T* tile) {
-    if (e[0] + (E)(s.tl & 1) <= 0 || e[1] + (E)((s.tl >> 1) & 1) <= 0 || e[2] + (E)((s.tl >> 2) & 1) <= 0) return;
-    store_min<kVis>(s, plane_bits(s, i * 256 + 128 - s.X[0], j * 256 + 128 - s.Y[0]), slot, tile);
+// LDS row pitch of a tile: 8 words more than the tile's edge, so that the 64
+// pixels of an aligned 8x8 block lie in 64 different banks.
+template <int TS>
+constexpr int tile_pitch() {
+    return TS + 8;
 }
 
-// True when every pixel centre of [rx0, rx1] x [ry0, ry1] passes plot()'s
-// three edge tests.  Each edge value is affine in the pixel indices, so its
+// True when every pixel centre of [rx0, rx1] x [ry0, ry1] passes the three
+// edge tests.  Each edge value is affine in the pixel indices, so its
 // minimum over the rectangle is at a corner, and the test `e + tl > 0` holds
 // everywhere once it holds at the four corners.
 __device__ __forceinline__ bool rect_inside(const Setup& s, int rx0, int rx1, int ry0, int ry1) {
@@ -1009,92 +1001,274 @@ __device__ __forceinline__ bool rect_inside(const Setup& s, int rx0, int rx1, in
     return true;
 }
 
-// One thread covers the whole (small) rectangle, row by row.  When every
-// edge value inside the triangle's bounding box fits in 32 bits, the exact
-// stepping runs in int32.
-template <int TS, bool kVis, typename E>
-__device__ __forceinline__ void raster_rect_self_t(const Setup& s, const Edges& E64, int x0, int y0, int rx0, int rx1,
-                                                   int ry0, int ry1, typename KeyOf<kVis>::T* tile) {
-    E row[3], dx[3], dy[3];
+// The edge tests of one record over one tile in 32 bits.  Edge k's value at
+// pixel (i, j) of the tile is E + 256 (j ex - i ey) with E its value at the
+// tile's first pixel centre, so
+//   E + 256 (..) + tl > 0   <=>   ((E + tl - 1) >> 8) + j ex - i ey >= 0
+// exactly (`>>` rounds down).  Within a tile of at most 64 pixels the second
+// part stays below 2^30 in magnitude when |ex| and |ey| are below 2^23, and a
+// first part of 2^30 or more then decides the test in the whole tile, so it is
+// clamped there and every sum fits in int32; the factors fit the 24-bit
+// multipliers.  ok is false for longer edges: 32,768 pixels and more, which
+// the guard band (four times the view) allows only in views of kBigView pixels
+// and more; the kernels' kBig variants send those records to raster_rect_slow.
+constexpr int kBigView = (1 << 23) / 256 / (int)kGuard;
+inline bool big_view(const RasterCfg& cfg) { return cfg.w >= kBigView || cfg.h >= kBigView; }
+struct TileEdges {
+    int e[3];
+    int ex[3], ey[3];
+    bool ok;
+};
+__device__ __forceinline__ TileEdges tile_edges(const Setup& s, int x0, int y0) {
+    TileEdges t;
+    t.ok = true;
+    const int Px = x0 * 256 + 128, Py = y0 * 256 + 128;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        row[k] = (E)E64.e[k];
-        dx[k] = (E)E64.dx[k];
-        dy[k] = (E)E64.dy[k];
+        const int a = (k + 1) % 3, b = (k + 2) % 3;
+        const int ex = s.X[b] - s.X[a], ey = s.Y[b] - s.Y[a];
+        const long long E = (long long)ex * (Py - s.Y[a]) - (long long)ey * (Px - s.X[a]) + ((s.tl >> k) & 1) - 1;
+        const long long r = E >> 8;
+        t.e[k] = (int)(r > (1ll << 30) ? (1ll << 30) - 1 : r < -(1ll << 30) ? -(1ll << 30) : r);
+        t.ex[k] = ex;
+        t.ey[k] = ey;
+        t.ok = t.ok && abs(ex) < (1 << 23) && abs(ey) < (1 << 23);
     }
+    return t;
+}
+
+// Pixels n0, n0 + n, ... of the rectangle with the 64-bit edge functions.
+template <int TS, bool kVis>
+__device__ __forceinline__ void raster_rect_slow(const Setup& s, int x0, int y0, int rx0, int rx1, int ry0, int ry1,
+                                                 int n0, int n, typename KeyOf<kVis>::T* tile) {
+    const int rw = rx1 - rx0 + 1, area = rw * (ry1 - ry0 + 1);
+    for (int q = n0; q < area; q += n) {
+        const int i = rx0 + q % rw, j = ry0 + q / rw;
+        float z;
+        if (eval_setup(s, i, j, z)) store_min<kVis>(s.id, fbits(z), (j - y0) * tile_pitch<TS>() + (i - x0), tile);
+    }
+}
+
+// One thread covers the whole (small) rectangle, row by row.
+template <int TS, bool kVis>
+__device__ __forceinline__ void raster_rect_self(const Setup& s, const TileEdges& t, int x0, int y0, int rx0, int rx1,
+                                                 int ry0, int ry1, typename KeyOf<kVis>::T* tile) {
+    int row[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) row[k] = t.e[k] + __mul24(ry0 - y0, t.ex[k]) - __mul24(rx0 - x0, t.ey[k]);
+    const int width = rx1 - rx0;
+    const float dx0 = (float)(rx0 * 256 + 128 - s.X[0]);
+    int slot0 = (ry0 - y0) * tile_pitch<TS>() + (rx0 - x0);
     for (int j = ry0; j <= ry1; ++j) {
-        E e[3] = {row[0], row[1], row[2]};
-        for (int i = rx0; i <= rx1; ++i) {
-            plot<kVis, E>(s, e, i, j, (j - y0) * TS + (i - x0), tile);
-#pragma unroll
-            for (int k = 0; k < 3; ++k) e[k] += dx[k];
+        int e0 = row[0], e1 = row[1], e2 = row[2];
+        const float bdy = s.B * (float)(j * 256 + 128 - s.Y[0]);
+        float dx = dx0;  // pixel-centre offsets are at most 2^24: exact in FP32, steps too
+        const int end = slot0 + width;
+        for (int slot = slot0; slot <= end; ++slot) {
+            if ((e0 | e1 | e2) >= 0)
+                store_min<kVis>(s.id, window_bits(s.z0 + (s.A * dx + bdy), s.zoff), slot, tile);
+            e0 -= t.ey[0];
+            e1 -= t.ey[1];
+            e2 -= t.ey[2];
+            dx += 256.0f;
         }
+        slot0 += tile_pitch<TS>();
 #pragma unroll
-        for (int k = 0; k < 3; ++k) row[k] += dy[k];
+        for (int k = 0; k < 3; ++k) row[k] += t.ex[k];
     }
 }
 
-template <int TS, bool kVis>
-__device__ __forceinline__ void raster_rect_self(const Setup& s, int x0, int y0, int rx0, int rx1, int ry0, int ry1,
-                                                 typename KeyOf<kVis>::T* tile) {
-    Edges E;
-    edges_at(s, rx0, ry0, E);
-    const long long bw = (long long)max(s.X[0], max(s.X[1], s.X[2])) - min(s.X[0], min(s.X[1], s.X[2]));
-    const long long bh = (long long)max(s.Y[0], max(s.Y[1], s.Y[2])) - min(s.Y[0], min(s.Y[1], s.Y[2]));
-    // |e| <= 2*bw*bh inside the box and one step past it adds at most
-    // 256*max(bw, bh), so with these bounds every value stays below 2^30.
-    if (bw * bh < (1ll << 28) && bw < (1 << 20) && bh < (1 << 20))
-        raster_rect_self_t<TS, kVis, int>(s, E, x0, y0, rx0, rx1, ry0, ry1, tile);
-    else
-        raster_rect_self_t<TS, kVis, long long>(s, E, x0, y0, rx0, rx1, ry0, ry1, tile);
+// 8x8-pixel blocks of the tile that a rectangle (tile-local pixels) touches,
+// bit (TS / 8) * by + bx of block (bx, by).
+template <int TS>
+__device__ __forceinline__ unsigned long long block_mask(int rx0, int rx1, int ry0, int ry1) {
+    constexpr int NB = TS / 8;
+    const int bx0 = rx0 >> 3, bx1 = rx1 >> 3, by0 = ry0 >> 3, by1 = ry1 >> 3;
+    const unsigned row = (2u << bx1) - (1u << bx0);
+    unsigned long long m;
+    if constexpr (NB == 8) {
+        const unsigned r4 = row * 0x01010101u;
+        m = ((unsigned long long)r4 << 32) | r4;
+    } else {
+        m = row * 0x1111u;
+    }
+    return m & (~0ull << (NB * by0)) & (~0ull >> (63 - (NB * by1 + NB - 1)));
 }
 
-// The workgroup covers the rectangle in row groups of cw columns, cw the
-// smallest power of two (8 to TS) not below the rectangle's width: thread t
-// owns column rx0 + t % cw and every (kRasterThreads / cw)-th row from
-// ry0 + t / cw, so a wave covers 64 / cw rows and at least half its lanes
-// hold a pixel column.
+// Keeps a value in a vector register (the compiler otherwise forms sums of
+// wave-uniform values with scalar multiplications).
+__device__ __forceinline__ int in_vector(int v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+// Lane b: the largest depth (as bits) that block b of the tile holds now.
+// Depths only fall, so a value that other waves have lowered since is still an
+// upper bound.  The lanes start at different rows and halves of their blocks,
+// which spreads each read over the banks.
 template <int TS, bool kVis>
-__device__ __forceinline__ void raster_rect_group(const Setup& s, int x0, int y0, int rx0, int rx1, int ry0, int ry1,
-                                                  int tid, typename KeyOf<kVis>::T* tile) {
-    const int rw = rx1 - rx0 + 1;
-    int lg = 3;
-    while ((1 << lg) < rw) ++lg;  // rw <= TS
-    const int i = rx0 + (tid & ((1 << lg) - 1));
-    if (i > rx1) return;
-    int j = ry0 + (tid >> lg);
-    if (j > ry1) return;
-    const int row_step = kRasterThreads >> lg;
-    if (rect_inside(s, rx0, rx1, ry0, ry1)) {
-        // every pixel centre of the rectangle passes the three edge tests
-#pragma unroll 4
-        for (; j <= ry1; j += row_step)
-            store_min<kVis>(s, plane_bits(s, i * 256 + 128 - s.X[0], j * 256 + 128 - s.Y[0]),
-                            (j - y0) * TS + (i - x0), tile);
-        return;
-    }
-    Edges E;
-    edges_at(s, i, j, E);
-    long long e[3] = {E.e[0], E.e[1], E.e[2]};
-    long long step[3];
+__device__ __forceinline__ uint32_t block_zmax(int lane, const typename KeyOf<kVis>::T* tile) {
+    constexpr int NB = TS / 8;
+    const int bx = lane % NB, by = lane / NB;
+    uint32_t z = 0u;
+    if (lane < NB * NB) {
+#pragma unroll 2
+        for (int r = 0; r < 8; ++r) {
+            const int row = (by * 8 + ((r + by) & 7)) * tile_pitch<TS>() + bx * 8;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) step[k] = E.dy[k] * row_step;
-    for (; j <= ry1; j += row_step) {
-        plot<kVis, long long>(s, e, i, j, (j - y0) * TS + (i - x0), tile);
+            for (int h = 0; h < 2; ++h) {
+                const int at = row + ((h + by) & 1) * 4;
+                if constexpr (kVis) {
 #pragma unroll
-        for (int k = 0; k < 3; ++k) e[k] += step[k];
+                    for (int q = 0; q < 4; ++q) z = max(z, (uint32_t)(tile[at + q] >> 32));
+                } else {
+                    const uint4 v = *reinterpret_cast<const uint4*>(&tile[at]);
+                    z = max(max(z, max(v.x, v.y)), max(v.z, v.w));
+                }
+            }
+        }
     }
+    return z;
+}
+
+// The wave covers one record (all arguments but `lane` and `zmax` are
+// wave-uniform): lane b first tests block b of the tile against the three
+// edges (the block's pixel nearest to each edge's inside) and against the
+// depth the block already has (zmax, block_zmax's), then the blocks left are
+// taken row by row, a lane per pixel, 12 vector instructions each.  The
+// record's smallest depth in a block is that of the corner pixel its plane
+// falls to: every rounded step of the depth expression is monotonic in dx and
+// in dy, so no pixel of the block comes out below it.
+// kWhole: blocks that lie inside all three edges (most of a ground plane's)
+// are taken without edge tests.
+template <int TS, bool kVis, bool kWhole>
+__device__ __forceinline__ void raster_blocks(const int er[3], const int ex[3], const int ey[3], float z0, float A,
+                                              float B, float zoff, int dx0, int dy0, uint32_t id,
+                                              unsigned long long blocks, int lane, uint32_t zmax,
+                                              typename KeyOf<kVis>::T* tile) {
+    constexpr int NB = TS / 8;
+    const int blx = (lane % NB) * 8, bly = (lane / NB) * 8;
+    const int lx = lane & 7, ly = lane >> 3;
+    int near[3], off[3], step[3], inner[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int far = er[k] + max(0, 7 * ex[k]) + max(0, -7 * ey[k]);
+        near[k] = far + __mul24(bly, ex[k]) - __mul24(blx, ey[k]);
+        if constexpr (kWhole) inner[k] = near[k] - 7 * (abs(ex[k]) + abs(ey[k]));
+        off[k] = in_vector(er[k] + __mul24(ly, ex[k]) - __mul24(lx, ey[k]));
+        step[k] = in_vector(-ey[k]);
+    }
+    const uint32_t zmin =
+        window_bits(z0 + (A * (float)(dx0 + (blx + (A < 0.0f ? 7 : 0)) * 256) +
+                          B * (float)(dy0 + (bly + (B < 0.0f ? 7 : 0)) * 256)), zoff);
+    const bool open = kVis ? zmin <= zmax : zmin < zmax;
+    unsigned long long live = __ballot((near[0] | near[1] | near[2]) >= 0 && open) & blocks;
+    unsigned long long whole = 0ull;
+    if constexpr (kWhole) whole = __ballot((inner[0] | inner[1] | inner[2]) >= 0);
+    const int dxl = in_vector(dx0 + lx * 256), dyl = in_vector(dy0 + ly * 256);
+    const int slot = ly * tile_pitch<TS>() + lx;
+    while (live) {
+        const int row = (__ffsll((long long)live) - 1) / NB;
+        unsigned cols = (unsigned)(live >> (row * NB)) & ((1u << NB) - 1u);
+        const unsigned inside = (unsigned)(whole >> (row * NB));
+        live &= ~((unsigned long long)cols << (row * NB));
+        const int e0 = in_vector(off[0] + 8 * row * ex[0]), e1 = in_vector(off[1] + 8 * row * ex[1]),
+                  e2 = in_vector(off[2] + 8 * row * ex[2]);
+        const float bdy = B * (float)(dyl + row * 2048);
+        const int srow = in_vector(slot + row * 8 * tile_pitch<TS>());
+        while (cols) {
+            const int bx = __ffs((int)cols) - 1, i = 8 * bx;
+            cols &= cols - 1;
+            if ((kWhole && (inside >> bx & 1u)) ||
+                ((e0 + __mul24(i, step[0])) | (e1 + __mul24(i, step[1])) | (e2 + __mul24(i, step[2]))) >= 0)
+                store_min<kVis>(id, window_bits(z0 + (A * (float)(dxl + (i << 8)) + bdy), zoff), srow + i, tile);
+        }
+    }
+}
+
+__device__ __forceinline__ int lane_int(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ float lane_float(float v, int l) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+
+// raster_blocks for the records of the lanes with `want`, one after another;
+// the wave looks at the tile's depths again after every kZmaxAge of them.
+constexpr int kZmaxAge = 8;
+template <int TS, bool kVis, bool kWhole>
+__device__ __forceinline__ void raster_lanes(const Setup& s, const TileEdges& t, unsigned long long blocks, bool want,
+                                             int x0, int y0, int lane, uint32_t& zmax, int& age,
+                                             typename KeyOf<kVis>::T* tile) {
+    const int dx0 = x0 * 256 + 128 - s.X[0], dy0 = y0 * 256 + 128 - s.Y[0];
+    unsigned long long todo = __ballot(want);
+    while (todo) {
+        const int l = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        if (++age == kZmaxAge) {
+            age = 0;
+            zmax = block_zmax<TS, kVis>(lane, tile);
+        }
+        const int er[3] = {lane_int(t.e[0], l), lane_int(t.e[1], l), lane_int(t.e[2], l)};
+        const int a0 = lane_int(t.ex[0], l), a1 = lane_int(t.ex[1], l);
+        const int b0 = lane_int(t.ey[0], l), b1 = lane_int(t.ey[1], l);
+        const int ex[3] = {a0, a1, -(a0 + a1)}, ey[3] = {b0, b1, -(b0 + b1)};  // the edges close
+        const unsigned long long m = ((unsigned long long)(unsigned)lane_int((int)(blocks >> 32), l) << 32) |
+                                     (unsigned)lane_int((int)(unsigned)blocks, l);
+        raster_blocks<TS, kVis, kWhole>(er, ex, ey, lane_float(s.z0, l), lane_float(s.A, l), lane_float(s.B, l),
+                                lane_float(s.zoff, l), lane_int(dx0, l), lane_int(dy0, l),
+                                kVis ? (uint32_t)lane_int((int)s.id, l) : 0u, m, lane, zmax, tile);
+    }
+}
+
+// Why both: on a 200k-triangle soup in one 2048^2 map the raster took 213 us
+// with records over 256 pixels covered by the whole workgroup, one after
+// another between barriers (each wave repeating the record's setup for a
+// quarter of its pixels), and 130 us with a wave per record; a batch of twelve
+// frames (soups on 512^2-4096^2 maps) 4.82 and 2.94 ms.  Sending every record
+// over 256 pixels to the wave, whatever its neighbours' size, takes the batch
+// 3.26 ms.  Before the 32-bit edges and the vector-register steps a block
+// took 20 vector and 18 scalar instructions (batch 3.06 ms).
+//
+// Records a lane rasterizes alone: those with at most self_bound() pixels of
+// bounding box in the tile.  The wave then runs as long as the largest such
+// box (about 14 vector instructions a pixel), while a larger record takes the
+// whole wave for the instructions in `cost` (its blocks by box size).  The
+// bound that is cheapest for these 64 records, out of 8, 16, .. 1024 pixels.
+__device__ __forceinline__ int self_bound(int area, bool has) {
+    constexpr int cost[8] = {75, 80, 90, 105, 135, 190, 285, 500};  // boxes over 8, 16, .. 1024 pixels
+    unsigned long long over = __ballot(has && area > 1024);
+    int sum = cost[7] * __popcll(over);
+    int best = 1024, least = sum + 14 * 1024;
+#pragma unroll
+    for (int q = 6; q >= 0; --q) {
+        const int b = 8 << q;
+        const unsigned long long o = __ballot(has && area > b);
+        sum += cost[q] * __popcll(o & ~over);
+        over = o;
+        if (sum + 14 * b < least) {
+            least = sum + 14 * b;
+            best = b;
+        }
+    }
+    return best;
 }
 
 // One (tile, map) of the raster.  kFallback: the map's lists overflowed the
 // workspace, so every (triangle, piece) pair is visited with full clipping.
-template <int TS, bool kVis, bool kFallback>
+//
+// Each wave takes 64 records of every 256 (a record per lane: load, box, edge
+// values).  `spread` interleaves them, so that a short list reaches all four
+// waves: for launches that leave the GPU room (spread_lists).  Small records are rasterized by their lane, larger ones by the wave in 8x8
+// blocks; no barrier stands between the records.  Where the list is short,
+// records of many blocks (a ground plane) are put aside and covered by the
+// four waves together at the end.
+template <int TS, bool kVis, bool kFallback, bool kBig>
 __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                             const BinBufs& b, void* out, int map, int tile_id,
-                                            typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec) {
-    const int tid = threadIdx.x;
+                                            typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec, bool spread) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tx = tile_id % cfg.tiles_x, ty = tile_id / cfg.tiles_x;
     constexpr int kTilePx = TS * TS;
+    constexpr int kWaves = kRasterThreads / 64;
     const int x0 = tx * TS, y0 = ty * TS;
     const int x1 = min(x0 + TS - 1, cfg.w - 1), y1 = min(y0 + TS - 1, cfg.h - 1);
     const int ntiles = cfg.tiles_x * cfg.tiles_y;
@@ -1133,68 +1307,98 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
             }
         }
     }
+    constexpr int kWords = TS * tile_pitch<TS>();
     if constexpr (!kVis) {  // 16-byte LDS writes
         constexpr uint32_t c = KeyOf<kVis>::clear;
-        for (int q = tid; q < kTilePx / 4; q += kRasterThreads) reinterpret_cast<uint4*>(tile)[q] = make_uint4(c, c, c, c);
+        for (int q = tid; q < kWords / 4; q += kRasterThreads) reinterpret_cast<uint4*>(tile)[q] = make_uint4(c, c, c, c);
     } else {
-        for (int p = tid; p < kTilePx; p += kRasterThreads) tile[p] = KeyOf<kVis>::clear;
+        for (int p = tid; p < kWords; p += kRasterThreads) tile[p] = KeyOf<kVis>::clear;
     }
     if (tid == 0) nrec = 0;
-    float mvp[16];
-    mvps.load(map, mvp);
     __syncthreads();
+    // records of more blocks than this are put aside for the four waves
+    const int aside = end - begin <= (uint32_t)kShareList ? kShareBlocks : kShareBlocksLong;
+    uint32_t zmax = 0xFFFFFFFFu;  // lane b: bound of block b's depths, read `age` wave records ago
+    int age = 0;
     for (uint32_t base = begin; base < end; base += kRasterThreads) {
-        uint32_t k = base + tid;
-        if (k < end) {
-            uint32_t entry = kFallback ? k : b.entries[(size_t)map * b.cap + k];
+        const uint32_t k = base + (uint32_t)(spread ? lane * kWaves + wave : tid);
+        Setup s;
+        bool has = k < end;
+        if (has) {
+            const uint32_t entry = kFallback ? k : b.entries[(size_t)map * b.cap + k];
             if (!kFallback && (entry & kWideBit)) {
-                const Setup& w = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
-                int slot = atomicAdd(&nrec, 1);
-                if (slot < kRecQueue) {
-                    rec[slot] = w;
-                } else {
-                    int rx0 = max(x0, w.px0), rx1 = min(x1, w.px1), ry0 = max(y0, w.py0), ry1 = min(y1, w.py1);
-                    if (rx0 <= rx1 && ry0 <= ry1) raster_rect_self<TS, kVis>(w, x0, y0, rx0, rx1, ry0, ry1, tile);
-                }
+                s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
             } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
                 // a directly binned triangle: the count pass stored its setup
-                const Setup s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry);
-                int rx0 = max(x0, s.px0), rx1 = min(x1, s.px1), ry0 = max(y0, s.py0), ry1 = min(y1, s.py1);
-                if (rx0 <= rx1 && ry0 <= ry1) {
-                    int slot = kRecQueue;
-                    if ((rx1 - rx0 + 1) * (ry1 - ry0 + 1) > kSelfRasterMaxPx) slot = atomicAdd(&nrec, 1);
-                    if (slot < kRecQueue) rec[slot] = s;
-                    else raster_rect_self<TS, kVis>(s, x0, y0, rx0, rx1, ry0, ry1, tile);
-                }
+                s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
             } else {
+                float mvp[16];
+                mvps.load(map, mvp);
                 Tri<0> t;
-                bool ok;
                 if constexpr (kFallback)
-                    get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, ok);
+                    get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, has);
                 else
-                    classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, ok);
-                if (ok) {
-                    int rx0 = max(x0, t.px0), rx1 = min(x1, t.px1), ry0 = max(y0, t.py0), ry1 = min(y1, t.py1);
-                    if (rx0 <= rx1 && ry0 <= ry1) {
-                        Setup s = to_setup(t, entry);
-                        int slot = kRecQueue;
-                        if ((rx1 - rx0 + 1) * (ry1 - ry0 + 1) > kSelfRasterMaxPx) slot = atomicAdd(&nrec, 1);
-                        if (slot < kRecQueue) rec[slot] = s;
-                        else raster_rect_self<TS, kVis>(s, x0, y0, rx0, rx1, ry0, ry1, tile);
-                    }
+                    classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, has);
+                if (has) s = to_setup(t, entry);
+            }
+        }
+        int rx0 = 0, rx1 = -1, ry0 = 0, ry1 = -1;
+        if (has) {
+            rx0 = max(x0, s.px0);
+            rx1 = min(x1, s.px1);
+            ry0 = max(y0, s.py0);
+            ry1 = min(y1, s.py1);
+            has = rx0 <= rx1 && ry0 <= ry1;
+        }
+        TileEdges t = {};
+        unsigned long long blocks = 0;
+        int area = 0;
+        if (has) {
+            t = tile_edges(s, x0, y0);
+            blocks = block_mask<TS>(rx0 - x0, rx1 - x0, ry0 - y0, ry1 - y0);
+            area = (rx1 - rx0 + 1) * (ry1 - ry0 + 1);
+            if ((kBig && !t.ok) || __popcll(blocks) > aside) {
+                const int slot = atomicAdd(&nrec, 1);
+                if (slot < kRecQueue) {
+                    rec[slot] = s;
+                    has = false;
+                } else if (kBig && !t.ok) {
+                    raster_rect_slow<TS, kVis>(s, x0, y0, rx0, rx1, ry0, ry1, 0, 1, tile);
+                    has = false;
                 }
             }
         }
-        __syncthreads();
-        const int nq = min(nrec, kRecQueue);
-        for (int q = 0; q < nq; ++q) {
-            const Setup s = rec[q];
-            int rx0 = max(x0, s.px0), rx1 = min(x1, s.px1), ry0 = max(y0, s.py0), ry1 = min(y1, s.py1);
-            if (rx0 > rx1 || ry0 > ry1) continue;
-            raster_rect_group<TS, kVis>(s, x0, y0, rx0, rx1, ry0, ry1, tid, tile);
+        const int bound = self_bound(area, has);
+        const bool self = has && area <= bound;
+        raster_lanes<TS, kVis, false>(s, t, blocks, has && !self, x0, y0, lane, zmax, age, tile);
+        if (self) raster_rect_self<TS, kVis>(s, t, x0, y0, rx0, rx1, ry0, ry1, tile);
+    }
+    __syncthreads();
+    const int nq = min(nrec, kRecQueue);
+    if (nq > 0) {  // uniform: the records put aside, block rows (by % 4 == wave) per wave
+        Setup s;
+        TileEdges t = {};
+        unsigned long long blocks = 0;
+        const bool has = lane < nq;
+        if (has) {
+            s = rec[lane];
+            t = tile_edges(s, x0, y0);
+            unsigned long long rows = 0;
+#pragma unroll
+            for (int r = 0; r < TS / 8; r += kWaves) rows |= ((1ull << (TS / 8)) - 1ull) << ((TS / 8) * (r + wave));
+            blocks = rows & block_mask<TS>(max(x0, s.px0) - x0, min(x1, s.px1) - x0, max(y0, s.py0) - y0,
+                                           min(y1, s.py1) - y0);
         }
-        __syncthreads();
-        if (tid == 0) nrec = 0;
+        raster_lanes<TS, kVis, true>(s, t, blocks, has && (!kBig || t.ok), x0, y0, lane, zmax, age, tile);
+        if constexpr (kBig) {
+            unsigned long long slow = __ballot(has && !t.ok);
+            while (slow) {
+                const Setup q = rec[__ffsll((long long)slow) - 1];
+                slow &= slow - 1;
+                raster_rect_slow<TS, kVis>(q, x0, y0, max(x0, q.px0), min(x1, q.px1), max(y0, q.py0), min(y1, q.py1),
+                                           tid, kRasterThreads, tile);
+            }
+        }
         __syncthreads();
     }
     // Write the tile once.  Depth maps go out with non-temporal stores: a
@@ -1211,26 +1415,26 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
         if (full) {
             typedef float f4 __attribute__((ext_vector_type(4)));
             for (int q = tid; q < kTilePx / 4; q += kRasterThreads) {
-                int r = q / (TS / 4), cidx = (q % (TS / 4)) * 4;
-                int j = y0 + r;
+                const int r = q / (TS / 4), cidx = (q % (TS / 4)) * 4;
+                const int j = y0 + r;
                 if (j > y1) continue;
-                const f4 v = {__uint_as_float(tile[r * TS + cidx + 0]), __uint_as_float(tile[r * TS + cidx + 1]),
-                              __uint_as_float(tile[r * TS + cidx + 2]), __uint_as_float(tile[r * TS + cidx + 3])};
+                const f4 v = *reinterpret_cast<const f4*>(&tile[r * tile_pitch<TS>() + cidx]);
                 __builtin_nontemporal_store(v, reinterpret_cast<f4*>(dst + (size_t)j * cfg.w + x0 + cidx));
             }
         } else {
             for (int p = tid; p < kTilePx; p += kRasterThreads) {
-                int i = x0 + p % TS, j = y0 + p / TS;
+                const int i = x0 + p % TS, j = y0 + p / TS;
                 if (i > x1 || j > y1) continue;
-                __builtin_nontemporal_store(__uint_as_float(tile[p]), dst + (size_t)j * cfg.w + i);
+                __builtin_nontemporal_store(__uint_as_float(tile[(p / TS) * tile_pitch<TS>() + p % TS]),
+                                            dst + (size_t)j * cfg.w + i);
             }
         }
     } else {
         unsigned long long* dst = reinterpret_cast<unsigned long long*>(out) + (size_t)map * plane;
         for (int p = tid; p < kTilePx; p += kRasterThreads) {
-            int i = x0 + p % TS, j = y0 + p / TS;
+            const int i = x0 + p % TS, j = y0 + p / TS;
             if (i > x1 || j > y1) continue;
-            dst[(size_t)j * cfg.w + i] = tile[p];
+            dst[(size_t)j * cfg.w + i] = tile[(p / TS) * tile_pitch<TS>() + p % TS];
         }
     }
 }
@@ -1243,23 +1447,23 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
 // holding only the ground) arrive in runs that pile onto a few CUs while the
 // rest idle.  Tile-major order spreads each costly tile's maps over the XCDs
 // and CUs.
-template <int TS, bool kVis>
-__global__ __launch_bounds__(kRasterThreads) void k_raster(MeshView mesh, MvpSource mvps, RasterCfg cfg, BinBufs b,
-                                                           void* out, int map_base, int map_count) {
-    __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * TS];
+template <int TS, bool kVis, bool kBig>
+__global__ __launch_bounds__(kRasterThreads, kVis || kBig ? 1 : 8) void k_raster(MeshView mesh, MvpSource mvps, RasterCfg cfg, BinBufs b,
+                                                           void* out, int map_base, int map_count, bool spread) {
+    __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     const int map = map_base + (int)(blockIdx.x % (unsigned)map_count);
     const int tile_id = (int)(blockIdx.x / (unsigned)map_count);
     if (b.overflow[map]) return;
-    raster_tile<TS, kVis, false>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec);
+    raster_tile<TS, kVis, false, kBig>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, spread);
 }
 
 // One workgroup per tile, looping over the maps whose lists overflowed.
 template <int TS, bool kVis>
 __global__ __launch_bounds__(kRasterThreads) void k_raster_fallback(MeshView mesh, MvpSource mvps, RasterCfg cfg,
                                                                     BinBufs b, void* out, int nmaps) {
-    __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * TS];
+    __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     // The usual case is no overflowed map: the threads read the flags
@@ -1269,7 +1473,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_raster_fallback(MeshView mes
     if (!__syncthreads_or(any)) return;
     for (int map = 0; map < nmaps; ++map) {
         if (!b.overflow[map]) continue;
-        raster_tile<TS, kVis, true>(mesh, mvps, cfg, b, out, map, blockIdx.x, tile, rec, nrec);
+        raster_tile<TS, kVis, true, true>(mesh, mvps, cfg, b, out, map, blockIdx.x, tile, rec, nrec, true);
         __syncthreads();
     }
 }
@@ -1443,7 +1647,7 @@ inline size_t layout(int ntris, int nmaps, int w, int h, bool vis, Workspace* ws
     size_t o_tiles = off; off = align256(off + sizeof(uint32_t) * (size_t)(ntris > 0 ? ntris : 0) * nmaps);
     const bool records = 4 * (64 / ts) * (64 / ts) <= 4;  // the tile code's span (wide_span<ts>() <= 4)
     size_t o_setups = off;
-    if (records) off = align256(off + sizeof(SetupRec) * (size_t)(ntris > 0 ? ntris : 0) * nmaps);
+    if (records) off = align256(off + kRecStride * (size_t)(ntris > 0 ? ntris : 0) * nmaps);
     // the G-buffer pass (one map): visibility keys and the clipped pieces' attributes
     const uint32_t acap = vis ? std::min(ccap, kAttrTriangles) : 0u;
     size_t o_vis = off;

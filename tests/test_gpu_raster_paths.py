@@ -26,3 +26,52 @@ def test_gbuffer_of_clipped_triangles(gi, oracle_lib, cuda, n_small, n_clip, lis
     for name, got, want in (("position", g.position, pos), ("normal", g.normal, nrm), ("facing", g.facing, fac)):
         got = got.cpu().numpy()
         assert bits_equal(got, want), mismatch_report(got, want, name)
+
+
+@pytest.mark.parametrize("w,h", [(4096, 70), (8191, 64), (8192, 64), (16384, 65)])
+def test_depth_of_long_edges(gi, oracle_lib, cuda, w, h):
+    """Records whose edges run to the guard band (4 views) and slivers across
+    many tiles: the 32-bit edge tests up to 8,191 pixels, the 64-bit ones
+    beyond."""
+    rng = np.random.default_rng(w)
+    n = 40
+    pos = rng.uniform(-1.0, 1.0, size=(n, 3, 3))
+    pos[:, :, 0] *= rng.choice([0.5, 3.0, 30.0], size=(n, 3))
+    pos[:, :, 1] *= rng.choice([0.5, 3.0, 30.0], size=(n, 3))
+    pos[:, :, 2] *= 0.2
+    pos[0] = [[-90, -90, 0.9], [90, -90, 0.9], [0, 170, 0.9]]
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3).astype(np.float32), np.zeros((3 * n, 3), np.float32),
+                          np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvp = np.eye(4, dtype=np.float32).reshape(1, 16)
+    got = gi.render_shadow_map(gi.DeviceMesh.from_mesh(mesh), mvp, w, h).cpu().numpy()[0]
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp[0], w, h)
+    assert bits_equal(got, want), mismatch_report(got, want, f"{w}x{h}")
+    assert (want < 0.9).mean() > 0.05
+
+
+@pytest.mark.parametrize("n,edge,w,h", [(1, 8.0, 64, 64), (5, 30.0, 65, 63), (300, 2.0, 64, 64), (300, 12.0, 130, 70),
+                                        (900, 25.0, 192, 128), (700, 60.0, 257, 129), (6000, 4.0, 96, 64)])
+def test_depth_and_visibility_by_triangle_size(gi, oracle_lib, cuda, n, edge, w, h):
+    """Triangles of about `edge` pixels over a covering quad: records that a
+    lane rasterizes alone, that a wave takes in blocks, and that are put
+    aside, in short and long lists; depth maps and (through the G-buffer) the
+    visible triangle of every pixel, whose ties go to the lower index."""
+    rng = np.random.default_rng(n)
+    cen = rng.uniform(-1.0, 1.0, size=(n, 1, 3)) * [1.0, 1.0, 0.9]
+    size = rng.lognormal(0.0, 0.6, size=(n, 1, 1)) * edge * np.array([2.0 / w, 2.0 / h, 0.05])
+    pos = cen + rng.uniform(-1.0, 1.0, size=(n, 3, 3)) * size
+    pos[n // 2:n // 2 + n // 10] = pos[:n // 10]  # equal depths
+    quad = [[[-1, -1, 0.95], [1, -1, 0.95], [1, 1, 0.95]], [[-1, -1, 0.95], [1, 1, 0.95], [-1, 1, 0.95]]]
+    pos = np.concatenate([pos, quad]).astype(np.float32)
+    nt = len(pos)
+    nrm = rng.normal(size=(3 * nt, 3)).astype(np.float32)
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3), nrm, np.arange(3 * nt, dtype=np.int32).reshape(nt, 3))
+    mvp = np.eye(4, dtype=np.float32).reshape(16)
+    dm = gi.DeviceMesh.from_mesh(mesh)
+    got = gi.render_shadow_map(dm, mvp, w, h).cpu().numpy()[0]
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp, w, h)
+    assert bits_equal(got, want), mismatch_report(got, want, "depth")
+    g = gi.render_gbuffer(dm, mvp, w, h)
+    pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
+    assert bits_equal(g.position.cpu().numpy(), pos_o)
+    assert bits_equal(g.normal.cpu().numpy(), nrm_o), mismatch_report(g.normal.cpu().numpy(), nrm_o, "normal")
