@@ -17,7 +17,8 @@
 //   4. k_raster   one workgroup per (tile, map): resolve the tile's list into an
 //                 LDS tile with ds_min on the FP32 depth bits (non-negative
 //                 floats order like uint32) or on 64-bit (depth, id) keys,
-//                 then write the tile to HBM once with 16-byte stores.
+//                 then write the tile to HBM once with 16-byte stores
+//                 (k_raster_split: a long list's tile in regions).
 // atomicMin makes the result independent of list order, so the output is
 // deterministic.  When a map's lists would exceed the workspace, that map falls
 // back to every workgroup scanning the whole mesh (slower, same result).
@@ -52,6 +53,16 @@ namespace {
 // Tiles of a launch up to which every workgroup is resident at once.
 constexpr size_t kSpreadTiles = 2048;
 
+// Whether a depth pass of nmaps maps splits long tile lists (k_raster_split):
+// while its tiles are few enough (six per resident workgroup) that a long list
+// can outlast the rest: nine 2048^2 maps of a far mesh took 118 us without and
+// 98 us with, while with 64 maps of 2048^2 every CU has 250 tiles to draw from.
+constexpr size_t kSplitTiles = 12288;
+constexpr int kSplitMaps = 64;  // its workers hold a map's task count per lane
+bool splits_lists(int ntiles, int nmaps) {
+    return nmaps <= kSplitMaps && (size_t)ntiles * nmaps <= kSplitTiles;
+}
+
 // Binning of every map (count, clip, scan, scatter) and the raster of the
 // maps whose lists overflowed the workspace.
 template <bool kVis>
@@ -73,7 +84,8 @@ int bin_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, const Rast
             hipLaunchKernelGGL(k_clip<0>, dim3(kClipBlocks, nmaps), dim3(kClipThreads), 0, s, mesh, mvps, cfg, b);
         hipLaunchKernelGGL((k_bin_wide<kTile, false>), gw, dim3(256), 0, s, cfg, b);
     }
-    hipLaunchKernelGGL(k_scan, dim3(nmaps), dim3(kScanThreads), 0, s, b, ntiles);
+    hipLaunchKernelGGL(k_scan, dim3(nmaps), dim3(kScanThreads), 0, s, b, ntiles,
+                       splits_lists(ntiles, nmaps) ? nmaps : 0);
     if (mesh.nt > 0) {
         if constexpr (wide_span<kTile>() <= 4) {
             // triangles' appends and the wide records' appends in one launch
@@ -94,19 +106,29 @@ int bin_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, const Rast
 // bin stage left in the workspace (maps that overflowed are skipped: the bin
 // stage rastered them).
 template <bool kVis>
-int raster_stage(const MeshView& mesh, const MvpSource& mvps, int map_begin, int map_count, const RasterCfg& cfg,
-                 const Workspace& ws, void* out, hipStream_t s, hipEvent_t ev_begin = nullptr,
+int raster_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, int map_begin, int map_count,
+                 const RasterCfg& cfg, const Workspace& ws, void* out, hipStream_t s, hipEvent_t ev_begin = nullptr,
                  hipEvent_t ev_end = nullptr) {
     const int ntiles = cfg.tiles_x * cfg.tiles_y;
     if (ev_begin && hipEventRecord(ev_begin, s) != hipSuccess) return GI_EDEVICE;
-    const dim3 grid((unsigned)(ntiles * map_count));
-    const bool spread = ntiles * (size_t)map_count <= kSpreadTiles;
-    if (big_view(cfg))
-        hipLaunchKernelGGL((k_raster<kTile, kVis, true>), grid, dim3(kRasterThreads), 0, s, mesh, mvps, cfg, ws.bins,
-                           out, map_begin, map_count, spread);
-    else
-        hipLaunchKernelGGL((k_raster<kTile, kVis, false>), grid, dim3(kRasterThreads), 0, s, mesh, mvps, cfg, ws.bins,
-                           out, map_begin, map_count, spread);
+    const unsigned tiles = (unsigned)(ntiles * map_count);
+    const dim3 block(kRasterThreads);
+    const bool spread = tiles <= kSpreadTiles;
+    if (splits_lists(ntiles, nmaps)) {
+        const dim3 grid(tiles + kSplitWorkers);
+        if (big_view(cfg))
+            hipLaunchKernelGGL((k_raster_split<kTile, kVis, true>), grid, block, 0, s, mesh, mvps, cfg, ws.bins, out,
+                               map_begin, map_count);
+        else
+            hipLaunchKernelGGL((k_raster_split<kTile, kVis, false>), grid, block, 0, s, mesh, mvps, cfg, ws.bins, out,
+                               map_begin, map_count);
+    } else if (big_view(cfg)) {
+        hipLaunchKernelGGL((k_raster<kTile, kVis, true>), dim3(tiles), block, 0, s, mesh, mvps, cfg, ws.bins, out,
+                           map_begin, map_count, spread);
+    } else {
+        hipLaunchKernelGGL((k_raster<kTile, kVis, false>), dim3(tiles), block, 0, s, mesh, mvps, cfg, ws.bins, out,
+                           map_begin, map_count, spread);
+    }
     if (ev_end && hipEventRecord(ev_end, s) != hipSuccess) return GI_EDEVICE;
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
@@ -116,7 +138,7 @@ int run_raster(const MeshView& mesh, const MvpSource& mvps, int nmaps, const Ras
                void* out, hipStream_t s, hipEvent_t ev_begin = nullptr, hipEvent_t ev_end = nullptr) {
     int rc = bin_stage<kVis>(mesh, mvps, nmaps, cfg, ws, out, s);
     if (rc != GI_OK) return rc;
-    return raster_stage<kVis>(mesh, mvps, 0, nmaps, cfg, ws, out, s, ev_begin, ev_end);
+    return raster_stage<kVis>(mesh, mvps, nmaps, 0, nmaps, cfg, ws, out, s, ev_begin, ev_end);
 }
 
 }  // namespace
@@ -224,7 +246,7 @@ int gi_depth_pass_raster(const float* positions_dev, int nverts, const int32_t* 
                          depth_out_dev, workspace_dev, workspace_bytes, d);
     if (rc != GI_OK) return rc;
     if (map_begin < 0 || map_count <= 0 || map_begin > nmaps - map_count) return GI_EINVAL;
-    return raster_stage<false>(d.mesh, d.mvps, map_begin, map_count, d.cfg, d.ws, depth_out_dev,
+    return raster_stage<false>(d.mesh, d.mvps, nmaps, map_begin, map_count, d.cfg, d.ws, depth_out_dev,
                                reinterpret_cast<hipStream_t>(stream),
                                opts ? reinterpret_cast<hipEvent_t>(opts->raster_begin_event) : nullptr,
                                opts ? reinterpret_cast<hipEvent_t>(opts->raster_end_event) : nullptr);

@@ -366,6 +366,17 @@ __device__ __forceinline__ SetupRec to_rec(const Tri<0>& t) {
     return r;
 }
 
+// Pixel-centre box of a record's vertices, not yet clamped to the view.
+__device__ __forceinline__ void rec_box(int X0, int Y0, uint32_t d1, uint32_t d2, int& px0, int& px1, int& py0,
+                                        int& py1) {
+    const int x1 = (int)(int16_t)(d1 & 0xFFFFu), x2 = (int)(int16_t)(d2 & 0xFFFFu);
+    const int y1 = (int)d1 >> 16, y2 = (int)d2 >> 16;
+    px0 = (X0 + min(0, min(x1, x2)) + 127) >> 8;
+    px1 = (X0 + max(0, max(x1, x2)) - 128) >> 8;
+    py0 = (Y0 + min(0, min(y1, y2)) + 127) >> 8;
+    py1 = (Y0 + max(0, max(y1, y2)) - 128) >> 8;
+}
+
 // Same box and tie rules as setup_piece, on the same 24.8 coordinates.
 __device__ __forceinline__ Setup from_rec(const SetupRec& r, uint32_t id, const RasterCfg& cfg) {
     Setup s;
@@ -375,10 +386,11 @@ __device__ __forceinline__ Setup from_rec(const SetupRec& r, uint32_t id, const 
     s.Y[1] = r.Y0 + ((int)r.d1 >> 16);
     s.X[2] = r.X0 + (int)(int16_t)(r.d2 & 0xFFFFu);
     s.Y[2] = r.Y0 + ((int)r.d2 >> 16);
-    s.px0 = max((min(s.X[0], min(s.X[1], s.X[2])) + 127) >> 8, 0);
-    s.px1 = min((max(s.X[0], max(s.X[1], s.X[2])) - 128) >> 8, cfg.w - 1);
-    s.py0 = max((min(s.Y[0], min(s.Y[1], s.Y[2])) + 127) >> 8, 0);
-    s.py1 = min((max(s.Y[0], max(s.Y[1], s.Y[2])) - 128) >> 8, cfg.h - 1);
+    rec_box(r.X0, r.Y0, r.d1, r.d2, s.px0, s.px1, s.py0, s.py1);
+    s.px0 = max(s.px0, 0);
+    s.px1 = min(s.px1, cfg.w - 1);
+    s.py0 = max(s.py0, 0);
+    s.py1 = min(s.py1, cfg.h - 1);
     s.tl = 0;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -904,10 +916,31 @@ __global__ __launch_bounds__(256) void k_bin_scatter(MeshView mesh, RasterCfg cf
 
 constexpr int kScatterTris = 4;  // triangles per thread in k_bin_scatter
 
+// Tiles of a map whose lists count as long, kept where the clip list was (dead
+// once k_clip has run): word 0 their number, word 1 the length from which a
+// list is one, then the tiles.
+__device__ __forceinline__ uint32_t* split_tiles(const BinBufs& b, int map) {
+    return b.clip + (size_t)map * b.ccap;
+}
+
+// Entries from which a tile's list is split, for a launch of `nmaps` maps like
+// one with `total` entries: a CU's even share of the launch, and no less than
+// kSplitMin, below which the 16 passes over the list cost more than they
+// spread.  A quarter of that share (1,024 for 256 below) splits lists whose
+// tiles fill the GPU anyway: 16 visibility maps of 1024^2 (50,002 triangles)
+// 235 us against 138 us, one 4096^2 map (100,822 triangles) 58 against 48 us.
+constexpr uint32_t kSplitMin = 48;
+__device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nmaps) {
+    const unsigned long long even = total * (unsigned)nmaps / 256ull;
+    return even > kSplitMin ? (uint32_t)min(even, 0x7FFFFFFFull) : kSplitMin;
+}
+
 // Exclusive scan of one map's tile counts; resets counts to 0 (they become
-// the scatter cursors) and flags maps whose lists exceed the workspace.
-__device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map) {
+// the scatter cursors), flags maps whose lists exceed the workspace and, for
+// launches that split long lists (split_maps > 0), lists those.
+__device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map, int split_maps) {
     __shared__ unsigned long long part[kScanThreads];
+    __shared__ uint32_t nsplit;
     uint32_t* c = b.counts + (size_t)map * ntiles;
     uint32_t* o = b.offsets + (size_t)map * (ntiles + 1);
     int per = (ntiles + kScanThreads - 1) / kScanThreads;
@@ -915,6 +948,7 @@ __device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map)
     unsigned long long s = 0;
     for (int i = lo; i < hi; ++i) s += c[i];
     part[threadIdx.x] = s;
+    if (threadIdx.x == 0) nsplit = 0;
     __syncthreads();
     for (int off = 1; off < kScanThreads; off <<= 1) {
         unsigned long long v = (threadIdx.x >= (unsigned)off) ? part[threadIdx.x - off] : 0ull;
@@ -923,20 +957,37 @@ __device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map)
         __syncthreads();
     }
     unsigned long long run = part[threadIdx.x] - s;  // exclusive prefix
+    const unsigned long long total = part[kScanThreads - 1];
+    const uint32_t bound = split_maps > 0 ? split_bound(total, split_maps) : 0u;
+    uint32_t* split = split_tiles(b, map);
     for (int i = lo; i < hi; ++i) {
         o[i] = (uint32_t)run;
-        run += c[i];
+        const uint32_t n = c[i];
+        run += n;
         c[i] = 0;
+        if (split_maps > 0 && n > bound) {
+            const uint32_t at = atomicAdd(&nsplit, 1u);
+            if (at + 2 < b.ccap) split[at + 2] = (uint32_t)i;
+        }
+    }
+    if (split_maps > 0) {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const bool fits = nsplit + 2 <= b.ccap;  // else no list of this map is split
+            split[0] = fits ? nsplit : 0u;
+            split[1] = fits ? bound : ~0u;
+        }
     }
     if (threadIdx.x == kScanThreads - 1) {
-        unsigned long long total = part[kScanThreads - 1];
         bool over = total > b.cap || b.wide_over[map] != 0;
         o[ntiles] = (uint32_t)(total > b.cap ? b.cap : total);
         b.overflow[map] = over ? 1 : 0;
     }
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan(BinBufs b, int ntiles) { scan_body(b, ntiles, blockIdx.x); }
+__global__ __launch_bounds__(kScanThreads) void k_scan(BinBufs b, int ntiles, int split_maps) {
+    scan_body(b, ntiles, blockIdx.x, split_maps);
+}
 
 // ---------------------------------------------------------------------------
 // Tile raster
@@ -1090,7 +1141,7 @@ __device__ __forceinline__ unsigned long long block_mask(int rx0, int rx1, int r
         const unsigned r4 = row * 0x01010101u;
         m = ((unsigned long long)r4 << 32) | r4;
     } else {
-        m = row * 0x1111u;
+        m = row * (NB == 4 ? 0x1111u : 0x5u);
     }
     return m & (~0ull << (NB * by0)) & (~0ull >> (63 - (NB * by1 + NB - 1)));
 }
@@ -1252,26 +1303,183 @@ __device__ __forceinline__ int self_bound(int area, bool has) {
     return best;
 }
 
+// A square region of a map (a tile, or a part of a long list's tile) that a
+// workgroup rasterizes into LDS: its edge RS, its first and last pixels.
+struct Region {
+    int x0, y0, x1, y1;
+};
+template <int RS>
+__device__ __forceinline__ Region region_at(const RasterCfg& cfg, int x0, int y0) {
+    return Region{x0, y0, min(x0 + RS - 1, cfg.w - 1), min(y0 + RS - 1, cfg.h - 1)};
+}
+
+template <int RS, bool kVis>
+__device__ __forceinline__ void clear_region(typename KeyOf<kVis>::T* tile, int& nrec) {
+    constexpr int kWords = RS * tile_pitch<RS>();
+    if constexpr (!kVis) {  // 16-byte LDS writes
+        constexpr uint32_t c = KeyOf<kVis>::clear;
+        for (int q = (int)threadIdx.x; q < kWords / 4; q += kRasterThreads)
+            reinterpret_cast<uint4*>(tile)[q] = make_uint4(c, c, c, c);
+    } else {
+        for (int p = (int)threadIdx.x; p < kWords; p += kRasterThreads) tile[p] = KeyOf<kVis>::clear;
+    }
+    if (threadIdx.x == 0) nrec = 0;
+}
+
+// What a wave knows of the region's depths: lane b the bound of block b's, as
+// read `age` wave records ago.
+struct ZBound {
+    uint32_t zmax;
+    int age;
+};
+
+// One round of list entries, one per lane (`has`: the lane has one).  Small
+// records are rasterized by their lane, larger ones by the wave in 8x8
+// blocks, those of more than `aside` blocks are put aside in `rec`.
+template <int TS, int RS, bool kVis, bool kFallback, bool kBig>
+__device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
+                                             const BinBufs& b, int map, const Region& g, uint32_t entry, bool has,
+                                             int aside, typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec,
+                                             ZBound& z) {
+    const int lane = (int)threadIdx.x & 63;
+    Setup s;
+    if (has) {
+        if (!kFallback && (entry & kWideBit)) {
+            s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
+        } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
+            // a directly binned triangle: the count pass stored its setup
+            s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
+        } else {
+            float mvp[16];
+            mvps.load(map, mvp);
+            Tri<0> t;
+            if constexpr (kFallback)
+                get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, has);
+            else
+                classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, has);
+            if (has) s = to_setup(t, entry);
+        }
+    }
+    int rx0 = 0, rx1 = -1, ry0 = 0, ry1 = -1;
+    if (has) {
+        rx0 = max(g.x0, s.px0);
+        rx1 = min(g.x1, s.px1);
+        ry0 = max(g.y0, s.py0);
+        ry1 = min(g.y1, s.py1);
+        has = rx0 <= rx1 && ry0 <= ry1;
+    }
+    TileEdges t = {};
+    unsigned long long blocks = 0;
+    int area = 0;
+    if (has) {
+        t = tile_edges(s, g.x0, g.y0);
+        blocks = block_mask<RS>(rx0 - g.x0, rx1 - g.x0, ry0 - g.y0, ry1 - g.y0);
+        area = (rx1 - rx0 + 1) * (ry1 - ry0 + 1);
+        if ((kBig && !t.ok) || __popcll(blocks) > aside) {
+            const int slot = atomicAdd(&nrec, 1);
+            if (slot < kRecQueue) {
+                rec[slot] = s;
+                has = false;
+            } else if (kBig && !t.ok) {
+                raster_rect_slow<RS, kVis>(s, g.x0, g.y0, rx0, rx1, ry0, ry1, 0, 1, tile);
+                has = false;
+            }
+        }
+    }
+    const int bound = self_bound(area, has);
+    const bool self = has && area <= bound;
+    raster_lanes<RS, kVis, false>(s, t, blocks, has && !self, g.x0, g.y0, lane, z.zmax, z.age, tile);
+    if (self) raster_rect_self<RS, kVis>(s, t, g.x0, g.y0, rx0, rx1, ry0, ry1, tile);
+}
+
+// The records put aside, block rows by % 4 == wave per wave; then the region
+// is complete.  Depth maps go out with non-temporal stores: a frame writes far
+// more map bytes than the caches hold (64 x 16 MiB), and with ordinary stores
+// the last-written lines stay dirty in the MALL and are written back while
+// the screen pass reads the maps.  On the 64-sample 1080p frame this took the
+// raster from 0.363 to 0.346 ms, the soft pass that follows from 0.374 to
+// 0.341 ms and the frame from 0.991 to 0.940 ms.
+template <int RS, bool kVis, bool kBig>
+__device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region& g, void* out, int map,
+                                              typename KeyOf<kVis>::T* tile, const Setup* rec, const int& nrec,
+                                              ZBound& z) {
+    constexpr int kWaves = kRasterThreads / 64;
+    const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    __syncthreads();
+    const int nq = min(nrec, kRecQueue);
+    if (nq > 0) {  // uniform
+        Setup s;
+        TileEdges t = {};
+        unsigned long long blocks = 0;
+        const bool has = lane < nq;
+        if (has) {
+            s = rec[lane];
+            t = tile_edges(s, g.x0, g.y0);
+            unsigned long long rows = 0;
+#pragma unroll
+            for (int r = 0; r < RS / 8; r += kWaves) rows |= ((1ull << (RS / 8)) - 1ull) << ((RS / 8) * (r + wave));
+            blocks = rows & block_mask<RS>(max(g.x0, s.px0) - g.x0, min(g.x1, s.px1) - g.x0,
+                                           max(g.y0, s.py0) - g.y0, min(g.y1, s.py1) - g.y0);
+        }
+        raster_lanes<RS, kVis, true>(s, t, blocks, has && (!kBig || t.ok), g.x0, g.y0, lane, z.zmax, z.age, tile);
+        if constexpr (kBig) {
+            unsigned long long slow = __ballot(has && !t.ok);
+            while (slow) {
+                const Setup q = rec[__ffsll((long long)slow) - 1];
+                slow &= slow - 1;
+                raster_rect_slow<RS, kVis>(q, g.x0, g.y0, max(g.x0, q.px0), min(g.x1, q.px1), max(g.y0, q.py0),
+                                           min(g.y1, q.py1), tid, kRasterThreads, tile);
+            }
+        }
+        __syncthreads();
+    }
+    constexpr int kPx = RS * RS;
+    const size_t plane = (size_t)cfg.w * cfg.h;
+    if constexpr (!kVis) {
+        float* dst = reinterpret_cast<float*>(out) + (size_t)map * plane;
+        const bool full = (g.x1 - g.x0 + 1 == RS) && ((cfg.w & 3) == 0);
+        if (full) {
+            typedef float f4 __attribute__((ext_vector_type(4)));
+            for (int q = tid; q < kPx / 4; q += kRasterThreads) {
+                const int r = q / (RS / 4), cidx = (q % (RS / 4)) * 4;
+                const int j = g.y0 + r;
+                if (j > g.y1) continue;
+                const f4 v = *reinterpret_cast<const f4*>(&tile[r * tile_pitch<RS>() + cidx]);
+                __builtin_nontemporal_store(v, reinterpret_cast<f4*>(dst + (size_t)j * cfg.w + g.x0 + cidx));
+            }
+        } else {
+            for (int p = tid; p < kPx; p += kRasterThreads) {
+                const int i = g.x0 + p % RS, j = g.y0 + p / RS;
+                if (i > g.x1 || j > g.y1) continue;
+                __builtin_nontemporal_store(__uint_as_float(tile[(p / RS) * tile_pitch<RS>() + p % RS]),
+                                            dst + (size_t)j * cfg.w + i);
+            }
+        }
+    } else {
+        unsigned long long* dst = reinterpret_cast<unsigned long long*>(out) + (size_t)map * plane;
+        for (int p = tid; p < kPx; p += kRasterThreads) {
+            const int i = g.x0 + p % RS, j = g.y0 + p / RS;
+            if (i > g.x1 || j > g.y1) continue;
+            dst[(size_t)j * cfg.w + i] = tile[(p / RS) * tile_pitch<RS>() + p % RS];
+        }
+    }
+}
+
 // One (tile, map) of the raster.  kFallback: the map's lists overflowed the
 // workspace, so every (triangle, piece) pair is visited with full clipping.
 //
 // Each wave takes 64 records of every 256 (a record per lane: load, box, edge
-// values).  `spread` interleaves them, so that a short list reaches all four
-// waves: for launches that leave the GPU room (spread_lists).  Small records are rasterized by their lane, larger ones by the wave in 8x8
-// blocks; no barrier stands between the records.  Where the list is short,
-// records of many blocks (a ground plane) are put aside and covered by the
-// four waves together at the end.
+// values); no barrier stands between the rounds.  `spread` interleaves them,
+// so that a short list reaches all four waves: for launches that leave the GPU
+// room (kSpreadTiles).
 template <int TS, bool kVis, bool kFallback, bool kBig>
 __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                             const BinBufs& b, void* out, int map, int tile_id,
                                             typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec, bool spread) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int tx = tile_id % cfg.tiles_x, ty = tile_id / cfg.tiles_x;
-    constexpr int kTilePx = TS * TS;
     constexpr int kWaves = kRasterThreads / 64;
-    const int x0 = tx * TS, y0 = ty * TS;
-    const int x1 = min(x0 + TS - 1, cfg.w - 1), y1 = min(y0 + TS - 1, cfg.h - 1);
     const int ntiles = cfg.tiles_x * cfg.tiles_y;
+    const Region g = region_at<TS>(cfg, tile_id % cfg.tiles_x * TS, tile_id / cfg.tiles_x * TS);
     uint32_t begin = 0, end;
     if constexpr (!kFallback) {
         begin = b.offsets[(size_t)map * (ntiles + 1) + tile_id];
@@ -1284,17 +1492,18 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
         // centre (most tiles of a large ground plane): each depth is that
         // plane's, written straight from registers.  The LDS path would store
         // the same bits: min(clear, z) is z for every clamped depth.
-        if (end - begin == 1 && x1 - x0 + 1 == TS && y1 - y0 + 1 == TS && (cfg.w & 3) == 0) {
+        if (end - begin == 1 && g.x1 - g.x0 + 1 == TS && g.y1 - g.y0 + 1 == TS && (cfg.w & 3) == 0) {
             const uint32_t entry = b.entries[(size_t)map * b.cap + begin];
             if (entry & kWideBit) {
                 const Setup& w = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
                 const Setup s = w;
-                if (s.px0 <= x0 && s.px1 >= x1 && s.py0 <= y0 && s.py1 >= y1 && rect_inside(s, x0, x1, y0, y1)) {
+                if (s.px0 <= g.x0 && s.px1 >= g.x1 && s.py0 <= g.y0 && s.py1 >= g.y1 &&
+                    rect_inside(s, g.x0, g.x1, g.y0, g.y1)) {
                     typedef float f4 __attribute__((ext_vector_type(4)));
                     float* dst = reinterpret_cast<float*>(out) + (size_t)map * ((size_t)cfg.w * cfg.h);
-                    for (int q = tid; q < kTilePx / 4; q += kRasterThreads) {
+                    for (int q = tid; q < TS * TS / 4; q += kRasterThreads) {
                         const int r = q / (TS / 4), cidx = (q % (TS / 4)) * 4;
-                        const int i = x0 + cidx, j = y0 + r;
+                        const int i = g.x0 + cidx, j = g.y0 + r;
                         const int dy = j * 256 + 128 - s.Y[0];
                         const f4 v = {__uint_as_float(plane_bits(s, i * 256 + 128 - s.X[0], dy)),
                                       __uint_as_float(plane_bits(s, (i + 1) * 256 + 128 - s.X[0], dy)),
@@ -1307,136 +1516,102 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
             }
         }
     }
-    constexpr int kWords = TS * tile_pitch<TS>();
-    if constexpr (!kVis) {  // 16-byte LDS writes
-        constexpr uint32_t c = KeyOf<kVis>::clear;
-        for (int q = tid; q < kWords / 4; q += kRasterThreads) reinterpret_cast<uint4*>(tile)[q] = make_uint4(c, c, c, c);
-    } else {
-        for (int p = tid; p < kWords; p += kRasterThreads) tile[p] = KeyOf<kVis>::clear;
-    }
-    if (tid == 0) nrec = 0;
+    clear_region<TS, kVis>(tile, nrec);
     __syncthreads();
-    // records of more blocks than this are put aside for the four waves
     const int aside = end - begin <= (uint32_t)kShareList ? kShareBlocks : kShareBlocksLong;
-    uint32_t zmax = 0xFFFFFFFFu;  // lane b: bound of block b's depths, read `age` wave records ago
-    int age = 0;
+    ZBound z{0xFFFFFFFFu, 0};
     for (uint32_t base = begin; base < end; base += kRasterThreads) {
         const uint32_t k = base + (uint32_t)(spread ? lane * kWaves + wave : tid);
-        Setup s;
-        bool has = k < end;
-        if (has) {
-            const uint32_t entry = kFallback ? k : b.entries[(size_t)map * b.cap + k];
-            if (!kFallback && (entry & kWideBit)) {
-                s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
-            } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
-                // a directly binned triangle: the count pass stored its setup
-                s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
-            } else {
-                float mvp[16];
-                mvps.load(map, mvp);
-                Tri<0> t;
-                if constexpr (kFallback)
-                    get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, has);
-                else
-                    classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, has);
-                if (has) s = to_setup(t, entry);
-            }
-        }
-        int rx0 = 0, rx1 = -1, ry0 = 0, ry1 = -1;
-        if (has) {
-            rx0 = max(x0, s.px0);
-            rx1 = min(x1, s.px1);
-            ry0 = max(y0, s.py0);
-            ry1 = min(y1, s.py1);
-            has = rx0 <= rx1 && ry0 <= ry1;
-        }
-        TileEdges t = {};
-        unsigned long long blocks = 0;
-        int area = 0;
-        if (has) {
-            t = tile_edges(s, x0, y0);
-            blocks = block_mask<TS>(rx0 - x0, rx1 - x0, ry0 - y0, ry1 - y0);
-            area = (rx1 - rx0 + 1) * (ry1 - ry0 + 1);
-            if ((kBig && !t.ok) || __popcll(blocks) > aside) {
-                const int slot = atomicAdd(&nrec, 1);
-                if (slot < kRecQueue) {
-                    rec[slot] = s;
-                    has = false;
-                } else if (kBig && !t.ok) {
-                    raster_rect_slow<TS, kVis>(s, x0, y0, rx0, rx1, ry0, ry1, 0, 1, tile);
-                    has = false;
-                }
-            }
-        }
-        const int bound = self_bound(area, has);
-        const bool self = has && area <= bound;
-        raster_lanes<TS, kVis, false>(s, t, blocks, has && !self, x0, y0, lane, zmax, age, tile);
-        if (self) raster_rect_self<TS, kVis>(s, t, x0, y0, rx0, rx1, ry0, ry1, tile);
+        const bool has = k < end;
+        const uint32_t entry = kFallback ? k : (has ? b.entries[(size_t)map * b.cap + k] : 0u);
+        raster_round<TS, TS, kVis, kFallback, kBig>(mesh, mvps, cfg, b, map, g, entry, has, aside, tile, rec, nrec, z);
     }
-    __syncthreads();
-    const int nq = min(nrec, kRecQueue);
-    if (nq > 0) {  // uniform: the records put aside, block rows (by % 4 == wave) per wave
-        Setup s;
-        TileEdges t = {};
-        unsigned long long blocks = 0;
-        const bool has = lane < nq;
-        if (has) {
-            s = rec[lane];
-            t = tile_edges(s, x0, y0);
-            unsigned long long rows = 0;
+    finish_region<TS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z);
+}
+
+// ---------------------------------------------------------------------------
+// Long lists.  Where a launch has few tiles, one tile's list can be the whole
+// launch's time (a mesh far away, a soup in the middle of a large map: 64
+// tiles of 1,024 hold 200,000 triangles).  k_scan lists the tiles whose lists
+// are long beside the launch's average (split_bound); each is rasterized in 16
+// regions of 16x16 pixels by workgroups of their own.  A region's workgroup
+// goes through the tile's whole list, but reads only each record's box (its
+// first 16 bytes, kSplitLoads in flight per thread), and rasterizes the
+// entries that touch the region from a list in LDS.  Raster of one map, tiles
+// only and with split lists: 200k soup, 2048^2: 130 and 47 us (its G-buffer at
+// 1920x1080: 232 and 85 us); 100,822 triangles seen from 315 units, 2048^2: 98
+// and 43 us; a 3,970-triangle scene, 1024^2: 43 and 17 us, 256^2: 26 and 13 us.
+// ---------------------------------------------------------------------------
+constexpr int kSplitEdge = 16;
+constexpr int kSplitRegions = (kTile / kSplitEdge) * (kTile / kSplitEdge);
+constexpr int kSplitLoads = 8;                              // entries per thread and pass over the list
+constexpr int kSplitPass = kSplitLoads * kRasterThreads;    // entries a pass looks at, and its LDS list's size
+
+// The region list in LDS, behind the region's pixels in the tile's memory.
+template <int TS, bool kVis>
+__device__ __forceinline__ uint32_t* split_list(typename KeyOf<kVis>::T* tile) {
+    static_assert((size_t)(TS * tile_pitch<TS>() - kSplitEdge * tile_pitch<kSplitEdge>()) *
+                          sizeof(typename KeyOf<kVis>::T) >= (size_t)kSplitPass * 4, "the list fits behind the region");
+    return reinterpret_cast<uint32_t*>(tile + kSplitEdge * tile_pitch<kSplitEdge>());
+}
+
+template <int TS, bool kVis, bool kBig>
+__device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
+                                              const BinBufs& b, void* out, int map, int tile_id, int part,
+                                              typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec, int& nlist) {
+    constexpr int kParts = TS / kSplitEdge, RS = kSplitEdge, kWaves = kRasterThreads / 64;
+    const int tid = (int)threadIdx.x;
+    const int ntiles = cfg.tiles_x * cfg.tiles_y;
+    const Region g = region_at<RS>(cfg, tile_id % cfg.tiles_x * TS + part % kParts * RS,
+                                   tile_id / cfg.tiles_x * TS + part / kParts * RS);
+    if (g.x0 >= cfg.w || g.y0 >= cfg.h) return;  // uniform
+    const uint32_t begin = b.offsets[(size_t)map * (ntiles + 1) + tile_id];
+    const uint32_t end = b.offsets[(size_t)map * (ntiles + 1) + tile_id + 1];
+    const uint32_t* entries = b.entries + (size_t)map * b.cap;
+    uint32_t* list = split_list<TS, kVis>(tile);
+    clear_region<RS, kVis>(tile, nrec);
+    ZBound z{0xFFFFFFFFu, 0};
+    for (uint32_t base = begin; base < end; base += kSplitPass) {
+        if (tid == 0) nlist = 0;
+        __syncthreads();  // also: the region is cleared, the last pass's list is done with
+        uint32_t e[kSplitLoads];
 #pragma unroll
-            for (int r = 0; r < TS / 8; r += kWaves) rows |= ((1ull << (TS / 8)) - 1ull) << ((TS / 8) * (r + wave));
-            blocks = rows & block_mask<TS>(max(x0, s.px0) - x0, min(x1, s.px1) - x0, max(y0, s.py0) - y0,
-                                           min(y1, s.py1) - y0);
+        for (int q = 0; q < kSplitLoads; ++q) {
+            const uint32_t k = base + (uint32_t)(q * kRasterThreads + tid);
+            e[q] = k < end ? entries[k] : ~0u;
         }
-        raster_lanes<TS, kVis, true>(s, t, blocks, has && (!kBig || t.ok), x0, y0, lane, zmax, age, tile);
-        if constexpr (kBig) {
-            unsigned long long slow = __ballot(has && !t.ok);
-            while (slow) {
-                const Setup q = rec[__ffsll((long long)slow) - 1];
-                slow &= slow - 1;
-                raster_rect_slow<TS, kVis>(q, x0, y0, max(x0, q.px0), min(x1, q.px1), max(y0, q.py0), min(y1, q.py1),
-                                           tid, kRasterThreads, tile);
+        bool hit[kSplitLoads];
+#pragma unroll
+        for (int q = 0; q < kSplitLoads; ++q) {
+            hit[q] = false;
+            if (e[q] == ~0u) continue;
+            int px0, px1, py0, py1;
+            if (e[q] & kWideBit) {
+                const Setup& w = b.wide[(size_t)map * b.wcap + (e[q] & ~kWideBit)];
+                px0 = w.px0;
+                px1 = w.px1;
+                py0 = w.py0;
+                py1 = w.py1;
+            } else {
+                const SetupRec& r = b.setups[(size_t)map * b.tstride + (e[q] >> 3)];
+                rec_box(r.X0, r.Y0, r.d1, r.d2, px0, px1, py0, py1);
             }
+            hit[q] = px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0;
         }
+#pragma unroll
+        for (int q = 0; q < kSplitLoads; ++q)
+            if (hit[q]) list[atomicAdd(&nlist, 1)] = e[q];
         __syncthreads();
-    }
-    // Write the tile once.  Depth maps go out with non-temporal stores: a
-    // frame writes far more map bytes than the caches hold (64 x 16 MiB), and
-    // with ordinary stores the last-written lines stay dirty in the MALL and
-    // are written back while the screen pass reads the maps.  On the
-    // 64-sample 1080p frame this took the raster from 0.363 to 0.346 ms, the
-    // soft pass that follows from 0.374 to 0.341 ms and the frame from 0.991
-    // to 0.940 ms.
-    const size_t plane = (size_t)cfg.w * cfg.h;
-    if constexpr (!kVis) {
-        float* dst = reinterpret_cast<float*>(out) + (size_t)map * plane;
-        const bool full = (x1 - x0 + 1 == TS) && ((cfg.w & 3) == 0);
-        if (full) {
-            typedef float f4 __attribute__((ext_vector_type(4)));
-            for (int q = tid; q < kTilePx / 4; q += kRasterThreads) {
-                const int r = q / (TS / 4), cidx = (q % (TS / 4)) * 4;
-                const int j = y0 + r;
-                if (j > y1) continue;
-                const f4 v = *reinterpret_cast<const f4*>(&tile[r * tile_pitch<TS>() + cidx]);
-                __builtin_nontemporal_store(v, reinterpret_cast<f4*>(dst + (size_t)j * cfg.w + x0 + cidx));
-            }
-        } else {
-            for (int p = tid; p < kTilePx; p += kRasterThreads) {
-                const int i = x0 + p % TS, j = y0 + p / TS;
-                if (i > x1 || j > y1) continue;
-                __builtin_nontemporal_store(__uint_as_float(tile[(p / TS) * tile_pitch<TS>() + p % TS]),
-                                            dst + (size_t)j * cfg.w + i);
-            }
+        const int n = nlist;
+        for (int k0 = 0; k0 < n; k0 += kRasterThreads) {
+            const int k = k0 + (tid & 63) * kWaves + (tid >> 6);
+            const bool has = k < n;
+            raster_round<TS, RS, kVis, false, kBig>(mesh, mvps, cfg, b, map, g, has ? list[k] : 0u, has,
+                                                    (RS / 8) * (RS / 8), tile, rec, nrec, z);
         }
-    } else {
-        unsigned long long* dst = reinterpret_cast<unsigned long long*>(out) + (size_t)map * plane;
-        for (int p = tid; p < kTilePx; p += kRasterThreads) {
-            const int i = x0 + p % TS, j = y0 + p / TS;
-            if (i > x1 || j > y1) continue;
-            dst[(size_t)j * cfg.w + i] = tile[(p / TS) * tile_pitch<TS>() + p % TS];
-        }
+        __syncthreads();  // nlist and the list are rewritten by the next pass
     }
+    finish_region<RS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z);
 }
 
 // Binned raster: one workgroup per (tile, map); overflowed maps are left to
@@ -1448,8 +1623,10 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
 // rest idle.  Tile-major order spreads each costly tile's maps over the XCDs
 // and CUs.
 template <int TS, bool kVis, bool kBig>
-__global__ __launch_bounds__(kRasterThreads, kVis || kBig ? 1 : 8) void k_raster(MeshView mesh, MvpSource mvps, RasterCfg cfg, BinBufs b,
-                                                           void* out, int map_base, int map_count, bool spread) {
+__global__ __launch_bounds__(kRasterThreads, kVis || kBig ? 1 : 8) void k_raster(MeshView mesh, MvpSource mvps,
+                                                                                 RasterCfg cfg, BinBufs b, void* out,
+                                                                                 int map_base, int map_count,
+                                                                                 bool spread) {
     __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
@@ -1457,6 +1634,55 @@ __global__ __launch_bounds__(kRasterThreads, kVis || kBig ? 1 : 8) void k_raster
     const int tile_id = (int)(blockIdx.x / (unsigned)map_count);
     if (b.overflow[map]) return;
     raster_tile<TS, kVis, false, kBig>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, spread);
+}
+
+// k_raster for launches that split long lists: the first workgroups take a
+// (tile, map) each, and of a split tile its first region; kSplitWorkers more
+// take the other regions in turn.
+constexpr int kSplitWorkers = 1024;
+template <int TS, bool kVis, bool kBig>
+__global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, MvpSource mvps, RasterCfg cfg,
+                                                                 BinBufs b, void* out, int map_base, int map_count) {
+    __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
+    __shared__ Setup rec[kRecQueue];
+    __shared__ int nrec, nlist;
+    const int ntiles = cfg.tiles_x * cfg.tiles_y;
+    const int bid = (int)blockIdx.x - kSplitWorkers;  // the regions first: they are the long ones
+    int map = 0, tile_id = 0, part = 0;
+    // the workers' walk: lane m holds the tasks of map m (at most 64 maps)
+    int tasks = 0, m = 0, first = 0, t = (int)blockIdx.x;
+    if (bid >= 0) {
+        map = map_base + bid % map_count;
+        tile_id = bid / map_count;
+        if (b.overflow[map]) return;
+        const uint32_t* o = b.offsets + (size_t)map * (ntiles + 1) + tile_id;
+        if (o[1] - o[0] <= split_tiles(b, map)[1]) {
+            raster_tile<TS, kVis, false, kBig>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, true);
+            return;
+        }
+    } else {
+        const int lane = (int)threadIdx.x & 63;
+        if (lane < map_count && !b.overflow[map_base + lane])
+            tasks = (int)split_tiles(b, map_base + lane)[0] * (kSplitRegions - 1);
+    }
+    for (;;) {
+        if (bid < 0) {
+            int n = __builtin_amdgcn_readlane(tasks, m);
+            while (t >= n) {  // uniform: on to the next map with a task for this worker
+                first = (first + n) % kSplitWorkers;
+                if (++m == map_count) return;
+                t = ((int)blockIdx.x + kSplitWorkers - first) % kSplitWorkers;
+                n = __builtin_amdgcn_readlane(tasks, m);
+            }
+            map = map_base + m;
+            tile_id = (int)split_tiles(b, map)[2 + t / (kSplitRegions - 1)];
+            part = 1 + t % (kSplitRegions - 1);
+            t += kSplitWorkers;
+        }
+        raster_region<TS, kVis, kBig>(mesh, mvps, cfg, b, out, map, tile_id, part, tile, rec, nrec, nlist);
+        if (bid >= 0) return;
+        __syncthreads();  // the region's LDS is used again
+    }
 }
 
 // One workgroup per tile, looping over the maps whose lists overflowed.
