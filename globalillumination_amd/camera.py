@@ -18,8 +18,8 @@ def _f16() -> np.ndarray:
 
 
 def _ptr(a: np.ndarray) -> ctypes.c_void_p:
-    assert a.dtype == np.float32 and a.flags["C_CONTIGUOUS"]
-    return ctypes.c_void_p(a.ctypes.data)
+    assert a.dtype == np.float32 and a.flags.c_contiguous
+    return ctypes.c_void_p(a.__array_interface__["data"][0])
 
 
 def perspective(fovy_deg: float, aspect: float, znear: float, zfar: float) -> np.ndarray:
