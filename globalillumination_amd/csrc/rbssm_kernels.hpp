@@ -568,6 +568,8 @@ __global__ __launch_bounds__(kBlockThreads) void k_rbssm_classify(GBufferView gb
                                                                    PcssUniforms q, float* __restrict__ out,
                                                                    unsigned* __restrict__ counters,
                                                                    uint2* __restrict__ list) {
+    __shared__ float off[64];
+    const int nb = pcss_offsets(q.bfw, q.bsw, off);
     int x, y;
     pixel_of_block(gb.w, gb.h, x, y);
     bool loop = false;
@@ -587,7 +589,7 @@ __global__ __launch_bounds__(kBlockThreads) void k_rbssm_classify(GBufferView gb
             if (u.pre_eval)
                 shadow = pre_evaluation(u, vx, vy, vz, gb.nrm[k], gb.nrm[plane + k], gb.nrm[2 * plane + k]);
             if (sc[3] > 0.0f && shadow == 1.0f) {
-                const float avg = pcss_blocker(D, q, n0, n1, n2);
+                const float avg = pcss_blocker(D, off, nb, n0, n1, n2);
                 pw = pcss_penumbra(q, avg, n2);
                 const float stepSize = 2.0f * pw / (float)q.ks;
                 loop = !(stepSize <= 0.0f || stepSize >= 1.0f);

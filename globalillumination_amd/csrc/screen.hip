@@ -439,7 +439,8 @@ int gi_pcss_pass(const gi_gbuffer* gbuffer, const float* depth_dev, const gi_pcs
     DepthMap D{depth_dev, p->shadow_map_width, p->shadow_map_height, (float)p->shadow_map_width,
                (float)p->shadow_map_height};
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    hipLaunchKernelGGL(k_pcss, grid_for(gb.w, gb.h), dim3(kBlockThreads), 0, s, gb, D, u, q, out_dev);
+    hipLaunchKernelGGL(k_pcss, grid_for(gb.w, gb.h), dim3(kBlockThreads), pcss_table_bytes(q), s, gb, D, u, q,
+                       out_dev);
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
 
