@@ -5,27 +5,27 @@
 // camera G-buffer, soft-shadow parameters), each the work of one
 // renderMonteCarlo frame (SoftShadowMapping/src/main.cpp:756-811).  Instead
 // of a launch sequence per instance, every stage of the depth pass runs as one
-// persistent kernel over all instances' work items, and the screen pass as one
-// persistent kernel per PCF variant:
-//   kb_zero, kb_fill       clear the bin counters of every instance and the
-//                          work-queue counters;
+// kernel over all instances' work items, and the screen pass as one kernel per
+// PCF variant:
+//   kb_zero, kb_fill       clear the overflow flag and the bin counters of
+//                          every instance;
 //   kb_bin, kb_clip,       binning (count), clipping, wide records, scan and
 //   kb_bin_wide, kb_scan,  binning (scatter), over (instance, map, triangle
 //   kb_bin, kb_bin_wide    block) items in a fixed stride;
-//   kb_raster              (instance, map, tile) items from a work queue;
+//   kb_raster              a workgroup per (instance, tile, map);
 //   kb_raster_fallback     overflowed maps;
-//   kb_soft                (instance, pixel block) items from per-XCD work
-//                          queues, each XCD draining a contiguous,
-//                          cost-balanced range so its L2 serves neighbouring
-//                          pixels.
+//   kb_soft                a workgroup per (instance, pixel block), each XCD
+//                          taking a contiguous, cost-balanced range so its L2
+//                          serves neighbouring pixels.
 // The per-item work is the single-instance kernels' own device code
 // (raster_kernels.hpp, screen_kernels.hpp), so every map and shadow value is
 // bit-identical to gi_depth_pass + gi_soft_shadow_pass per instance.  The
 // plan's launches can be captured in one hipGraph; gi_batch_autotune picks the
-// raster tile edge, the screen block shape and the persistent grid sizes by
-// measurement.
+// raster tile edge, the screen block shape and the binning stages' grid size
+// by measurement.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <cstring>
@@ -46,9 +46,7 @@ constexpr int kScreenThreads = 256;
 constexpr int kNtGroups = 3;  // soft variants: generic loop, 3 taps per axis, 4 taps per axis
 constexpr int kShapes = 5;    // screen blocks 64x4, 32x8, 16x16 (row-major waves), 16x16 of 8x8 wave
                               // tiles, 64x4 of 16x4 wave tiles
-constexpr int kCounters = 64;  // [0] raster queue, [1] a map of the depth run overflowed (until the
-                               // screen run clears it), [1 + 8 g + x] screen queue of group g on XCD x,
-                               // [63] the autotuner's overflow flag
+constexpr int kCounters = 2;  // [0] a map of the depth run overflowed, [1] scratch of overflowed()
 
 struct RasterJob {
     MeshView mesh;
@@ -66,7 +64,7 @@ struct RasterTable {
     const RasterJob* jobs;
     const uint32_t* prefix;  // kStages x (njobs + 1): items of each stage per job, exclusive prefix
     int njobs;
-    uint32_t* counter;       // [0] raster work queue, [1] set when a map overflowed
+    uint32_t* counter;       // [0] set when a map overflowed
 };
 
 struct SoftJob {
@@ -84,7 +82,6 @@ struct SoftTable {
     const uint32_t* prefix;  // njobs + 1
     int njobs;
     const uint32_t* xr;      // [2 x, 2 x + 1]: item range of XCD x
-    uint32_t* counters;      // one per XCD
 };
 
 // Job holding work item `item` (largest j with pre[j] <= item; jobs without
@@ -213,7 +210,7 @@ __global__ __launch_bounds__(kScanThreads) void kb_scan(RasterTable t) {
         scan_body(J.b, J.ntiles, map, 0);
         // the thread that decided the map's overflow raises the batch's flag
         // (kb_raster_fallback does nothing without it)
-        if (threadIdx.x == kScanThreads - 1 && J.b.overflow[map]) t.counter[1] = 1u;
+        if (threadIdx.x == kScanThreads - 1 && J.b.overflow[map]) t.counter[0] = 1u;
         __syncthreads();
     }
 }
@@ -229,28 +226,26 @@ __global__ void kb_overflow_any(RasterTable t, uint32_t* __restrict__ flag) {
     }
 }
 
-// (instance, map, tile) items from a work queue: tiles differ widely in cost.
+// One workgroup per (instance, tile, map) item, from item `first` on; the
+// maps of a tile lie side by side (k_raster's order, for its reason).  The
+// hardware hands out workgroups as they fit, which balances the tiles' widely
+// different costs with no queue of ours: a workgroup of a queue holds its
+// place on the CU through the chain of counter, job and list loads of each
+// item.  Twelve frames of soups (512^2 to 4096^2 maps): 2.79 ms from a queue
+// with 8 workgroups per CU, 2.20 ms so.
 template <int TS, bool kBig>
-__global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_raster(RasterTable t) {
+__global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_raster(RasterTable t, uint32_t first) {
     __shared__ __align__(16) uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
-    __shared__ uint32_t s_item;
     const uint32_t* pre = t.prefix + kStRaster * (t.njobs + 1);
-    const uint32_t total = pre[t.njobs];
-    for (;;) {
-        if (threadIdx.x == 0) s_item = atomicAdd(t.counter, 1u);
-        __syncthreads();
-        const uint32_t item = s_item;
-        __syncthreads();
-        if (item >= total) break;  // uniform: every workgroup ends once the queue is drained
-        const int j = find_job(pre, t.njobs, item);
-        const RasterJob& J = t.jobs[j];
-        const uint32_t local = item - pre[j];
-        const int map = (int)(local / J.ntiles), tile_id = (int)(local % J.ntiles);
-        if (J.b.overflow[map]) continue;  // left to kb_raster_fallback
-        raster_tile<TS, false, false, kBig>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, false);
-    }
+    const uint32_t item = first + blockIdx.x;
+    const int j = find_job(pre, t.njobs, item);
+    const RasterJob& J = t.jobs[j];
+    const uint32_t local = item - pre[j];
+    const int map = (int)(local % (uint32_t)J.nmaps), tile_id = (int)(local / (uint32_t)J.nmaps);
+    if (J.b.overflow[map]) return;  // left to kb_raster_fallback
+    raster_tile<TS, false, false, kBig>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, false);
 }
 
 template <int TS>
@@ -258,7 +253,7 @@ __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable
     __shared__ uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
-    if (t.counter[1] == 0u) return;  // no map overflowed (kb_scan)
+    if (t.counter[0] == 0u) return;  // no map overflowed (kb_scan)
     const uint32_t* pre = t.prefix + kStFallback * (t.njobs + 1);
     const uint32_t total = pre[t.njobs];
     for (uint32_t item = blockIdx.x; item < total; item += gridDim.x) {
@@ -274,15 +269,19 @@ __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable
     }
 }
 
-// (instance, pixel block) items.  XCD x (hardware hands consecutive
-// workgroups to the XCDs round-robin) drains items [xr[2x], xr[2x+1]) through
-// its own queue.
+// One workgroup per (instance, pixel block) item.  XCD x (hardware hands
+// consecutive workgroups to the XCDs round-robin) takes items [xr[2x],
+// xr[2x+1]), from number `first` of each range on.  The pass waits for its
+// gathers, so it wants every wave the registers allow (8 per SIMD) and no wave
+// waiting for the slowest of a workgroup's before the next item: twelve frames
+// (640x480 to 1920x1080, 1-16 samples) take 295 us, 813 us from per-XCD queues
+// with 4 workgroups per CU.
 template <int NT, int BX, int BY, bool kWaveTiles>
-__global__ __launch_bounds__(kScreenThreads) void kb_soft(SoftTable t) {
+__global__ __launch_bounds__(kScreenThreads) void kb_soft(SoftTable t, uint32_t first) {
     static_assert(BX * BY == kScreenThreads, "block shape");
-    __shared__ uint32_t s_item;
     const int xcd = (int)(blockIdx.x % kXcds);
-    const uint32_t lo = t.xr[2 * xcd], hi = t.xr[2 * xcd + 1];
+    const uint32_t item = t.xr[2 * xcd] + first + blockIdx.x / kXcds;
+    if (item >= t.xr[2 * xcd + 1]) return;
     int tx = (int)threadIdx.x % BX, ty = (int)threadIdx.x / BX;
     if constexpr (kWaveTiles && BX == 64) {  // four 16x4 wave tiles side by side
         tx = ((int)threadIdx.x >> 6) * 16 + ((int)threadIdx.x & 15);
@@ -290,18 +289,11 @@ __global__ __launch_bounds__(kScreenThreads) void kb_soft(SoftTable t) {
     } else if constexpr (kWaveTiles) {
         wave_tile_xy((int)threadIdx.x, tx, ty);
     }
-    for (;;) {
-        if (threadIdx.x == 0) s_item = lo + atomicAdd(&t.counters[xcd], 1u);
-        __syncthreads();
-        const uint32_t item = s_item;
-        __syncthreads();
-        if (item >= hi) break;  // uniform: every workgroup ends once its range is drained
-        const int j = find_job(t.prefix, t.njobs, item);
-        const SoftJob& J = t.jobs[j];
-        const uint32_t local = item - t.prefix[j];
-        const int x = (int)(local % (uint32_t)J.bx_n) * BX + tx, y = (int)(local / (uint32_t)J.bx_n) * BY + ty;
-        if (x < J.gb.w && y < J.gb.h) soft_pixel<NT>(J.gb, J.maps, J.smw, J.smh, J.trans, J.u, J.out, x, y);
-    }
+    const int j = find_job(t.prefix, t.njobs, item);
+    const SoftJob& J = t.jobs[j];
+    const uint32_t local = item - t.prefix[j];
+    const int x = (int)(local % (uint32_t)J.bx_n) * BX + tx, y = (int)(local / (uint32_t)J.bx_n) * BY + ty;
+    if (x < J.gb.w && y < J.gb.h) soft_pixel<NT>(J.gb, J.maps, J.smw, J.smh, J.trans, J.u, J.out, x, y);
 }
 
 // ---------------------------------------------------------------------------
@@ -380,6 +372,7 @@ struct SoftGroup {
     const uint32_t* prefix;
     const uint32_t* xr;
     int njobs;
+    uint32_t longest;  // items of the longest XCD range
 };
 
 }  // namespace
@@ -425,12 +418,19 @@ void launch_scatter(const RasterVariant& R, const RasterTable& tab, char* ws, un
     }
 }
 
+// Workgroups per launch of the one-per-item stages: a grid's threads are
+// counted in 32 bits.
+constexpr uint32_t kMaxGroups = 1u << 23;
+
 template <int TS>
-void launch_raster(unsigned grid, const RasterTable& tab, bool big, hipStream_t s) {
-    if (big)
-        hipLaunchKernelGGL((kb_raster<TS, true>), dim3(grid), dim3(kRasterThreads), 0, s, tab);
-    else
-        hipLaunchKernelGGL((kb_raster<TS, false>), dim3(grid), dim3(kRasterThreads), 0, s, tab);
+void launch_raster(uint32_t total, const RasterTable& tab, bool big, hipStream_t s) {
+    for (uint32_t first = 0; first < total; first += kMaxGroups) {
+        const dim3 grid(total - first < kMaxGroups ? total - first : kMaxGroups);
+        if (big)
+            hipLaunchKernelGGL((kb_raster<TS, true>), grid, dim3(kRasterThreads), 0, s, tab, first);
+        else
+            hipLaunchKernelGGL((kb_raster<TS, false>), grid, dim3(kRasterThreads), 0, s, tab, first);
+    }
 }
 
 int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
@@ -438,7 +438,7 @@ int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
     const RasterVariant& R = b->rv[v];
     RasterTable tab{R.jobs, R.prefix, b->n, b->counters};
     const unsigned cap = (unsigned)(b->ncu * T.raster_groups);
-    hipLaunchKernelGGL(kb_zero, dim3(1), dim3(kCounters), 0, s, b->counters, 2);
+    hipLaunchKernelGGL(kb_zero, dim3(1), dim3(64), 0, s, b->counters, 1);
     unsigned g;
     if ((g = grid_of(R.total[kStFill], cap))) hipLaunchKernelGGL(kb_fill, dim3(g), dim3(256), 0, s, tab);
 #define GI_DEPTH_STAGES(TS)                                                                                        \
@@ -451,8 +451,7 @@ int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
     launch_scatter<TS>(R, tab, b->ws, cap, s);                                                                     \
     if ((g = grid_of(R.total[kStWide], cap)))                                                                       \
         hipLaunchKernelGGL((kb_bin_wide<TS, true>), dim3(g), dim3(256), 0, s, tab);                                 \
-    if ((g = grid_of(R.total[kStRaster], cap)))                                                                     \
-        launch_raster<TS>(g, tab, b->big, s);                                                                       \
+    launch_raster<TS>(R.total[kStRaster], tab, b->big, s);                                                          \
     if ((g = grid_of(R.total[kStFallback], cap)))                                                                   \
         hipLaunchKernelGGL((kb_raster_fallback<TS>), dim3(g), dim3(kRasterThreads), 0, s, tab);
     if (T.tile == 32) {
@@ -465,28 +464,28 @@ int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
 }
 
 template <int NT>
-void launch_soft(int shape, unsigned grid, const SoftTable& tab, hipStream_t s) {
+void launch_soft(int shape, unsigned grid, const SoftTable& tab, uint32_t first, hipStream_t s) {
     switch (shape) {
-    case 0: hipLaunchKernelGGL((kb_soft<NT, 64, 4, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab); break;
-    case 1: hipLaunchKernelGGL((kb_soft<NT, 32, 8, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab); break;
-    case 2: hipLaunchKernelGGL((kb_soft<NT, 16, 16, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab); break;
-    case 3: hipLaunchKernelGGL((kb_soft<NT, 16, 16, true>), dim3(grid), dim3(kScreenThreads), 0, s, tab); break;
-    default: hipLaunchKernelGGL((kb_soft<NT, 64, 4, true>), dim3(grid), dim3(kScreenThreads), 0, s, tab); break;
+    case 0: hipLaunchKernelGGL((kb_soft<NT, 64, 4, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab, first); break;
+    case 1: hipLaunchKernelGGL((kb_soft<NT, 32, 8, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab, first); break;
+    case 2: hipLaunchKernelGGL((kb_soft<NT, 16, 16, false>), dim3(grid), dim3(kScreenThreads), 0, s, tab, first); break;
+    case 3: hipLaunchKernelGGL((kb_soft<NT, 16, 16, true>), dim3(grid), dim3(kScreenThreads), 0, s, tab, first); break;
+    default: hipLaunchKernelGGL((kb_soft<NT, 64, 4, true>), dim3(grid), dim3(kScreenThreads), 0, s, tab, first); break;
     }
 }
 
 int run_screen(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
-    hipLaunchKernelGGL(kb_zero, dim3(1), dim3(kCounters), 0, s, b->counters + 1, kCounters - 1);
-    unsigned grid = (unsigned)(b->ncu * T.screen_groups);
-    grid = (grid + kXcds - 1) / kXcds * kXcds;
     for (int g = 0; g < kNtGroups; ++g) {
         const SoftGroup& G = b->sg[T.screen_shape][g];
         if (G.njobs == 0) continue;
-        SoftTable tab{G.jobs, G.prefix, G.njobs, G.xr, b->counters + 1 + kXcds * g};
-        switch (kGroupNt[g]) {
-        case 3: launch_soft<3>(T.screen_shape, grid, tab, s); break;
-        case 4: launch_soft<4>(T.screen_shape, grid, tab, s); break;
-        default: launch_soft<0>(T.screen_shape, grid, tab, s); break;
+        SoftTable tab{G.jobs, G.prefix, G.njobs, G.xr};
+        for (uint32_t first = 0; first < G.longest; first += kMaxGroups / kXcds) {
+            const unsigned grid = kXcds * (G.longest - first < kMaxGroups / kXcds ? G.longest - first : kMaxGroups / kXcds);
+            switch (kGroupNt[g]) {
+            case 3: launch_soft<3>(T.screen_shape, grid, tab, first, s); break;
+            case 4: launch_soft<4>(T.screen_shape, grid, tab, first, s); break;
+            default: launch_soft<0>(T.screen_shape, grid, tab, first, s); break;
+            }
         }
     }
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
@@ -496,8 +495,8 @@ int run_screen(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
 int overflowed(gi_batch* b, const gi_batch_tuning& T, hipStream_t s, bool* any) {
     const RasterVariant& R = b->rv[T.tile == 32 ? 0 : 1];
     RasterTable tab{R.jobs, R.prefix, b->n, b->counters};
-    uint32_t* flag = b->counters + kCounters - 1;  // not used by the screen queues of the groups
-    hipLaunchKernelGGL(kb_zero, dim3(1), dim3(kCounters), 0, s, flag, 1);
+    uint32_t* flag = b->counters + kCounters - 1;
+    hipLaunchKernelGGL(kb_zero, dim3(1), dim3(64), 0, s, flag, 1);
     hipLaunchKernelGGL(kb_overflow_any, dim3(64), dim3(256), 0, s, tab, flag);
     uint32_t h = 0;
     if (hipMemcpyAsync(&h, flag, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess) return GI_EDEVICE;
@@ -673,9 +672,11 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
                 if (x > 0) xr[2 * (x - 1) + 1] = item;
                 if (x < kXcds) xr[2 * x] = item;
             }
+            uint32_t longest = 0;
+            for (int x = 0; x < kXcds; ++x) longest = std::max(longest, xr[2 * x + 1] - xr[2 * x]);
             b->sg[sh][g] = SoftGroup{reinterpret_cast<const SoftJob*>(base + L.sjobs[sh][g]),
                                      reinterpret_cast<const uint32_t*>(base + L.sprefix[sh][g]),
-                                     reinterpret_cast<const uint32_t*>(base + L.sxr[sh][g]), nj};
+                                     reinterpret_cast<const uint32_t*>(base + L.sxr[sh][g]), nj, longest};
         }
     }
     if (hipMemcpy(base, img.data(), img.size(), hipMemcpyHostToDevice) != hipSuccess) {
@@ -725,19 +726,16 @@ int gi_batch_autotune(gi_batch* b, gi_stream stream, int reps, gi_batch_tuning* 
             }
         }
     // the maps of the last depth run stay in place for the screen candidates
-    for (int sh = 0; sh < kShapes; ++sh)
-        for (int k = 0; k < 4; ++k) {
-            T.screen_shape = sh;
-            T.screen_groups = groups[k];
-            float ms = 0.0f;
-            int rc = timed(b, T, s, reps, false, &ms);
-            if (rc != GI_OK) return rc;
-            if (ms < best_s) {
-                best_s = ms;
-                bestT.screen_shape = sh;
-                bestT.screen_groups = groups[k];
-            }
+    for (int sh = 0; sh < kShapes; ++sh) {
+        T.screen_shape = sh;
+        float ms = 0.0f;
+        int rc = timed(b, T, s, reps, false, &ms);
+        if (rc != GI_OK) return rc;
+        if (ms < best_s) {
+            best_s = ms;
+            bestT.screen_shape = sh;
         }
+    }
     b->tuning = bestT;
     if (best) *best = bestT;
     if (best_ms) *best_ms = best_r + best_s;
