@@ -231,8 +231,8 @@ __global__ void kb_overflow_any(RasterTable t, uint32_t* __restrict__ flag) {
 // hardware hands out workgroups as they fit, which balances the tiles' widely
 // different costs with no queue of ours: a workgroup of a queue holds its
 // place on the CU through the chain of counter, job and list loads of each
-// item.  Twelve frames of soups (512^2 to 4096^2 maps): 2.79 ms from a queue
-// with 8 workgroups per CU, 2.20 ms so.
+// item.  Twelve frames of soups (512^2 to 4096^2 maps): 2.74 ms from a queue
+// with 8 workgroups per CU, 2.01 ms so.
 template <int TS, bool kBig>
 __global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_raster(RasterTable t, uint32_t first) {
     __shared__ __align__(16) uint32_t tile[TS * tile_pitch<TS>()];

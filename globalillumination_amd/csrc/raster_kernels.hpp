@@ -29,7 +29,7 @@ constexpr int kMaxPoly = 9;
 // 160 KiB (7 of 20,484 bytes ran 3% slower).
 constexpr int kRecQueue = 28;  // LDS setup records that a workgroup puts aside
 constexpr int kShareList = 128;   // entries up to which a tile's list counts as short
-constexpr int kShareBlocks = 16;      // blocks over which a record of a short list is put aside
+constexpr int kShareBlocks = 4;       // blocks over which a record of a short list is put aside
 constexpr int kShareBlocksLong = 44;  // and of a long one
 constexpr int kScanThreads = 1024;
 
@@ -1153,6 +1153,18 @@ __device__ __forceinline__ int in_vector(int v) {
     return v;
 }
 
+// The same for a scalar register.
+__device__ __forceinline__ int in_scalar(int v) {
+    asm("" : "+s"(v));
+    return v;
+}
+// a * b + c of factors of 24 bits (tile_edges), b wave-uniform.
+__device__ __forceinline__ int mad24(int a, int b, int c) {
+    int r;
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(b), "v"(c));
+    return r;
+}
+
 // Lane b: the largest depth (as bits) that block b of the tile holds now.
 // Depths only fall, so a value that other waves have lowered since is still an
 // upper bound.  The lanes start at different rows and halves of their blocks,
@@ -1186,12 +1198,13 @@ __device__ __forceinline__ uint32_t block_zmax(int lane, const typename KeyOf<kV
 // wave-uniform): lane b first tests block b of the tile against the three
 // edges (the block's pixel nearest to each edge's inside) and against the
 // depth the block already has (zmax, block_zmax's), then the blocks left are
-// taken row by row, a lane per pixel, 12 vector instructions each.  The
+// taken row by row, a lane per pixel, 13 vector instructions each.  The
 // record's smallest depth in a block is that of the corner pixel its plane
 // falls to: every rounded step of the depth expression is monotonic in dx and
 // in dy, so no pixel of the block comes out below it.
 // kWhole: blocks that lie inside all three edges (most of a ground plane's)
-// are taken without edge tests.
+// are taken in a loop of their own, with no edge tests and no lane masking (8
+// vector and 6 scalar instructions each).
 template <int TS, bool kVis, bool kWhole>
 __device__ __forceinline__ void raster_blocks(const int er[3], const int ex[3], const int ey[3], float z0, float A,
                                               float B, float zoff, int dx0, int dy0, uint32_t id,
@@ -1203,11 +1216,12 @@ __device__ __forceinline__ void raster_blocks(const int er[3], const int ex[3], 
     int near[3], off[3], step[3], inner[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        const int far = er[k] + max(0, 7 * ex[k]) + max(0, -7 * ey[k]);
-        near[k] = far + __mul24(bly, ex[k]) - __mul24(blx, ey[k]);
-        if constexpr (kWhole) inner[k] = near[k] - 7 * (abs(ex[k]) + abs(ey[k]));
-        off[k] = in_vector(er[k] + __mul24(ly, ex[k]) - __mul24(lx, ey[k]));
         step[k] = in_vector(-ey[k]);
+        const int ny = -ey[k];
+        const int far = er[k] + max(0, 7 * ex[k]) + max(0, -7 * ey[k]);
+        near[k] = mad24(blx, ny, mad24(bly, ex[k], in_vector(far)));
+        if constexpr (kWhole) inner[k] = near[k] - in_scalar(7 * (abs(ex[k]) + abs(ey[k])));
+        off[k] = mad24(lx, ny, mad24(ly, ex[k], in_vector(er[k])));
     }
     const uint32_t zmin =
         window_bits(z0 + (A * (float)(dx0 + (blx + (A < 0.0f ? 7 : 0)) * 256) +
@@ -1218,21 +1232,30 @@ __device__ __forceinline__ void raster_blocks(const int er[3], const int ex[3], 
     if constexpr (kWhole) whole = __ballot((inner[0] | inner[1] | inner[2]) >= 0);
     const int dxl = in_vector(dx0 + lx * 256), dyl = in_vector(dy0 + ly * 256);
     const int slot = ly * tile_pitch<TS>() + lx;
+    constexpr unsigned kRow = (1u << NB) - 1u;
     while (live) {
         const int row = (__ffsll((long long)live) - 1) / NB;
-        unsigned cols = (unsigned)(live >> (row * NB)) & ((1u << NB) - 1u);
-        const unsigned inside = (unsigned)(whole >> (row * NB));
-        live &= ~((unsigned long long)cols << (row * NB));
-        const int e0 = in_vector(off[0] + 8 * row * ex[0]), e1 = in_vector(off[1] + 8 * row * ex[1]),
-                  e2 = in_vector(off[2] + 8 * row * ex[2]);
+        unsigned cols = (unsigned)(live >> (row * NB)) & kRow;
+        live &= ~((unsigned long long)kRow << (row * NB));
         const float bdy = B * (float)(dyl + row * 2048);
         const int srow = in_vector(slot + row * 8 * tile_pitch<TS>());
+        if constexpr (kWhole) {
+            unsigned inside = cols & (unsigned)(whole >> (row * NB));
+            cols &= ~inside;
+            while (inside) {
+                const int bx = __ffs((int)inside) - 1;
+                inside &= inside - 1;
+                store_min<kVis>(id, window_bits(z0 + (A * (float)(dxl + (bx << 11)) + bdy), zoff), srow + 8 * bx, tile);
+            }
+            if (!cols) continue;
+        }
+        const int e0 = in_vector(off[0] + 8 * row * ex[0]), e1 = in_vector(off[1] + 8 * row * ex[1]),
+                  e2 = in_vector(off[2] + 8 * row * ex[2]);
         while (cols) {
             const int bx = __ffs((int)cols) - 1, i = 8 * bx;
             cols &= cols - 1;
-            if ((kWhole && (inside >> bx & 1u)) ||
-                ((e0 + __mul24(i, step[0])) | (e1 + __mul24(i, step[1])) | (e2 + __mul24(i, step[2]))) >= 0)
-                store_min<kVis>(id, window_bits(z0 + (A * (float)(dxl + (i << 8)) + bdy), zoff), srow + i, tile);
+            if ((mad24(step[0], i, e0) | mad24(step[1], i, e1) | mad24(step[2], i, e2)) >= 0)
+                store_min<kVis>(id, window_bits(z0 + (A * (float)(dxl + (bx << 11)) + bdy), zoff), srow + i, tile);
         }
     }
 }
@@ -1274,10 +1297,10 @@ __device__ __forceinline__ void raster_lanes(const Setup& s, const TileEdges& t,
 // with records over 256 pixels covered by the whole workgroup, one after
 // another between barriers (each wave repeating the record's setup for a
 // quarter of its pixels), and 130 us with a wave per record; a batch of twelve
-// frames (soups on 512^2-4096^2 maps) 4.82 and 2.94 ms.  Sending every record
-// over 256 pixels to the wave, whatever its neighbours' size, takes the batch
-// 3.26 ms.  Before the 32-bit edges and the vector-register steps a block
-// took 20 vector and 18 scalar instructions (batch 3.06 ms).
+// frames (soups on 512^2-4096^2 maps) 4.82 and 2.94 ms.  In that batch a
+// short list is one wave's, so its records of more than kShareBlocks blocks
+// are put aside for all four: 2.12 ms with a bound of 16, 2.01 of 8, 1.96 of
+// 4, 1.97 of 2 (a workgroup per tile; 2.74 ms with 8 from a queue of tiles).
 //
 // Records a lane rasterizes alone: those with at most self_bound() pixels of
 // bounding box in the tile.  The wave then runs as long as the largest such
@@ -1392,8 +1415,10 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
     if (self) raster_rect_self<RS, kVis>(s, t, g.x0, g.y0, rx0, rx1, ry0, ry1, tile);
 }
 
-// The records put aside, block rows by % 4 == wave per wave; then the region
-// is complete.  Depth maps go out with non-temporal stores: a frame writes far
+// The records put aside; then the region is complete.  A record goes to one
+// wave, which sets it up once (about 80 vector instructions, as many as six
+// blocks take), and only the remainder of four is shared by block rows; with
+// `by_rows`, for launches that leave the GPU room, all are, which ends sooner.  Depth maps go out with non-temporal stores: a frame writes far
 // more map bytes than the caches hold (64 x 16 MiB), and with ordinary stores
 // the last-written lines stay dirty in the MALL and are written back while
 // the screen pass reads the maps.  On the 64-sample 1080p frame this took the
@@ -1402,7 +1427,7 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
 template <int RS, bool kVis, bool kBig>
 __device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region& g, void* out, int map,
                                               typename KeyOf<kVis>::T* tile, const Setup* rec, const int& nrec,
-                                              ZBound& z) {
+                                              ZBound& z, bool by_rows) {
     constexpr int kWaves = kRasterThreads / 64;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __syncthreads();
@@ -1416,12 +1441,16 @@ __device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region
             s = rec[lane];
             t = tile_edges(s, g.x0, g.y0);
             unsigned long long rows = 0;
+            if (!by_rows && lane < (nq & ~(kWaves - 1))) {
+                if (lane % kWaves == wave) rows = ~0ull;
+            } else {
 #pragma unroll
-            for (int r = 0; r < RS / 8; r += kWaves) rows |= ((1ull << (RS / 8)) - 1ull) << ((RS / 8) * (r + wave));
+                for (int r = 0; r < RS / 8; r += kWaves) rows |= ((1ull << (RS / 8)) - 1ull) << ((RS / 8) * (r + wave));
+            }
             blocks = rows & block_mask<RS>(max(g.x0, s.px0) - g.x0, min(g.x1, s.px1) - g.x0,
                                            max(g.y0, s.py0) - g.y0, min(g.y1, s.py1) - g.y0);
         }
-        raster_lanes<RS, kVis, true>(s, t, blocks, has && (!kBig || t.ok), g.x0, g.y0, lane, z.zmax, z.age, tile);
+        raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks && (!kBig || t.ok), g.x0, g.y0, lane, z.zmax, z.age, tile);
         if constexpr (kBig) {
             unsigned long long slow = __ballot(has && !t.ok);
             while (slow) {
@@ -1526,7 +1555,7 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
         const uint32_t entry = kFallback ? k : (has ? b.entries[(size_t)map * b.cap + k] : 0u);
         raster_round<TS, TS, kVis, kFallback, kBig>(mesh, mvps, cfg, b, map, g, entry, has, aside, tile, rec, nrec, z);
     }
-    finish_region<TS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z);
+    finish_region<TS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z, spread);
 }
 
 // ---------------------------------------------------------------------------
@@ -1611,7 +1640,7 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
         }
         __syncthreads();  // nlist and the list are rewritten by the next pass
     }
-    finish_region<RS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z);
+    finish_region<RS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z, true);
 }
 
 // Binned raster: one workgroup per (tile, map); overflowed maps are left to

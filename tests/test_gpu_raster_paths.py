@@ -75,3 +75,25 @@ def test_depth_and_visibility_by_triangle_size(gi, oracle_lib, cuda, n, edge, w,
     pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
     assert bits_equal(g.position.cpu().numpy(), pos_o)
     assert bits_equal(g.normal.cpu().numpy(), nrm_o), mismatch_report(g.normal.cpu().numpy(), nrm_o, "normal")
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 8, 27, 28, 29, 31, 33, 60, 200])
+def test_records_put_aside_by_count(gi, oracle_lib, cuda, n):
+    """n triangles that cover most of 32 tiles, in 65 maps (a launch of more
+    than 2,048 tiles, whose lists are not split): a tile's larger records go
+    one to a wave, the remainder of four by block rows, those over the queue's
+    28 to the wave that read them."""
+    rng = np.random.default_rng(100 + n)
+    w, h, maps = 512, 256, 65
+    pos = np.array([[-1.5, -1.5, 0.0], [2.5, -1.5, 0.0], [-1.5, 2.5, 0.0]]) + rng.uniform(-0.5, 0.5, size=(n, 3, 3))
+    pos[1::2, :, :2] *= -1.0
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3).astype(np.float32), np.zeros((3 * n, 3), np.float32),
+                          np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvps = np.tile(np.eye(4, dtype=np.float32).reshape(1, 16), (maps, 1))
+    mvps[1::2, 10] = 0.5  # every other map half as deep
+    got = gi.render_shadow_map(gi.DeviceMesh.from_mesh(mesh), mvps, w, h).cpu().numpy()
+    for first in (0, 1):
+        want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvps[first], w, h)
+        for k in range(first, maps, 2):
+            assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k}")
+        assert (want < 1.0).mean() > 0.3
