@@ -250,7 +250,7 @@ __global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_r
 
 template <int TS>
 __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable t) {
-    __shared__ uint32_t tile[TS * tile_pitch<TS>()];
+    __shared__ __align__(16) uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     if (t.counter[0] == 0u) return;  // no map overflowed (kb_scan)

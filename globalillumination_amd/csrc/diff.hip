@@ -13,13 +13,15 @@
 //
 // A texel's depth and barycentrics are affine in the texel centre, so the
 // per-triangle part is set up once per (map, triangle) (k_diff_setup) and a
-// texel evaluates two affine forms.  The adjoint of the texel depths with
+// texel evaluates affine forms.  The adjoint of the texel depths with
 // respect to the triangle's clip-space vertices is linear in G * lambda_j
 // (G = dL/dd, lambda_j the texel's barycentrics), so the texel adjoint only
 // sums w_j = sum G * lambda_j per (map, triangle) and k_diff_tri_bwd turns the
 // three sums into vertex and matrix gradients.
 //
-// Forward:  visibility raster, k_diff_setup, k_diff_depth, k_diff_shade.
+// Forward:  visibility raster, k_diff_setup, k_diff_shade (tap depths from keys
+//           and planes: a frame's taps read a small part of the texels, so the
+//           depth maps are never stored).
 // Backward: the visibility raster and k_diff_setup again (recomputed, nothing
 //           is kept from the forward pass), then k_diff_shade_bwd (pixel
 //           adjoint, tap depths from keys and planes: dL/d(B*M'_i) per block,
@@ -39,7 +41,7 @@ namespace gi {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTexPerThread = 4;   // texels per thread in the texel adjoint
+constexpr int kTexPerThread = 8;   // texels per thread in the texel adjoint
 constexpr int kGatherMax = 256;    // bbox texels up to which a triangle gathers its own adjoint
 constexpr int kLargeSlots = 4;     // large triangles a texel block sums in LDS
 constexpr int kMapsPerThread = 1;  // maps a triangle-adjoint thread walks (vertex gradients summed over them)
@@ -77,6 +79,17 @@ struct TriPlane {
     double a1, b1, a2, b2;
     double Z0, dZ1, dZ2;
     short bx0, bx1, by0, by1;
+};
+
+// The depth of a triangle's texels alone, about the texel (x0, y0) that holds
+// vertex 0: d = d0 + A (a - x0) + B (b - y0) (1 without a plane).  The taps of
+// the shading kernels are bound by the lines their gathers touch: 32 bytes a
+// texel here, 72 from TriPlane.  Against 80-bit arithmetic the two forms err
+// alike over triangles of 2 to 1000 texels, slivers included (both carry the
+// rounding of the projected area D).
+struct alignas(16) TexelPlane {
+    double d0, A, B;
+    int x0, y0;
 };
 
 __device__ __forceinline__ bool plane_ok(const TriPlane& p) { return p.X0 == p.X0; }
@@ -127,9 +140,25 @@ __device__ __forceinline__ bool tri_screen(const float* __restrict__ pos, const 
     return ok;
 }
 
-// One thread per (triangle, map).  grid (triangle blocks, S).
+__device__ __forceinline__ TexelPlane texel_plane(const TriPlane& p) {
+    TexelPlane q{1.0, 0.0, 0.0, 0, 0};
+    if (plane_ok(p)) {
+        const double cx = floor(fmax(-1e9, fmin(p.X0, 1e9))), cy = floor(fmax(-1e9, fmin(p.Y0, 1e9)));
+        q.A = p.a1 * p.dZ1 + p.a2 * p.dZ2;
+        q.B = p.b1 * p.dZ1 + p.b2 * p.dZ2;
+        q.d0 = p.Z0 + (q.A * ((cx + 0.5) - p.X0) + q.B * ((cy + 0.5) - p.Y0));
+        q.x0 = (int)cx;
+        q.y0 = (int)cy;
+    }
+    return q;
+}
+
+// One thread per (triangle, map).  grid (triangle blocks, S).  kAdjoint: also
+// what the adjoint needs (TriPlane, the large flags).
+template <bool kAdjoint>
 __global__ __launch_bounds__(kThreads) void k_diff_setup(const float* __restrict__ pos, const int* __restrict__ idx,
                                                          int ntris, const double* __restrict__ mvps, DiffCfg c,
+                                                         TexelPlane* __restrict__ texels,
                                                          TriPlane* __restrict__ planes,
                                                          unsigned char* __restrict__ large) {
     const int t = blockIdx.x * kThreads + threadIdx.x;
@@ -164,45 +193,17 @@ __global__ __launch_bounds__(kThreads) void k_diff_setup(const float* __restrict
         p.X0 = __builtin_nan("");
         p.Y0 = p.a1 = p.b1 = p.a2 = p.b2 = p.Z0 = p.dZ1 = p.dZ2 = 0.0;
     }
+    texels[(size_t)i * ntris + t] = texel_plane(p);
+    if (!kAdjoint) return;
     planes[(size_t)i * ntris + t] = p;
     large[(size_t)i * ntris + t] = (plane_ok(p) && plane_large(p)) ? 1 : 0;
 }
 
-// Triangle of a visibility key (a piece id is tri * 8 + piece), or -1.
-__device__ __forceinline__ int key_tri(unsigned long long key, int ntris) {
-    if (key == ~0ull) return -1;
-    const int t = (int)((key & 0xffffffffull) >> 3);
+// Triangle of texel k, or -1: a visibility key's low word is the piece id,
+// tri * 8 + piece, and all ones where no triangle is.
+__device__ __forceinline__ int vis_tri(const unsigned long long* __restrict__ vis, size_t k, int ntris) {
+    const int t = (int)(reinterpret_cast<const uint32_t*>(vis)[2 * k] >> 3);
     return t < ntris ? t : -1;
-}
-
-// Depth of texel (kx, ky) of one map from its visibility key and the plane
-// record of the triangle the key names; 1 for background.
-__device__ __forceinline__ double texel_depth(const unsigned long long* __restrict__ vk,
-                                              const TriPlane* __restrict__ pl, int ntris, uint32_t smw, uint32_t kx,
-                                              uint32_t ky) {
-    const int t = key_tri(vk[(size_t)ky * smw + kx], ntris);
-    double d = 1.0;
-    if (t >= 0) {
-        const TriPlane& p = pl[t];
-        if (p.X0 == p.X0) {
-            const double dx = ((double)kx + 0.5) - p.X0, dy = ((double)ky + 0.5) - p.Y0;
-            const double l1 = p.a1 * dx + p.b1 * dy, l2 = p.a2 * dx + p.b2 * dy;
-            d = p.Z0 + l1 * p.dZ1 + l2 * p.dZ2;
-        }
-    }
-    return d;
-}
-
-__global__ __launch_bounds__(kThreads) void k_diff_depth(const unsigned long long* __restrict__ vis,
-                                                         const TriPlane* __restrict__ planes, int ntris, DiffCfg c,
-                                                         double* __restrict__ depth) {
-    const uint32_t plane = (uint32_t)c.smw * (uint32_t)c.smh;  // < 2^31 (edges <= 16384)
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int map = blockIdx.y;
-    if (k >= plane) return;
-    const uint32_t ky = k / (uint32_t)c.smw, kx = k - ky * (uint32_t)c.smw;
-    depth[(size_t)map * plane + k] =
-        texel_depth(vis + (size_t)map * plane, planes + (size_t)map * ntris, ntris, (uint32_t)c.smw, kx, ky);
 }
 
 struct Tap {
@@ -228,13 +229,49 @@ __device__ __forceinline__ Tap project(const double m[16], double x, double y, d
     return t;
 }
 
-__device__ __forceinline__ double texel(const double* __restrict__ d, int a, int b, const DiffCfg& c) {
-    return (a >= 0 && a < c.smw && b >= 0 && b < c.smh) ? d[(size_t)b * c.smw + a] : 0.0;
+// The triangles of a pixel's four texels, row by row: -1 background, -2 outside
+// the map.  A row's two keys are one 16-byte load (of 8-byte alignment).
+__device__ __forceinline__ void tap_tris(const unsigned long long* __restrict__ vk, int ntris, const DiffCfg& c,
+                                         const Tap& t, int tri[4]) {
+    typedef unsigned pair __attribute__((ext_vector_type(4), aligned(8)));
+    const int ca = max(0, min(t.a0, c.smw - 2));
+#pragma unroll
+    for (int db = 0; db < 2; ++db) {
+        const int b = t.b0 + db, cb = max(0, min(b, c.smh - 1));
+        const unsigned long long* row = vk + (size_t)cb * c.smw + ca;
+        unsigned id[2];
+        if (c.smw >= 2) {  // uniform
+            const pair k = *reinterpret_cast<const pair*>(row);
+            id[0] = k.x;
+            id[1] = k.z;
+        } else {
+            id[0] = id[1] = reinterpret_cast<const unsigned*>(row)[0];
+        }
+#pragma unroll
+        for (int da = 0; da < 2; ++da) {
+            const int a = t.a0 + da;
+            const bool in = a >= 0 && a < c.smw && b >= 0 && b < c.smh;
+            const int tr = (int)(id[a == ca ? 0 : 1] >> 3);
+            tri[2 * db + da] = !in ? -2 : tr < ntris ? tr : -1;
+        }
+    }
 }
 
+// Depth of texel (a, b) from its triangle's record; 1 for background, 0
+// outside the map.
+__device__ __forceinline__ double texel_depth(const TexelPlane* __restrict__ pl, int tri, int a, int b) {
+    if (tri < 0) return tri == -1 ? 1.0 : 0.0;
+    const TexelPlane p = pl[tri];
+    return p.d0 + (p.A * (double)(a - p.x0) + p.B * (double)(b - p.y0));
+}
+
+// A pixel's mean over the maps.  Bound by the gathers of keys and records: 16
+// maps of 1024^2 under a 512^2 view 60 us (132 us with a pass that stored every
+// texel's depth before it; fetching the next map's keys ahead changes nothing).
 __global__ __launch_bounds__(kThreads) void k_diff_shade(const float* __restrict__ gpos,
                                                          const double* __restrict__ biased,
-                                                         const double* __restrict__ depth, DiffCfg c,
+                                                         const unsigned long long* __restrict__ vis,
+                                                         const TexelPlane* __restrict__ planes, int ntris, DiffCfg c,
                                                          float* __restrict__ out) {
     const size_t plane = (size_t)c.gw * c.gh;
     const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -251,7 +288,9 @@ __global__ __launch_bounds__(kThreads) void k_diff_shade(const float* __restrict
         double m[16];
         load_m(biased + 16 * i, m);
         const Tap t = project(m, x, y, z, c);
-        const double* d = depth + (size_t)i * msz;
+        int tri[4];
+        tap_tris(vis + (size_t)i * msz, ntris, c, t, tri);
+        const TexelPlane* pl = planes + (size_t)i * ntris;
         const double wu[2] = {1.0 - smoothw(t.fu), smoothw(t.fu)};
         const double wv[2] = {1.0 - smoothw(t.fv), smoothw(t.fv)};
         double q = 0.0;
@@ -259,23 +298,45 @@ __global__ __launch_bounds__(kThreads) void k_diff_shade(const float* __restrict
         for (int db = 0; db < 2; ++db)
 #pragma unroll
             for (int da = 0; da < 2; ++da)
-                q += wu[da] * wv[db] * sigmoid_d((texel(d, t.a0 + da, t.b0 + db, c) - t.z + c.bias) / c.tau);
+                q += wu[da] * wv[db] *
+                     sigmoid_d((texel_depth(pl, tri[2 * db + da], t.a0 + da, t.b0 + db) - t.z + c.bias) / c.tau);
         acc += c.si + (1.0 - c.si) * q;
     }
     out[k] = (float)(acc / (double)c.S);
 }
 
-// Block sum of 16 per-thread values into partial[16] (fixed order).
+// x + y with the halves of the wave transposed: lanes 0-31 get x's sum over
+// both halves, lanes 32-63 y's; swap_add16 the same by rows of 16 lanes.
+__device__ __forceinline__ double swap_add32(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double swap_add16(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Block sum of 16 per-thread values into partial[16] (fixed order).  Each step
+// halves the values a lane holds along with the lanes that share one, so a
+// wave exchanges 17 doubles (12 by lane swaps in registers) where 16 separate
+// sums exchange 96 through LDS.
 __device__ __forceinline__ void block_sum16(const double v[16], double* __restrict__ partial) {
     __shared__ double red[kThreads / 64][16];
     const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+    double a[8], b[4], c[2];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        double x = v[e];
+    for (int e = 0; e < 8; ++e) a[e] = swap_add32(v[e], v[e + 8]);
 #pragma unroll
-        for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-        if (lane == 0) red[wave][e] = x;
-    }
+    for (int e = 0; e < 4; ++e) b[e] = swap_add16(a[e], a[e + 4]);
+    const bool h8 = (lane & 8) != 0, h4 = (lane & 4) != 0;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) c[e] = (h8 ? b[e + 2] : b[e]) + __shfl_xor(h8 ? b[e] : b[e + 2], 8, 64);
+    double x = (h4 ? c[1] : c[0]) + __shfl_xor(h4 ? c[0] : c[1], 4, 64);
+    x += __shfl_xor(x, 2, 64);
+    x += __shfl_xor(x, 1, 64);
+    if ((lane & 3) == 0) red[wave][lane >> 2] = x;  // bits 5, 4, 3, 2 of the lane: 8, 4, 2, 1 of the element
     __syncthreads();
     if (threadIdx.x < 16) {
         double s = 0.0;
@@ -289,13 +350,14 @@ __device__ __forceinline__ void block_sum16(const double v[16], double* __restri
 // Pixel adjoint.  grid (pixel blocks of kBwdPixPerThread * kThreads pixels, S):
 // each thread adds the matrix terms of kBwdPixPerThread pixels (strided by
 // the block size, so every step reads coalesced) before the one block
-// reduction.  The tap depths are evaluated from the recomputed visibility
-// keys and plane records (texel_depth, the arithmetic k_diff_depth stores in
-// the forward pass), so backward never materialises the depth maps.
+// reduction.  Its float atomics take half the time: 16 maps of 1024^2 under a
+// 512^2 view 158 us, 88 us without them; without the zero ones left out and
+// with 72-byte plane records 178 us.  Handing taps to the neighbouring lane
+// first changes nothing (the view's pixels are several texels apart).
 __global__ __launch_bounds__(kThreads) void k_diff_shade_bwd(const float* __restrict__ gpos,
                                                              const double* __restrict__ biased,
                                                              const unsigned long long* __restrict__ vis,
-                                                             const TriPlane* __restrict__ planes, int ntris,
+                                                             const TexelPlane* __restrict__ planes, int ntris,
                                                              const float* __restrict__ grad_out, DiffCfg c,
                                                              float* __restrict__ grad_depth,
                                                              double* __restrict__ partial) {
@@ -314,23 +376,25 @@ __global__ __launch_bounds__(kThreads) void k_diff_shade_bwd(const float* __rest
             const Tap t = project(m, x, y, z, c);
             const size_t msz = (size_t)c.smw * c.smh;
             const unsigned long long* vk = vis + (size_t)i * msz;
-            const TriPlane* pl = planes + (size_t)i * ntris;
+            const TexelPlane* pl = planes + (size_t)i * ntris;
             const double su = smoothw(t.fu), sv = smoothw(t.fv);
             const double wu[2] = {1.0 - su, su}, wv[2] = {1.0 - sv, sv};
             const double dwu[2] = {-dsmoothw(t.fu), dsmoothw(t.fu)}, dwv[2] = {-dsmoothw(t.fv), dsmoothw(t.fv)};
+            int tri[4];
+            tap_tris(vk, ntris, c, t, tri);
             double gz = 0.0, gfu = 0.0, gfv = 0.0;
 #pragma unroll
             for (int db = 0; db < 2; ++db)
 #pragma unroll
                 for (int da = 0; da < 2; ++da) {
                     const int a = t.a0 + da, b = t.b0 + db;
-                    const bool in = a >= 0 && a < c.smw && b >= 0 && b < c.smh;
-                    const double dd = in ? texel_depth(vk, pl, ntris, (uint32_t)c.smw, (uint32_t)a, (uint32_t)b) : 0.0;
+                    const double dd = texel_depth(pl, tri[2 * db + da], a, b);
                     const double sg = sigmoid_d((dd - t.z + c.bias) / c.tau);
                     const double ds = sg * (1.0 - sg) / c.tau;
                     const double w = wu[da] * wv[db];
-                    if (in && gq != 0.0)
-                        unsafeAtomicAdd(&grad_depth[(size_t)i * msz + (size_t)b * c.smw + a], (float)(gq * w * ds));
+                    // most taps of a lit or shadowed pixel add nothing: their sigmoid is flat
+                    const float g = (float)(gq * w * ds);
+                    if (tri[2 * db + da] != -2 && g != 0.0f) unsafeAtomicAdd(&grad_depth[(size_t)i * msz + (size_t)b * c.smw + a], g);
                     gz -= w * ds;
                     gfu += dwu[da] * wv[db] * sg;
                     gfv += wu[da] * dwv[db] * sg;
@@ -353,15 +417,14 @@ __global__ __launch_bounds__(kThreads) void k_diff_shade_bwd(const float* __rest
 // texels; a ground plane covers most texels of every map): the sums of
 // G * lambda_j over each large triangle's texels.  grid (texel blocks, S);
 // each thread takes kTexPerThread texels strided by the block size
-// (coalesced).  Device-scope atomics on one triangle's cache line from every
-// wave would serialize, so a wave first reduces: its texels are 64
-// consecutive texels of a row, in which each triangle covers a contiguous
-// run, and a segmented scan leaves every run's sum in the run's last lane;
-// a wave that is one run keeps a running sum in lane 0 while consecutive rows
-// stay on that triangle.  Runs are added into kLargeSlots LDS slots per
-// block, written out as the block's LargePart entries that
-// k_diff_large_reduce adds into wsum; a block meeting more large triangles
-// than slots adds the rest to wsum with device atomics.
+// (coalesced), all their loads in flight together.  Device-scope atomics on one
+// triangle's cache line from every wave would serialize, so a lane sums its own
+// texels while they stay on one large triangle, the wave then adds up its lanes
+// a triangle at a time, and the sums go into kLargeSlots LDS slots per block,
+// written out as the block's LargePart entries that k_diff_large_reduce adds
+// into wsum; a block meeting more large triangles than slots adds the rest to
+// wsum with device atomics.  16 maps of 1024^2: 64 us, 94 us when every row of
+// 64 texels was reduced across the wave by itself.
 template <int kSlots>
 __device__ __forceinline__ void add_slots(int* slot_tri, double (*slot_w)[3], double* __restrict__ wsum, int tri,
                                           const double w[3]) {
@@ -402,75 +465,61 @@ __global__ __launch_bounds__(kThreads) void k_diff_texel_bwd(const unsigned long
     const unsigned char* __restrict__ lg = large + (size_t)i * ntris;
     unsigned char* __restrict__ tch = touched + (size_t)i * ntris;
     const int lane = threadIdx.x % 64;
-    const unsigned long long upto = (lane == 63) ? ~0ull : ((2ull << lane) - 1ull);  // lanes 0..lane
     const uint32_t base = (uint32_t)blockIdx.x * (kTexPerThread * kThreads) + threadIdx.x;
-    int cur = -1;  // lane 0: triangle of the running sum
+    // this lane's triangle and its sums; a lane meets few large triangles
+    int cur = -1;
     double run[3] = {0.0, 0.0, 0.0};
+    float G[kTexPerThread];
+    int tri[kTexPerThread];
+#pragma unroll
     for (int r = 0; r < kTexPerThread; ++r) {
         const uint32_t k = base + (uint32_t)r * kThreads;
-        double w[3] = {0.0, 0.0, 0.0};
-        int tri = -1;
-        const float G = (k < msz) ? gd[k] : 0.0f;
-        if (G != 0.0f) {
-            const int t = key_tri(vk[k], ntris);
-            if (t >= 0 && !lg[t]) tch[t] = 1;  // a small triangle with gradient: k_diff_tri_bwd gathers it
-            if (t >= 0 && lg[t]) {
-                const TriPlane& p = pl[t];
-                {
-                    tri = t;
-                    const uint32_t ky = k / (uint32_t)c.smw, kx = k - ky * (uint32_t)c.smw;
-                    const double dx = ((double)kx + 0.5) - p.X0, dy = ((double)ky + 0.5) - p.Y0;
-                    const double l1 = p.a1 * dx + p.b1 * dy, l2 = p.a2 * dx + p.b2 * dy;
-                    w[0] = (double)G * (1.0 - l1 - l2);
-                    w[1] = (double)G * l1;
-                    w[2] = (double)G * l2;
-                }
-            }
-        }
-        // every lane of the wave reaches this point
-        const unsigned long long valid = __ballot(tri >= 0);
-        if (valid == 0ull) continue;
-        // lanes without a contribution (w = 0) join the run of the nearest
-        // contributing lane at or below them
-        const unsigned long long below = valid & upto;
-        const int src = below ? 63 - __clzll((long long)below) : __ffsll((long long)valid) - 1;
-        tri = __shfl(tri, src, 64);
-        const int prev = __shfl_up(tri, 1, 64);
-        const unsigned long long heads = __ballot(lane == 0 || tri != prev);
-        if (heads == 1ull) {  // one run: the whole wave is one triangle
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                double x = w[j];
-#pragma unroll
-                for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
-                w[j] = x;
-            }
-            if (lane == 0) {
-                if (cur != tri) {
-                    add_slots<kLargeSlots>(slot_tri, slot_w, wsum, cur, run);
-                    cur = tri;
-                    run[0] = run[1] = run[2] = 0.0;
-                }
-                run[0] += w[0];
-                run[1] += w[1];
-                run[2] += w[2];
-            }
-            continue;
-        }
-        // segmented inclusive scan: lane sums its run from the run's head
-        const int head = 63 - __clzll((long long)(heads & upto));
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                const double y = __shfl_up(w[j], off, 64);
-                if (lane - off >= head) w[j] += y;
-            }
-        }
-        const bool tail = (lane == 63) || ((heads >> (lane + 1)) & 1ull);
-        if (tail) add_slots<kLargeSlots>(slot_tri, slot_w, wsum, tri, w);
+        G[r] = (k < msz) ? gd[k] : 0.0f;
     }
-    if (lane == 0) add_slots<kLargeSlots>(slot_tri, slot_w, wsum, cur, run);
+#pragma unroll
+    for (int r = 0; r < kTexPerThread; ++r) tri[r] = G[r] != 0.0f ? vis_tri(vk, base + (uint32_t)r * kThreads, ntris) : -1;
+#pragma unroll
+    for (int r = 0; r < kTexPerThread; ++r) {
+        if (tri[r] >= 0 && !lg[tri[r]]) {  // a small triangle with gradient: k_diff_tri_bwd gathers it
+            tch[tri[r]] = 1;
+            tri[r] = -1;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kTexPerThread; ++r) {
+        const int t = tri[r];
+        if (t < 0) continue;
+        if (t != cur) {
+            add_slots<kLargeSlots>(slot_tri, slot_w, wsum, cur, run);
+            cur = t;
+            run[0] = run[1] = run[2] = 0.0;
+        }
+        const TriPlane& p = pl[t];
+        const uint32_t k = base + (uint32_t)r * kThreads;
+        const uint32_t ky = k / (uint32_t)c.smw, kx = k - ky * (uint32_t)c.smw;
+        const double dx = ((double)kx + 0.5) - p.X0, dy = ((double)ky + 0.5) - p.Y0;
+        const double l1 = p.a1 * dx + p.b1 * dy, l2 = p.a2 * dx + p.b2 * dy;
+        run[0] += (double)G[r] * (1.0 - l1 - l2);
+        run[1] += (double)G[r] * l1;
+        run[2] += (double)G[r] * l2;
+    }
+    // the wave's sums, a triangle at a time; the lanes of a fifth one add their own
+    unsigned long long left = __ballot(cur >= 0);
+    for (int n = 0; n < 4 && left; ++n) {
+        const int t = __shfl(cur, __ffsll((long long)left) - 1, 64);
+        const bool mine = cur == t;
+        left &= ~__ballot(mine);
+        double w[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            double x = mine ? run[j] : 0.0;
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) x += __shfl_down(x, off, 64);
+            w[j] = x;
+        }
+        if (lane == 0) add_slots<kLargeSlots>(slot_tri, slot_w, wsum, t, w);
+    }
+    if (left >> lane & 1ull) add_slots<kLargeSlots>(slot_tri, slot_w, wsum, cur, run);
     __syncthreads();
     if (threadIdx.x < kLargeSlots) {
         LargePart lp;
@@ -555,27 +604,36 @@ __global__ __launch_bounds__(kThreads) void k_diff_tri_bwd(const float* __restri
                 } else if (touched[(size_t)i * ntris + t]) {
                     // bounding-box texels in batches whose loads are issued together
                     const size_t moff = (size_t)i * c.smw * c.smh;
-                    const int bw = p.bx1 - p.bx0 + 1, area = bbox_area(p);
+                    const int area = bbox_area(p);
+                    int x = p.bx0, y = p.by0;
                     for (int q0 = 0; q0 < area; q0 += kGatherBatch) {
-                        unsigned long long key[kGatherBatch];
+                        int tri[kGatherBatch];
                         float G[kGatherBatch];
+                        int xs = x, ys = y;
 #pragma unroll
                         for (int u = 0; u < kGatherBatch; ++u) {
-                            const int q = q0 + u;
-                            const size_t k = moff + (size_t)(p.by0 + q / bw) * c.smw + (p.bx0 + q % bw);
-                            key[u] = q < area ? vis[k] : ~0ull;
-                            G[u] = q < area ? grad_depth[k] : 0.0f;
+                            const bool in = q0 + u < area;
+                            const size_t k = moff + (size_t)ys * c.smw + xs;
+                            tri[u] = in ? vis_tri(vis, k, ntris) : -1;
+                            G[u] = in ? grad_depth[k] : 0.0f;
+                            if (++xs > p.bx1) {
+                                xs = p.bx0;
+                                ++ys;
+                            }
                         }
 #pragma unroll
                         for (int u = 0; u < kGatherBatch; ++u) {
-                            if (G[u] == 0.0f || key_tri(key[u], ntris) != t) continue;
-                            const int q = q0 + u;
-                            const double dx = ((double)(p.bx0 + q % bw) + 0.5) - p.X0;
-                            const double dy = ((double)(p.by0 + q / bw) + 0.5) - p.Y0;
-                            const double l1 = p.a1 * dx + p.b1 * dy, l2 = p.a2 * dx + p.b2 * dy;
-                            w[0] += (double)G[u] * (1.0 - l1 - l2);
-                            w[1] += (double)G[u] * l1;
-                            w[2] += (double)G[u] * l2;
+                            if (G[u] != 0.0f && tri[u] == t) {
+                                const double dx = ((double)x + 0.5) - p.X0, dy = ((double)y + 0.5) - p.Y0;
+                                const double l1 = p.a1 * dx + p.b1 * dy, l2 = p.a2 * dx + p.b2 * dy;
+                                w[0] += (double)G[u] * (1.0 - l1 - l2);
+                                w[1] += (double)G[u] * l1;
+                                w[2] += (double)G[u] * l2;
+                            }
+                            if (++x > p.bx1) {
+                                x = p.bx0;
+                                ++y;
+                            }
                         }
                     }
                 }
@@ -666,8 +724,8 @@ inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 struct DiffWs {
     float* mvps32;
     unsigned long long* vis;
-    double* depth;
     float* grad_depth;
+    TexelPlane* texels;
     TriPlane* planes;
     double* wsum;
     double* part_px;
@@ -690,8 +748,8 @@ size_t diff_layout(int ntris, int S, int smw, int smh, int gw, int gh, DiffWs* w
     size_t off = 0;
     size_t o_m32 = off; off = align256(off + sizeof(float) * 16 * (size_t)S);
     size_t o_vis = off; off = align256(off + sizeof(unsigned long long) * msz * S);
-    size_t o_depth = off; off = align256(off + sizeof(double) * msz * S);
     size_t o_gd = off; off = align256(off + sizeof(float) * msz * S);
+    size_t o_tx = off; off = align256(off + sizeof(TexelPlane) * (size_t)ntris * S);
     size_t o_pl = off; off = align256(off + sizeof(TriPlane) * (size_t)ntris * S);
     size_t o_ws = off; off = align256(off + sizeof(double) * 3 * (size_t)ntris * S);
     size_t o_ppx = off; off = align256(off + sizeof(double) * 16 * (size_t)px_blocks * S);
@@ -704,8 +762,8 @@ size_t diff_layout(int ntris, int S, int smw, int smh, int gw, int gh, DiffWs* w
     if (ws) {
         ws->mvps32 = reinterpret_cast<float*>(base + o_m32);
         ws->vis = reinterpret_cast<unsigned long long*>(base + o_vis);
-        ws->depth = reinterpret_cast<double*>(base + o_depth);
         ws->grad_depth = reinterpret_cast<float*>(base + o_gd);
+        ws->texels = reinterpret_cast<TexelPlane*>(base + o_tx);
         ws->planes = reinterpret_cast<TriPlane*>(base + o_pl);
         ws->wsum = reinterpret_cast<double*>(base + o_ws);
         ws->part_px = reinterpret_cast<double*>(base + o_ppx);
@@ -748,18 +806,14 @@ int check_common(const float* positions_dev, int nverts, const int32_t* indices_
 
 // Visibility raster, per-triangle planes and (forward) texel depths.
 int recompute(const float* pos, int nverts, const int32_t* idx, int ntris, const double* mvps, const DiffCfg& c,
-              const DiffWs& w, hipStream_t s, bool with_depth) {
+              const DiffWs& w, hipStream_t s, bool adjoint) {
     hipLaunchKernelGGL(k_to_f32, dim3((unsigned)((16 * c.S + 255) / 256)), dim3(256), 0, s, mvps, w.mvps32, 16 * c.S);
     int rc = internal::vis_raster(pos, nverts, idx, ntris, w.mvps32, c.S, c.smw, c.smh, w.vis, w.raster,
                                   w.raster_bytes, s);
     if (rc != GI_OK) return rc;
     if (ntris > 0)
-        hipLaunchKernelGGL(k_diff_setup, dim3((unsigned)w.tri_blocks, c.S), dim3(kThreads), 0, s, pos, idx, ntris,
-                           mvps, c, w.planes, w.large);
-    const size_t msz = (size_t)c.smw * c.smh;
-    if (with_depth)
-        hipLaunchKernelGGL(k_diff_depth, dim3((unsigned)((msz + kThreads - 1) / kThreads), c.S), dim3(kThreads), 0, s,
-                           w.vis, w.planes, ntris, c, w.depth);
+        hipLaunchKernelGGL(adjoint ? k_diff_setup<true> : k_diff_setup<false>, dim3((unsigned)w.tri_blocks, c.S),
+                           dim3(kThreads), 0, s, pos, idx, ntris, mvps, c, w.texels, w.planes, w.large);
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
 
@@ -791,10 +845,10 @@ int gi_diff_soft_forward(const float* positions_dev, int nverts, const int32_t* 
     if (need == 0) return GI_ENOTSUP;
     if (workspace_bytes < need) return GI_ENOSPACE;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, true);
+    rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, false);
     if (rc != GI_OK) return rc;
     hipLaunchKernelGGL(k_diff_shade, dim3(w.px_blocks), dim3(kThreads), 0, s, gbuffer->position_dev, biased_mvps_dev,
-                       w.depth, c, out_dev);
+                       w.vis, w.texels, ntris, c, out_dev);
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
 
@@ -815,12 +869,12 @@ int gi_diff_soft_backward(const float* positions_dev, int nverts, const int32_t*
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     // the forward intermediates are recomputed, not stored; the pixel adjoint
     // evaluates the texel depths it reads from the keys and planes
-    rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, false);
+    rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, true);
     if (rc != GI_OK) return rc;
     const size_t msz = (size_t)smw * smh * nsamples;
     hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(kThreads), 0, s, w.grad_depth, msz, 0.0f);
     hipLaunchKernelGGL(k_diff_shade_bwd, dim3(w.pxb_blocks, nsamples), dim3(kThreads), 0, s, gbuffer->position_dev,
-                       biased_mvps_dev, w.vis, w.planes, ntris, grad_out_dev, c, w.grad_depth, w.part_px);
+                       biased_mvps_dev, w.vis, w.texels, ntris, grad_out_dev, c, w.grad_depth, w.part_px);
     hipLaunchKernelGGL(k_diff_reduce, dim3(nsamples), dim3(kThreads), 0, s, w.part_px, w.pxb_blocks,
                        grad_biased_mvps_dev);
     if (ntris > 0) {

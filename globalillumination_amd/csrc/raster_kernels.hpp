@@ -1486,6 +1486,16 @@ __device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region
         }
     } else {
         unsigned long long* dst = reinterpret_cast<unsigned long long*>(out) + (size_t)map * plane;
+        if (g.x1 - g.x0 + 1 == RS && (cfg.w & 1) == 0) {  // 16-byte stores
+            for (int q = tid; q < kPx / 2; q += kRasterThreads) {
+                const int r = q / (RS / 2), cidx = (q % (RS / 2)) * 2;
+                const int j = g.y0 + r;
+                if (j > g.y1) continue;
+                const ulonglong2 v = *reinterpret_cast<const ulonglong2*>(&tile[r * tile_pitch<RS>() + cidx]);
+                *reinterpret_cast<ulonglong2*>(dst + (size_t)j * cfg.w + g.x0 + cidx) = v;
+            }
+            return;
+        }
         for (int p = tid; p < kPx; p += kRasterThreads) {
             const int i = g.x0 + p % RS, j = g.y0 + p / RS;
             if (i > g.x1 || j > g.y1) continue;

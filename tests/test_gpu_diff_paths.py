@@ -1,0 +1,50 @@
+"""The differentiable pass at the sizes where its kernels' indexing can go
+wrong: maps of one and two columns (a tap row's keys are read in pairs), odd
+maps and views, pixels whose taps leave the map, a coarse mesh (every triangle
+goes through the texel pass's sums) and a fine one (every triangle gathers).
+
+Tolerances as in test_gpu_diff.py: 1e-6 for the forward pass (FP64 throughout,
+FP32 output), 1e-3 |oracle| + 2e-5 max|oracle| per vertex coordinate (FP32 sums
+of float atomics); the light's gradient sums the same texel adjoints, so
+2e-5 of the sum of its four magnitudes."""
+import numpy as np
+import pytest
+
+from test_gpu_diff import Setup, _adjoint
+
+pytestmark = pytest.mark.gpu
+
+
+class _Sized(Setup):
+    def __init__(self, gi, oracle_lib, map_size, view, freq):
+        from globalillumination_amd import passes, scenes
+        from globalillumination_amd.diff import AreaLight, DiffParams, DiffScene, colmajor
+
+        self.mesh = scenes.Mesh.concat(scenes.displaced_icosphere(freq, seed=5), scenes.ground_quad(20.0, 20.0, 0.0))
+        self.light = AreaLight((0.0, 0.0, 0.0), 2.0 * scenes.stratified_jitter(4, seed=5), map_size)
+        self.L, self.r = np.array([3.0, 7.0, 2.0]), 0.25
+        cam = scenes.View((0.0, 6.0, 14.0), (0.0, 1.0, 0.0), *view, fov=75.0)
+        self.dm = passes.DeviceMesh.from_mesh(self.mesh)
+        self.gbuf = passes.render_gbuffer(self.dm, passes.view_matrices(cam)[2], *view)
+        self.params = DiffParams()
+        self.scene = DiffScene(self.dm.indices, self.gbuf, self.light, self.params)
+        self.gpos = self.gbuf.position.cpu().numpy()
+        self.pos64 = self.mesh.positions.astype(np.float64)
+        self.idx = self.mesh.indices.astype(np.int32)
+        self.oracle = oracle_lib
+        M = self.light.matrices(self.L, self.r)
+        self.vis = [oracle_lib.visibility_raster(self.mesh.positions, self.idx, colmajor(m).astype(np.float32), map_size,
+                                                 map_size) for m in M]
+
+
+@pytest.mark.parametrize("map_size,view,freq", [(1, (33, 17), 3), (2, (64, 64), 3), (3, (65, 49), 6), (65, (130, 67), 2),
+                                                (200, (95, 70), 1), (97, (160, 120), 24)])
+def test_forward_and_adjoint_by_size(gi, oracle_lib, cuda, map_size, view, freq):
+    st = _Sized(gi, oracle_lib, map_size, view, freq)
+    got, want = st.gpu_forward(st.L, st.r), st.oracle_forward(st.L, st.r)
+    assert np.abs(got - want).max() <= 1e-6
+    g = np.random.default_rng(map_size).standard_normal(st.gpos.shape[1:])
+    gL, gr, gv = _adjoint(st, g)
+    exact, light = st.oracle_adjoint(g)
+    assert (np.abs(gv - exact) <= 1e-3 * np.abs(exact) + 2e-5 * np.abs(exact).max()).all()
+    assert (np.abs(np.array([*gL, gr]) - light) <= 2e-5 * np.abs(light).sum()).all()
