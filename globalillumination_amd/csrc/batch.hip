@@ -196,7 +196,8 @@ __global__ __launch_bounds__(256) void kb_bin_wide(RasterTable t) {
         const int j = find_job(pre, t.njobs, item);
         const RasterJob& J = t.jobs[j];
         const uint32_t local = item - pre[j];
-        bin_wide_body<TS, kScatter>(J.cfg, J.b, (int)(local % kWideBlocks), kWideBlocks, (int)(local / kWideBlocks));
+        bin_wide_body<TS, kScatter>(J.cfg, J.b, (int)(local % kWideBlocks), kWideBlocks, (int)(local / kWideBlocks),
+                                    kWideBlocks);
     }
 }
 

@@ -754,16 +754,21 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(MeshView mesh, MvpSource 
     clip_body<NA>(mesh, mvps, cfg, b, blockIdx.x, gridDim.x, blockIdx.y);
 }
 
-// Wide pieces (setup records), kWideThreads threads per workgroup.  Part p
-// of nparts takes records p, p + nparts, p + 2 nparts, ..., one per thread,
-// kWideThreads records a round.  The round's (record, tile) pairs are
-// numbered through a prefix sum of the records' tile spans, and each thread
-// takes every kWideThreads-th pair, so the pairs' appends (whose scatter
-// atomics return the list slot) are all in flight at once whether the round
-// holds many records of a few tiles (a triangle soup on a large map) or one
-// record over the whole map (a ground plane's clipped piece); a map's few
-// records still go to different parts.
+// Wide pieces (setup records), kWideThreads threads per workgroup, nparts
+// workgroups a map.  A round holds kWideThreads records, one per thread; its
+// (record, tile) pairs are numbered through a prefix sum of the records' tile
+// spans, so that the pairs' appends (whose scatter atomics return the list
+// slot) are all in flight at once whether the round holds many records of a
+// few tiles or one record over the whole map.  A map of one round (a ground
+// plane's clipped pieces) has its pairs dealt to `shares` parts, each of which
+// numbers the same round: a piece over the 4,096 tiles of a 4096^2 map was one
+// part's 16 appends per thread, one after another (count 11.5 us, scatter 17
+// us; dealt out 4.7 and 10).  With more records, part p takes records p, p +
+// nparts, ... and every kWideThreads-th pair of them.  Launches of many maps
+// deal each map's to fewer parts, about 1,024 in all (wide_shares): 289 maps
+// of 81 tiles took 24 and 87 us with 64 parts each, 18 and 78 without dealing.
 constexpr int kWideThreads = 256;
+__device__ __forceinline__ int wide_shares(int nmaps) { return max(8, min(kWideBlocks, 1024 / nmaps)); }
 
 template <int TS, bool kScatter>
 __device__ __forceinline__ void wide_tile(const RasterCfg& cfg, const BinBufs& b, int map, int ntiles, const Setup& s,
@@ -775,17 +780,21 @@ __device__ __forceinline__ void wide_tile(const RasterCfg& cfg, const BinBufs& b
 }
 
 template <int TS, bool kScatter>
-__device__ __forceinline__ void bin_wide_body(const RasterCfg& cfg, const BinBufs& b, int part, int nparts, int map) {
+__device__ __forceinline__ void bin_wide_body(const RasterCfg& cfg, const BinBufs& b, int part, int nparts, int map,
+                                              int shares) {
     __shared__ int incl[kWideThreads];  // inclusive prefix of the round's spans
     __shared__ int wave_sum[kWideThreads / 64];
     if (kScatter && b.overflow[map]) return;  // uniform per workgroup
     const int ntiles = cfg.tiles_x * cfg.tiles_y;
     const uint32_t n = min(b.nwide[map], b.wcap);
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const uint32_t stride = (uint32_t)nparts;
+    const bool share = n <= (uint32_t)kWideThreads;
+    const uint32_t first = share ? 0u : (uint32_t)part, stride = share ? 1u : (uint32_t)nparts;
+    const int pair0 = share ? part * kWideThreads + tid : tid, pairs = share ? shares * kWideThreads : kWideThreads;
+    if (share && part >= shares) return;  // uniform
     const Setup* recs = b.wide + (size_t)map * b.wcap;
-    for (uint32_t r0 = 0; (uint32_t)part + stride * r0 < n; r0 += kWideThreads) {  // uniform
-        const uint32_t w = (uint32_t)part + stride * (r0 + (uint32_t)tid);
+    for (uint32_t r0 = 0; first + stride * r0 < n; r0 += kWideThreads) {  // uniform
+        const uint32_t w = first + stride * (r0 + (uint32_t)tid);
         int span = 0;
         if (w < n) {
             const Setup& s = recs[w];
@@ -807,7 +816,7 @@ __device__ __forceinline__ void bin_wide_body(const RasterCfg& cfg, const BinBuf
         }
         incl[tid] = base + v;
         lds_barrier();
-        for (int p = tid; p < total; p += kWideThreads) {
+        for (int p = pair0; p < total; p += pairs) {
             // the round's record holding pair p: the first k with incl[k] > p
             int lo = 0, hi = kWideThreads - 1;
             while (lo < hi) {
@@ -815,7 +824,7 @@ __device__ __forceinline__ void bin_wide_body(const RasterCfg& cfg, const BinBuf
                 if (incl[mid] > p) hi = mid;
                 else lo = mid + 1;
             }
-            const uint32_t wk = (uint32_t)part + stride * (r0 + (uint32_t)lo);
+            const uint32_t wk = first + stride * (r0 + (uint32_t)lo);
             const Setup s = recs[wk];
             const int tx0 = s.px0 / TS, ty0 = s.py0 / TS;
             const int ntx = s.px1 / TS - tx0 + 1;
@@ -828,7 +837,7 @@ __device__ __forceinline__ void bin_wide_body(const RasterCfg& cfg, const BinBuf
 
 template <int TS, bool kScatter>
 __global__ __launch_bounds__(256) void k_bin_wide(RasterCfg cfg, BinBufs b) {
-    bin_wide_body<TS, kScatter>(cfg, b, blockIdx.x, gridDim.x, blockIdx.y);
+    bin_wide_body<TS, kScatter>(cfg, b, blockIdx.x, gridDim.x, blockIdx.y, wide_shares((int)gridDim.y));
 }
 
 // The scatter pass when the count pass stored each triangle's tile code
@@ -908,7 +917,8 @@ __device__ __forceinline__ void bin_scatter_body(const MeshView& mesh, const Ras
 template <int TS, int kT>
 __global__ __launch_bounds__(256) void k_bin_scatter(MeshView mesh, RasterCfg cfg, BinBufs b, int tri_blocks) {
     if ((int)blockIdx.x >= tri_blocks) {  // uniform per workgroup
-        bin_wide_body<TS, true>(cfg, b, (int)blockIdx.x - tri_blocks, kWideBlocks, (int)blockIdx.y);
+        bin_wide_body<TS, true>(cfg, b, (int)blockIdx.x - tri_blocks, kWideBlocks, (int)blockIdx.y,
+                                wide_shares((int)gridDim.y));
         return;
     }
     bin_scatter_body<TS, kT>(mesh, cfg, b, (int)blockIdx.x, (int)blockIdx.y);

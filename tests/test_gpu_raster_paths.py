@@ -97,3 +97,22 @@ def test_records_put_aside_by_count(gi, oracle_lib, cuda, n):
         for k in range(first, maps, 2):
             assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k}")
         assert (want < 1.0).mean() > 0.3
+
+
+@pytest.mark.parametrize("n,maps", [(1, 1), (3, 2), (254, 1), (256, 1), (257, 1), (300, 3), (40, 20), (130, 130)])
+def test_wide_records_by_count(gi, oracle_lib, cuda, n, maps):
+    """n triangles over many tiles each, around the 256 records up to which a
+    map's (record, tile) pairs are dealt to all its workgroups, for few and
+    for many maps."""
+    rng = np.random.default_rng(200 + n)
+    w, h = 320, 200
+    pos = rng.uniform(-1.0, 1.0, size=(n, 3, 3)) * [0.999, 0.999, 0.9]
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3).astype(np.float32), np.zeros((3 * n, 3), np.float32),
+                          np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvps = np.tile(np.eye(4, dtype=np.float32).reshape(1, 16), (maps, 1))
+    mvps[1::2, 10] = 0.5
+    got = gi.render_shadow_map(gi.DeviceMesh.from_mesh(mesh), mvps, w, h).cpu().numpy()
+    for first in range(min(maps, 2)):
+        want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvps[first], w, h)
+        for k in range(first, maps, 2):
+            assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k}")
