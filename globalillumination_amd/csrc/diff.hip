@@ -44,7 +44,6 @@ constexpr int kThreads = 256;
 constexpr int kTexPerThread = 8;   // texels per thread in the texel adjoint
 constexpr int kGatherMax = 256;    // bbox texels up to which a triangle gathers its own adjoint
 constexpr int kLargeSlots = 4;     // large triangles a texel block sums in LDS
-constexpr int kMapsPerThread = 1;  // maps a triangle-adjoint thread walks (vertex gradients summed over them)
 constexpr int kGatherBatch = 8;    // bounding-box texels whose keys a gather loads together
 constexpr int kBwdPixPerThread = 4;  // pixels a pixel-adjoint thread sums before the block reduction
 
@@ -561,8 +560,14 @@ __global__ __launch_bounds__(kThreads) void k_diff_large_reduce(const LargePart*
     }
 }
 
-// Triangle adjoint.  grid (triangle blocks, S / kMapsPerThread): a thread
-// walks kMapsPerThread maps of one triangle.  w_j = sum of G * lambda_j
+// Maps a triangle-adjoint thread walks.  The float atomics of its vertex
+// gradients bound the kernel, so a thread sums two maps' first where that
+// leaves the GPU its workgroups: 50k triangles in 16 maps 70 us, 91 with one map
+// a thread, 76 with four, 132 with eight.
+inline int maps_per_thread(int tri_blocks, int S) { return (long long)tri_blocks * S >= 2048 ? 2 : 1; }
+
+// Triangle adjoint.  grid (triangle blocks, ceil(S / per)): a thread walks
+// `per` maps of one triangle.  w_j = sum of G * lambda_j
 // over the triangle's texels in map i: gathered here over the triangle's
 // bounding box (texels whose visibility key names it) for small triangles,
 // read from the texel pass's sums for large ones.  The texel depths then move
@@ -578,30 +583,38 @@ __global__ __launch_bounds__(kThreads) void k_diff_tri_bwd(const float* __restri
                                                            const unsigned long long* __restrict__ vis,
                                                            const float* __restrict__ grad_depth,
                                                            const double* __restrict__ wsum_all,
+                                                           const unsigned char* __restrict__ large,
                                                            const unsigned char* __restrict__ touched, DiffCfg c,
-                                                           float* __restrict__ grad_pos,
+                                                           int per, float* __restrict__ grad_pos,
                                                            double* __restrict__ partial) {
     const int t = blockIdx.x * kThreads + threadIdx.x;
     // vertex gradients summed over this thread's maps, added once at the end
     double gvs[3][3];
 #pragma unroll
     for (int j = 0; j < 3; ++j) gvs[j][0] = gvs[j][1] = gvs[j][2] = 0.0;
-    const int i0 = blockIdx.y * kMapsPerThread;
-    const int i1 = min(i0 + kMapsPerThread, c.S);
+    const int i0 = blockIdx.y * per;
+    const int i1 = min(i0 + per, c.S);
     for (int i = i0; i < i1; ++i) {
         double gm[16];
 #pragma unroll
         for (int e = 0; e < 16; ++e) gm[e] = 0.0;
         double w[3] = {0.0, 0.0, 0.0};
-        if (t < ntris) {
+        // two flag bytes tell whether the triangle has gradient at all: most
+        // workgroups end here
+        const bool big = t < ntris && large[(size_t)i * ntris + t], small = t < ntris && touched[(size_t)i * ntris + t];
+        if (!__syncthreads_or(big || small)) {
+            if (threadIdx.x < 16) partial[((size_t)i * gridDim.x + blockIdx.x) * 16 + threadIdx.x] = 0.0;
+            continue;
+        }
+        if (big || small) {
             const TriPlane p = planes[(size_t)i * ntris + t];
             if (plane_ok(p)) {
-                if (plane_large(p)) {
+                if (big) {
                     const double* ws = wsum_all + ((size_t)i * ntris + t) * 3;
                     w[0] = ws[0];
                     w[1] = ws[1];
                     w[2] = ws[2];
-                } else if (touched[(size_t)i * ntris + t]) {
+                } else {
                     // bounding-box texels in batches whose loads are issued together
                     const size_t moff = (size_t)i * c.smw * c.smh;
                     const int area = bbox_area(p);
@@ -735,6 +748,7 @@ struct DiffWs {
     unsigned char* touched;
     void* raster;
     size_t raster_bytes;
+    size_t zero_words;  // from grad_depth on: the adjoint's sums and flags
     int px_blocks, pxb_blocks, tri_blocks, tx_blocks;
 };
 
@@ -748,15 +762,18 @@ size_t diff_layout(int ntris, int S, int smw, int smh, int gw, int gh, DiffWs* w
     size_t off = 0;
     size_t o_m32 = off; off = align256(off + sizeof(float) * 16 * (size_t)S);
     size_t o_vis = off; off = align256(off + sizeof(unsigned long long) * msz * S);
+    // cleared together before the adjoint: [zero, zero_end)
+    const size_t zero = off;
     size_t o_gd = off; off = align256(off + sizeof(float) * msz * S);
+    size_t o_ws = off; off = align256(off + sizeof(double) * 3 * (size_t)ntris * S);
+    size_t o_tc = off; off = align256(off + (size_t)ntris * S);
+    const size_t zero_words = (off - zero) / sizeof(float);
     size_t o_tx = off; off = align256(off + sizeof(TexelPlane) * (size_t)ntris * S);
     size_t o_pl = off; off = align256(off + sizeof(TriPlane) * (size_t)ntris * S);
-    size_t o_ws = off; off = align256(off + sizeof(double) * 3 * (size_t)ntris * S);
     size_t o_ppx = off; off = align256(off + sizeof(double) * 16 * (size_t)px_blocks * S);
     size_t o_ptr = off; off = align256(off + sizeof(double) * 16 * (size_t)(tri_blocks > 0 ? tri_blocks : 1) * S);
     size_t o_lp = off; off = align256(off + sizeof(LargePart) * kLargeSlots * (size_t)tx_blocks * S);
     size_t o_lg = off; off = align256(off + (size_t)ntris * S);
-    size_t o_tc = off; off = align256(off + (size_t)ntris * S);
     size_t rbytes = internal::vis_raster_workspace_size(ntris, S, smw, smh);
     size_t o_r = off; off = align256(off + rbytes);
     if (ws) {
@@ -773,6 +790,7 @@ size_t diff_layout(int ntris, int S, int smw, int smh, int gw, int gh, DiffWs* w
         ws->touched = reinterpret_cast<unsigned char*>(base + o_tc);
         ws->raster = base + o_r;
         ws->raster_bytes = rbytes;
+        ws->zero_words = zero_words;
         ws->px_blocks = px_blocks;
         ws->pxb_blocks = pxb_blocks;
         ws->tri_blocks = tri_blocks;
@@ -871,24 +889,20 @@ int gi_diff_soft_backward(const float* positions_dev, int nverts, const int32_t*
     // evaluates the texel depths it reads from the keys and planes
     rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, true);
     if (rc != GI_OK) return rc;
-    const size_t msz = (size_t)smw * smh * nsamples;
-    hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(kThreads), 0, s, w.grad_depth, msz, 0.0f);
+    hipLaunchKernelGGL(k_fill_f32, dim3(2048), dim3(kThreads), 0, s, w.grad_depth, w.zero_words, 0.0f);
     hipLaunchKernelGGL(k_diff_shade_bwd, dim3(w.pxb_blocks, nsamples), dim3(kThreads), 0, s, gbuffer->position_dev,
                        biased_mvps_dev, w.vis, w.texels, ntris, grad_out_dev, c, w.grad_depth, w.part_px);
     hipLaunchKernelGGL(k_diff_reduce, dim3(nsamples), dim3(kThreads), 0, s, w.part_px, w.pxb_blocks,
                        grad_biased_mvps_dev);
     if (ntris > 0) {
-        hipLaunchKernelGGL(k_fill_f64, dim3(256), dim3(kThreads), 0, s, w.wsum, (size_t)3 * ntris * nsamples, 0.0);
-        // touched flags: the region is 256-byte aligned and padded, so whole words clear it
-        hipLaunchKernelGGL(k_fill_f32, dim3(64), dim3(kThreads), 0, s, reinterpret_cast<float*>(w.touched),
-                           ((size_t)ntris * nsamples + 3) / 4, 0.0f);
         hipLaunchKernelGGL(k_diff_texel_bwd, dim3(w.tx_blocks, nsamples), dim3(kThreads), 0, s, w.vis, w.planes,
                            w.large, ntris, w.grad_depth, c, w.wsum, w.parts, w.touched);
         hipLaunchKernelGGL(k_diff_large_reduce, dim3(nsamples), dim3(kThreads), 0, s, w.parts, w.tx_blocks, ntris,
                            w.wsum);
-        hipLaunchKernelGGL(k_diff_tri_bwd, dim3(w.tri_blocks, (nsamples + kMapsPerThread - 1) / kMapsPerThread),
+        const int per = maps_per_thread(w.tri_blocks, nsamples);
+        hipLaunchKernelGGL(k_diff_tri_bwd, dim3(w.tri_blocks, (nsamples + per - 1) / per),
                            dim3(kThreads), 0, s, positions_dev,
-                           indices_dev, ntris, mvps_dev, w.planes, w.vis, w.grad_depth, w.wsum, w.touched, c,
+                           indices_dev, ntris, mvps_dev, w.planes, w.vis, w.grad_depth, w.wsum, w.large, w.touched, c, per,
                            grad_positions_dev, w.part_tri);
         hipLaunchKernelGGL(k_diff_reduce, dim3(nsamples), dim3(kThreads), 0, s, w.part_tri, w.tri_blocks,
                            grad_mvps_dev);
