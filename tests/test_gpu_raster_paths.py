@@ -116,3 +116,18 @@ def test_wide_records_by_count(gi, oracle_lib, cuda, n, maps):
         want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvps[first], w, h)
         for k in range(first, maps, 2):
             assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k}")
+
+
+@pytest.mark.parametrize("w,h", [(64, 64), (64, 4096), (2048, 2048), (4096, 1100), (4096, 2240)])
+def test_tile_lists_by_grid(gi, oracle_lib, cuda, w, h):
+    """The scan of a map's tile counts with one tile, one per thread, and
+    several per thread of its workgroup."""
+    rng = np.random.default_rng(w + h)
+    n = 400
+    pos = rng.uniform(-1.0, 1.0, size=(n, 1, 3)) * [0.95, 0.95, 0.9] + rng.uniform(-0.05, 0.05, size=(n, 3, 3))
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3).astype(np.float32), np.zeros((3 * n, 3), np.float32),
+                          np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvp = np.eye(4, dtype=np.float32).reshape(1, 16)
+    got = gi.render_shadow_map(gi.DeviceMesh.from_mesh(mesh), mvp, w, h).cpu().numpy()[0]
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp[0], w, h)
+    assert bits_equal(got, want), mismatch_report(got, want, f"{w}x{h}")
