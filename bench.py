@@ -263,16 +263,15 @@ def diff_timing(gi, torch, steps, warmup):
     fb = float(np.mean([e[1].elapsed_time(e[2]) for e in evs]))
     # Algorithmic bytes (lower bounds: the texels the taps read are not
     # counted).  Forward, per texel of the S maps: the 64-bit visibility key
-    # written and read back, the FP64 depth written (24 B); per (map,
-    # triangle): the vertices read twice (72 B), the 80-byte plane record
-    # written and read back and its size flag (161 B); per pixel: position in,
-    # output out (16 B).  Backward repeats the key and plane work and adds the
-    # FP32 texel adjoint cleared, scatter-added and read (12 B per texel), the
-    # key read by the texel adjoint (8 B) and the pixel adjoint's output
-    # gradient read (4 B per pixel).
+    # written (8 B); per (map, triangle): the vertices read twice (72 B) and the
+    # 32-byte depth record written; per pixel: position in, output out (16 B).
+    # Backward repeats that and adds the FP32 texel adjoint cleared,
+    # scatter-added and read (12 B per texel), the key read by the texel adjoint
+    # (8 B), the 80-byte plane record written and read back and its size flag
+    # (161 B), and the pixel adjoint's output gradient read (4 B per pixel).
     S, msz, nt, npx = len(light.offsets), light.map_size ** 2, wl.mesh.ntris, g.width * g.height
-    fwd_bytes = S * msz * 24 + S * nt * (72 + 161) + npx * 16
-    bwd_bytes = S * msz * (16 + 12 + 8) + S * nt * (72 + 161) + npx * 20
+    fwd_bytes = S * msz * 8 + S * nt * (72 + 32) + npx * 16
+    bwd_bytes = S * msz * (8 + 12 + 8) + S * nt * (72 + 32 + 161) + npx * 20
     return {"workload": "differentiable soft shadows: 16 samples, 1024^2 maps, 512x512 view, "
                         f"{wl.mesh.ntris:,}-triangle displaced icosphere + ground",
             "fwd_ms": round(fwd, 4), "fwd_bwd_ms": round(fb, 4), "fwd_bwd_over_fwd": round(fb / fwd, 3),
@@ -287,7 +286,7 @@ def diff_timing(gi, torch, steps, warmup):
 def batch_timing(gi, torch, steps):
     """The 32-instance batch (maps 512^2-4096^2, views 640x480-1920x1080,
     5k-300k-triangle soups, 1-16 light samples, seed 4): the per-instance
-    passes one after another, the batch's persistent launches, and the same
+    passes one after another, the batch's stage launches, and the same
     launches replayed from a hipGraph, after the autotuner has picked the
     launch shape.  HIP events on the current stream; inputs resident."""
     import numpy as np

@@ -4,7 +4,7 @@ An instance is the work of one renderMonteCarlo frame
 (SoftShadowMapping/src/main.cpp:756-811): the depth maps of its light samples
 and the soft-shadow screen pass over its camera G-buffer.  A Batch runs many
 instances (different meshes, map sizes, sample counts and views) as one
-sequence of persistent kernels, optionally captured in one hipGraph; every
+sequence of kernels over all of them, optionally captured in one hipGraph; every
 map and shadow value equals the per-instance passes (render_shadow_map +
 render_monte_carlo) bit for bit.
 """

@@ -763,7 +763,7 @@ __global__ __launch_bounds__(kClipThreads) void k_clip(MeshView mesh, MvpSource 
 // plane's clipped pieces) has its pairs dealt to `shares` parts, each of which
 // numbers the same round: a piece over the 4,096 tiles of a 4096^2 map was one
 // part's 16 appends per thread, one after another (count 11.5 us, scatter 17
-// us; dealt out 4.7 and 10).  With more records, part p takes records p, p +
+// us; dealt out 4.5 and 8.4).  With more records, part p takes records p, p +
 // nparts, ... and every kWideThreads-th pair of them.  Launches of many maps
 // deal each map's to fewer parts, about 1,024 in all (wide_shares): 289 maps
 // of 81 tiles took 24 and 87 us with 64 parts each, 18 and 78 without dealing.

@@ -538,8 +538,8 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
                     gi_batch** out);
 int gi_batch_set_tuning(gi_batch* b, const gi_batch_tuning* t);
 int gi_batch_get_tuning(const gi_batch* b, gi_batch_tuning* t);
-/* Enqueues the whole batch: the raster stages as persistent kernels over all
- * instances, then the screen pass as one persistent kernel per PCF variant.
+/* Enqueues the whole batch: each raster stage as one kernel over all
+ * instances, then the screen pass as one kernel per PCF variant.
  * Launches only (no allocation, copy or memset), so it can be captured. */
 int gi_batch_run(gi_batch* b, gi_stream stream);
 /* Times every tuning candidate on `stream` (reps runs each, after one
