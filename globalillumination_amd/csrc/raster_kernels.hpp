@@ -934,14 +934,19 @@ __device__ __forceinline__ uint32_t* split_tiles(const BinBufs& b, int map) {
 }
 
 // Entries from which a tile's list is split, for a launch of `nmaps` maps like
-// one with `total` entries: a CU's even share of the launch, and no less than
-// kSplitMin, below which the 16 passes over the list cost more than they
-// spread.  A quarter of that share (1,024 for 256 below) splits lists whose
-// tiles fill the GPU anyway: 16 visibility maps of 1024^2 (50,002 triangles)
-// 235 us against 138 us, one 4096^2 map (100,822 triangles) 58 against 48 us.
+// one with `total` entries in `ntiles` tiles: a CU's even share of the launch,
+// and no less than kSplitMin, below which the 16 passes over the list cost more
+// than they spread.  A quarter of that share splits lists whose tiles fill the
+// GPU anyway: 16 visibility maps of 1024^2 (50,002 triangles, 4,096 tiles) 235 us
+// against 138 us, one 4096^2 map (100,822 triangles) 58 against 48 us.  Launches
+// of at most 1,024 tiles, four a CU, do not fill it, and take the quarter: the
+// 510 tiles of a 200k-triangle soup's G-buffer 67 us, 83 with the whole share;
+// single maps of 16 to 1,024 tiles with few long lists are the same with both.
 constexpr uint32_t kSplitMin = 48;
-__device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nmaps) {
-    const unsigned long long even = total * (unsigned)nmaps / 256ull;
+constexpr int kSplitRoomy = 1024;
+__device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nmaps, int ntiles) {
+    const unsigned long long shares = (long long)ntiles * nmaps <= kSplitRoomy ? 1024ull : 256ull;
+    const unsigned long long even = total * (unsigned)nmaps / shares;
     return even > kSplitMin ? (uint32_t)min(even, 0x7FFFFFFFull) : kSplitMin;
 }
 
@@ -976,7 +981,7 @@ __device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map,
         run += k < wave ? wave_sum[k] : 0ull;
         total += wave_sum[k];
     }
-    const uint32_t bound = split_maps > 0 ? split_bound(total, split_maps) : 0u;
+    const uint32_t bound = split_maps > 0 ? split_bound(total, split_maps, ntiles) : 0u;
     uint32_t* split = split_tiles(b, map);
     for (int i = lo; i < hi; ++i) {
         o[i] = (uint32_t)run;
@@ -1596,7 +1601,7 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
 // first 16 bytes, kSplitLoads in flight per thread), and rasterizes the
 // entries that touch the region from a list in LDS.  Raster of one map, tiles
 // only and with split lists: 200k soup, 2048^2: 130 and 47 us (its G-buffer at
-// 1920x1080: 232 and 85 us); 100,822 triangles seen from 315 units, 2048^2: 98
+// 1920x1080: 232 and 67 us); 100,822 triangles seen from 315 units, 2048^2: 98
 // and 43 us; a 3,970-triangle scene, 1024^2: 43 and 17 us, 256^2: 26 and 13 us.
 // ---------------------------------------------------------------------------
 constexpr int kSplitEdge = 16;

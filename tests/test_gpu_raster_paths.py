@@ -131,3 +131,25 @@ def test_tile_lists_by_grid(gi, oracle_lib, cuda, w, h):
     got = gi.render_shadow_map(gi.DeviceMesh.from_mesh(mesh), mvp, w, h).cpu().numpy()[0]
     want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp[0], w, h)
     assert bits_equal(got, want), mismatch_report(got, want, f"{w}x{h}")
+
+
+@pytest.mark.parametrize("w,h,n", [(2048, 2048, 200), (2048, 2048, 6000), (2049, 2048, 6000), (320, 200, 3000),
+                                   (1024, 512, 40000)])
+def test_long_lists_by_launch(gi, oracle_lib, cuda, w, h, n):
+    """Triangles that crowd a few tiles of launches with 1,024 tiles and fewer
+    (whose lists are split from a quarter of a CU's share) and with more;
+    depth map and G-buffer."""
+    rng = np.random.default_rng(n)
+    cen = rng.uniform(-1.0, 1.0, size=(n, 1, 3)) * [200.0 / w, 200.0 / h, 0.9]
+    pos = (cen + rng.uniform(-1.0, 1.0, size=(n, 3, 3)) * [12.0 / w, 12.0 / h, 0.05]).astype(np.float32)
+    nrm = rng.normal(size=(3 * n, 3)).astype(np.float32)
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3), nrm, np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvp = np.eye(4, dtype=np.float32).reshape(16)
+    dm = gi.DeviceMesh.from_mesh(mesh)
+    got = gi.render_shadow_map(dm, mvp, w, h).cpu().numpy()[0]
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp, w, h)
+    assert bits_equal(got, want), mismatch_report(got, want, "depth")
+    g = gi.render_gbuffer(dm, mvp, w, h)
+    pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
+    assert bits_equal(g.position.cpu().numpy(), pos_o)
+    assert bits_equal(g.normal.cpu().numpy(), nrm_o)
