@@ -234,8 +234,8 @@ __global__ void kb_overflow_any(RasterTable t, uint32_t* __restrict__ flag) {
 // place on the CU through the chain of counter, job and list loads of each
 // item.  Twelve frames of soups (512^2 to 4096^2 maps): 2.74 ms from a queue
 // with 8 workgroups per CU, 2.01 ms so.
-template <int TS, bool kBig>
-__global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_raster(RasterTable t, uint32_t first) {
+template <int TS>
+__global__ __launch_bounds__(kRasterThreads, TS == 32 ? 1 : 8) void kb_raster(RasterTable t, uint32_t first) {
     __shared__ __align__(16) uint32_t tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
@@ -246,7 +246,7 @@ __global__ __launch_bounds__(kRasterThreads, kBig || TS == 32 ? 1 : 8) void kb_r
     const uint32_t local = item - pre[j];
     const int map = (int)(local % (uint32_t)J.nmaps), tile_id = (int)(local / (uint32_t)J.nmaps);
     if (J.b.overflow[map]) return;  // left to kb_raster_fallback
-    raster_tile<TS, false, false, kBig>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, false);
+    raster_tile<TS, false, false>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, false);
 }
 
 template <int TS>
@@ -263,8 +263,7 @@ __global__ __launch_bounds__(kRasterThreads) void kb_raster_fallback(RasterTable
         const int tile_id = (int)(item - pre[j]);
         for (int map = 0; map < J.nmaps; ++map) {
             if (!J.b.overflow[map]) continue;
-            raster_tile<TS, false, true, true>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec,
-                                               true);
+            raster_tile<TS, false, true>(J.mesh, mvp_of(J), J.cfg, J.b, J.out, map, tile_id, tile, rec, nrec, true);
             __syncthreads();
         }
     }
@@ -389,7 +388,6 @@ struct gi_batch {
     SoftGroup sg[kShapes][kNtGroups];
     uint32_t* counters;
     char* ws;  // the workspace: every job's binning buffers lie in it
-    bool big;  // some map is a big_view
 };
 
 struct gi_batch_graph {
@@ -424,13 +422,10 @@ void launch_scatter(const RasterVariant& R, const RasterTable& tab, char* ws, un
 constexpr uint32_t kMaxGroups = 1u << 23;
 
 template <int TS>
-void launch_raster(uint32_t total, const RasterTable& tab, bool big, hipStream_t s) {
+void launch_raster(uint32_t total, const RasterTable& tab, hipStream_t s) {
     for (uint32_t first = 0; first < total; first += kMaxGroups) {
         const dim3 grid(total - first < kMaxGroups ? total - first : kMaxGroups);
-        if (big)
-            hipLaunchKernelGGL((kb_raster<TS, true>), grid, dim3(kRasterThreads), 0, s, tab, first);
-        else
-            hipLaunchKernelGGL((kb_raster<TS, false>), grid, dim3(kRasterThreads), 0, s, tab, first);
+        hipLaunchKernelGGL((kb_raster<TS>), grid, dim3(kRasterThreads), 0, s, tab, first);
     }
 }
 
@@ -452,7 +447,7 @@ int run_depth(gi_batch* b, const gi_batch_tuning& T, hipStream_t s) {
     launch_scatter<TS>(R, tab, b->ws, cap, s);                                                                     \
     if ((g = grid_of(R.total[kStWide], cap)))                                                                       \
         hipLaunchKernelGGL((kb_bin_wide<TS, true>), dim3(g), dim3(256), 0, s, tab);                                 \
-    launch_raster<TS>(R.total[kStRaster], tab, b->big, s);                                                          \
+    launch_raster<TS>(R.total[kStRaster], tab, s);                                                                  \
     if ((g = grid_of(R.total[kStFallback], cap)))                                                                   \
         hipLaunchKernelGGL((kb_raster_fallback<TS>), dim3(g), dim3(kRasterThreads), 0, s, tab);
     if (T.tile == 32) {
@@ -581,7 +576,6 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
     b->tuning = gi_batch_tuning{64, 4, 3, 4};
     b->counters = reinterpret_cast<uint32_t*>(base + L.counters);
     b->ws = base;
-    b->big = false;
     for (int v = 0; v < 2; ++v) {
         const int ts = kTiles[v];
         RasterJob* jobs = reinterpret_cast<RasterJob*>(img.data() + L.rjobs[v]);
@@ -596,7 +590,6 @@ int gi_batch_create(const gi_batch_instance* inst, int n, void* workspace_dev, s
             J.mvps = I.light_mvps_dev;
             J.cfg = RasterCfg{I.sm_width, I.sm_height, (I.sm_width + ts - 1) / ts, (I.sm_height + ts - 1) / ts,
                               I.polygon_offset_factor, I.polygon_offset_units};
-            b->big = b->big || big_view(J.cfg);
             J.b = ws.bins;
             J.out = I.maps_dev;
             J.nzero = (uint32_t)zero_words(I.nsamples, J.cfg);

@@ -114,21 +114,12 @@ int raster_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, int map
     const unsigned tiles = (unsigned)(ntiles * map_count);
     const dim3 block(kRasterThreads);
     const bool spread = tiles <= kSpreadTiles;
-    if (splits_lists(ntiles, nmaps)) {
-        const dim3 grid(tiles + kSplitWorkers);
-        if (big_view(cfg))
-            hipLaunchKernelGGL((k_raster_split<kTile, kVis, true>), grid, block, 0, s, mesh, mvps, cfg, ws.bins, out,
-                               map_begin, map_count);
-        else
-            hipLaunchKernelGGL((k_raster_split<kTile, kVis, false>), grid, block, 0, s, mesh, mvps, cfg, ws.bins, out,
-                               map_begin, map_count);
-    } else if (big_view(cfg)) {
-        hipLaunchKernelGGL((k_raster<kTile, kVis, true>), dim3(tiles), block, 0, s, mesh, mvps, cfg, ws.bins, out,
-                           map_begin, map_count, spread);
-    } else {
-        hipLaunchKernelGGL((k_raster<kTile, kVis, false>), dim3(tiles), block, 0, s, mesh, mvps, cfg, ws.bins, out,
-                           map_begin, map_count, spread);
-    }
+    if (splits_lists(ntiles, nmaps))
+        hipLaunchKernelGGL((k_raster_split<kTile, kVis>), dim3(tiles + kSplitWorkers), block, 0, s, mesh, mvps, cfg,
+                           ws.bins, out, map_begin, map_count);
+    else
+        hipLaunchKernelGGL((k_raster<kTile, kVis>), dim3(tiles), block, 0, s, mesh, mvps, cfg, ws.bins, out, map_begin,
+                           map_count, spread);
     if (ev_end && hipEventRecord(ev_end, s) != hipSuccess) return GI_EDEVICE;
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }

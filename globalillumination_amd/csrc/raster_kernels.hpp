@@ -308,10 +308,23 @@ __device__ __forceinline__ uint32_t fbits(float f) { return __float_as_uint(f); 
 // per map in HBM (written once by the binning pass); pieces a whole workgroup
 // rasterizes are shared through LDS.
 // ---------------------------------------------------------------------------
+// An edge of 2^23 units (32,768 pixels) or more in x or y, past the 24-bit
+// factors of tile_edges: such a record takes the 64-bit edge functions.  The
+// vertices themselves decide: the guard band keeps an unclipped triangle's
+// edges below four views, but a clipped vertex's x and w are rounded one by one
+// and can lie outside it by any factor (a ground of 10^8 units seen from 1:
+// 1.7%, so past the limit from views of 8,060 pixels on).
+constexpr int kLongEdge = 8;
+__device__ __forceinline__ int long_edge(const int X[3], const int Y[3]) {
+    const int dx = max(max(abs(X[1] - X[0]), abs(X[2] - X[1])), abs(X[0] - X[2]));
+    const int dy = max(max(abs(Y[1] - Y[0]), abs(Y[2] - Y[1])), abs(Y[0] - Y[2]));
+    return max(dx, dy) < (1 << 23) ? 0 : kLongEdge;
+}
+
 struct Setup {
     int X[3], Y[3];            // 24.8 fixed-point window coordinates
     int px0, px1, py0, py1;    // pixel-centre bounding box (clamped)
-    int tl;                    // bit k: top-left tie bit of the edge opposite vertex k
+    int tl;                    // bit k: top-left tie bit of the edge opposite vertex k; kLongEdge
     uint32_t id;               // tri * 8 + fan piece
     float z0, A, B, zoff;      // depth plane about vertex 0
 };
@@ -325,7 +338,7 @@ __device__ __forceinline__ Setup to_setup(const Tri<NA>& t, uint32_t id) {
         s.Y[i] = t.Y[i];
     }
     s.px0 = t.px0; s.px1 = t.px1; s.py0 = t.py0; s.py1 = t.py1;
-    s.tl = t.tl[0] | (t.tl[1] << 1) | (t.tl[2] << 2);
+    s.tl = t.tl[0] | (t.tl[1] << 1) | (t.tl[2] << 2) | long_edge(t.X, t.Y);
     s.id = id;
     s.z0 = t.z0; s.A = t.A; s.B = t.B; s.zoff = t.zoff;
     return s;
@@ -1083,19 +1096,13 @@ __device__ __forceinline__ bool rect_inside(const Setup& s, int rx0, int rx1, in
 // part stays below 2^30 in magnitude when |ex| and |ey| are below 2^23, and a
 // first part of 2^30 or more then decides the test in the whole tile, so it is
 // clamped there and every sum fits in int32; the factors fit the 24-bit
-// multipliers.  ok is false for longer edges: 32,768 pixels and more, which
-// the guard band (four times the view) allows only in views of kBigView pixels
-// and more; the kernels' kBig variants send those records to raster_rect_slow.
-constexpr int kBigView = (1 << 23) / 256 / (int)kGuard;
-inline bool big_view(const RasterCfg& cfg) { return cfg.w >= kBigView || cfg.h >= kBigView; }
+// multipliers.  Not for records with kLongEdge, which go to raster_long.
 struct TileEdges {
     int e[3];
     int ex[3], ey[3];
-    bool ok;
 };
 __device__ __forceinline__ TileEdges tile_edges(const Setup& s, int x0, int y0) {
     TileEdges t;
-    t.ok = true;
     const int Px = x0 * 256 + 128, Py = y0 * 256 + 128;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -1106,7 +1113,6 @@ __device__ __forceinline__ TileEdges tile_edges(const Setup& s, int x0, int y0) 
         t.e[k] = (int)(r > (1ll << 30) ? (1ll << 30) - 1 : r < -(1ll << 30) ? -(1ll << 30) : r);
         t.ex[k] = ex;
         t.ey[k] = ey;
-        t.ok = t.ok && abs(ex) < (1 << 23) && abs(ey) < (1 << 23);
     }
     return t;
 }
@@ -1379,33 +1385,41 @@ struct ZBound {
     int age;
 };
 
+// The setup record of a list entry; `has` becomes false for an empty piece.
+template <int TS, bool kFallback>
+__device__ __forceinline__ void load_setup(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
+                                           const BinBufs& b, int map, uint32_t entry, bool& has, Setup& s) {
+    if (!has) return;
+    if (!kFallback && (entry & kWideBit)) {
+        s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
+    } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
+        // a directly binned triangle: the count pass stored its setup
+        s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
+    } else {
+        float mvp[16];
+        mvps.load(map, mvp);
+        Tri<0> t;
+        if constexpr (kFallback)
+            get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, has);
+        else
+            classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, has);
+        if (has) s = to_setup(t, entry);
+    }
+}
+
 // One round of list entries, one per lane (`has`: the lane has one).  Small
 // records are rasterized by their lane, larger ones by the wave in 8x8
-// blocks, those of more than `aside` blocks are put aside in `rec`.
-template <int TS, int RS, bool kVis, bool kFallback, bool kBig>
+// blocks, those of more than `aside` blocks are put aside in `rec`; one with a
+// long edge leaves its flag in nrec (raster_long).
+constexpr int kHasLong = (int)0x80000000u;
+template <int TS, int RS, bool kVis, bool kFallback>
 __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                              const BinBufs& b, int map, const Region& g, uint32_t entry, bool has,
                                              int aside, typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec,
                                              ZBound& z) {
     const int lane = (int)threadIdx.x & 63;
     Setup s;
-    if (has) {
-        if (!kFallback && (entry & kWideBit)) {
-            s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
-        } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
-            // a directly binned triangle: the count pass stored its setup
-            s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
-        } else {
-            float mvp[16];
-            mvps.load(map, mvp);
-            Tri<0> t;
-            if constexpr (kFallback)
-                get_piece<0>(mesh, mvp, (int)(entry >> 3), (int)(entry & 7u), cfg, t, has);
-            else
-                classify<0>(mesh, mvp, (int)(entry >> 3), cfg, t, has);
-            if (has) s = to_setup(t, entry);
-        }
-    }
+    load_setup<TS, kFallback>(mesh, mvps, cfg, b, map, entry, has, s);
     int rx0 = 0, rx1 = -1, ry0 = 0, ry1 = -1;
     if (has) {
         rx0 = max(g.x0, s.px0);
@@ -1421,13 +1435,13 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
         t = tile_edges(s, g.x0, g.y0);
         blocks = block_mask<RS>(rx0 - g.x0, rx1 - g.x0, ry0 - g.y0, ry1 - g.y0);
         area = (rx1 - rx0 + 1) * (ry1 - ry0 + 1);
-        if ((kBig && !t.ok) || __popcll(blocks) > aside) {
-            const int slot = atomicAdd(&nrec, 1);
+        if (s.tl & kLongEdge) {
+            atomicOr(&nrec, kHasLong);
+            has = false;
+        } else if (__popcll(blocks) > aside) {
+            const int slot = atomicAdd(&nrec, 1) & ~kHasLong;
             if (slot < kRecQueue) {
                 rec[slot] = s;
-                has = false;
-            } else if (kBig && !t.ok) {
-                raster_rect_slow<RS, kVis>(s, g.x0, g.y0, rx0, rx1, ry0, ry1, 0, 1, tile);
                 has = false;
             }
         }
@@ -1436,6 +1450,44 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
     const bool self = has && area <= bound;
     raster_lanes<RS, kVis, false>(s, t, blocks, has && !self, g.x0, g.y0, lane, z.zmax, z.age, tile);
     if (self) raster_rect_self<RS, kVis>(s, t, g.x0, g.y0, rx0, rx1, ry0, ry1, tile);
+}
+
+// The records with a long edge among entries [begin, end), every record by the
+// whole workgroup with the 64-bit edge functions.  Walking the list again here
+// keeps those functions' registers out of raster_round.
+template <int TS, int RS, bool kVis, bool kFallback>
+__device__ __forceinline__ void raster_long(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
+                                            const BinBufs& b, int map, const Region& g, uint32_t begin, uint32_t end,
+                                            typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec) {
+    const int tid = (int)threadIdx.x;
+    for (uint32_t base = begin; base < end; base += kRasterThreads) {
+        const uint32_t k = base + (uint32_t)tid;
+        bool mine = k < end;
+        Setup s;
+        const uint32_t entry = kFallback ? k : (mine ? b.entries[(size_t)map * b.cap + k] : 0u);
+        load_setup<TS, kFallback>(mesh, mvps, cfg, b, map, entry, mine, s);
+        mine = mine && (s.tl & kLongEdge) && s.px0 <= g.x1 && s.px1 >= g.x0 && s.py0 <= g.y1 && s.py1 >= g.y0;
+        for (int n = kRecQueue + 1; n > kRecQueue;) {  // until the queue held all that were left
+            __syncthreads();
+            if (tid == 0) nrec = 0;
+            __syncthreads();
+            if (mine) {
+                const int slot = atomicAdd(&nrec, 1);
+                if (slot < kRecQueue) {
+                    rec[slot] = s;
+                    mine = false;
+                }
+            }
+            __syncthreads();
+            n = nrec;
+            for (int q = 0; q < min(n, kRecQueue); ++q) {
+                const Setup& r = rec[q];
+                raster_rect_slow<RS, kVis>(r, g.x0, g.y0, max(g.x0, r.px0), min(g.x1, r.px1), max(g.y0, r.py0),
+                                           min(g.y1, r.py1), tid, kRasterThreads, tile);
+            }
+        }
+    }
+    __syncthreads();
 }
 
 // The records put aside; then the region is complete.  A record goes to one
@@ -1447,14 +1499,16 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
 // the screen pass reads the maps.  On the 64-sample 1080p frame this took the
 // raster from 0.363 to 0.346 ms, the soft pass that follows from 0.374 to
 // 0.341 ms and the frame from 0.991 to 0.940 ms.
-template <int RS, bool kVis, bool kBig>
-__device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region& g, void* out, int map,
-                                              typename KeyOf<kVis>::T* tile, const Setup* rec, const int& nrec,
+template <int TS, int RS, bool kVis, bool kFallback>
+__device__ __forceinline__ void finish_region(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
+                                              const BinBufs& b, const Region& g, void* out, int map, uint32_t begin,
+                                              uint32_t end, typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec,
                                               ZBound& z, bool by_rows) {
     constexpr int kWaves = kRasterThreads / 64;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __syncthreads();
-    const int nq = min(nrec, kRecQueue);
+    const bool has_long = (nrec & kHasLong) != 0;
+    const int nq = min(nrec & ~kHasLong, kRecQueue);
     if (nq > 0) {  // uniform
         Setup s;
         TileEdges t = {};
@@ -1473,18 +1527,10 @@ __device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region
             blocks = rows & block_mask<RS>(max(g.x0, s.px0) - g.x0, min(g.x1, s.px1) - g.x0,
                                            max(g.y0, s.py0) - g.y0, min(g.y1, s.py1) - g.y0);
         }
-        raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks && (!kBig || t.ok), g.x0, g.y0, lane, z.zmax, z.age, tile);
-        if constexpr (kBig) {
-            unsigned long long slow = __ballot(has && !t.ok);
-            while (slow) {
-                const Setup q = rec[__ffsll((long long)slow) - 1];
-                slow &= slow - 1;
-                raster_rect_slow<RS, kVis>(q, g.x0, g.y0, max(g.x0, q.px0), min(g.x1, q.px1), max(g.y0, q.py0),
-                                           min(g.y1, q.py1), tid, kRasterThreads, tile);
-            }
-        }
+        raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks, g.x0, g.y0, lane, z.zmax, z.age, tile);
         __syncthreads();
     }
+    if (has_long) raster_long<TS, RS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, begin, end, tile, rec, nrec);  // uniform
     constexpr int kPx = RS * RS;
     const size_t plane = (size_t)cfg.w * cfg.h;
     if constexpr (!kVis) {
@@ -1534,7 +1580,7 @@ __device__ __forceinline__ void finish_region(const RasterCfg& cfg, const Region
 // values); no barrier stands between the rounds.  `spread` interleaves them,
 // so that a short list reaches all four waves: for launches that leave the GPU
 // room (kSpreadTiles).
-template <int TS, bool kVis, bool kFallback, bool kBig>
+template <int TS, bool kVis, bool kFallback>
 __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                             const BinBufs& b, void* out, int map, int tile_id,
                                             typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec, bool spread) {
@@ -1586,9 +1632,9 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
         const uint32_t k = base + (uint32_t)(spread ? lane * kWaves + wave : tid);
         const bool has = k < end;
         const uint32_t entry = kFallback ? k : (has ? b.entries[(size_t)map * b.cap + k] : 0u);
-        raster_round<TS, TS, kVis, kFallback, kBig>(mesh, mvps, cfg, b, map, g, entry, has, aside, tile, rec, nrec, z);
+        raster_round<TS, TS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, entry, has, aside, tile, rec, nrec, z);
     }
-    finish_region<TS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z, spread);
+    finish_region<TS, TS, kVis, kFallback>(mesh, mvps, cfg, b, g, out, map, begin, end, tile, rec, nrec, z, spread);
 }
 
 // ---------------------------------------------------------------------------
@@ -1617,7 +1663,7 @@ __device__ __forceinline__ uint32_t* split_list(typename KeyOf<kVis>::T* tile) {
     return reinterpret_cast<uint32_t*>(tile + kSplitEdge * tile_pitch<kSplitEdge>());
 }
 
-template <int TS, bool kVis, bool kBig>
+template <int TS, bool kVis>
 __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                               const BinBufs& b, void* out, int map, int tile_id, int part,
                                               typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec, int& nlist) {
@@ -1668,12 +1714,12 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
         for (int k0 = 0; k0 < n; k0 += kRasterThreads) {
             const int k = k0 + (tid & 63) * kWaves + (tid >> 6);
             const bool has = k < n;
-            raster_round<TS, RS, kVis, false, kBig>(mesh, mvps, cfg, b, map, g, has ? list[k] : 0u, has,
+            raster_round<TS, RS, kVis, false>(mesh, mvps, cfg, b, map, g, has ? list[k] : 0u, has,
                                                     (RS / 8) * (RS / 8), tile, rec, nrec, z);
         }
         __syncthreads();  // nlist and the list are rewritten by the next pass
     }
-    finish_region<RS, kVis, kBig>(cfg, g, out, map, tile, rec, nrec, z, true);
+    finish_region<TS, RS, kVis, false>(mesh, mvps, cfg, b, g, out, map, begin, end, tile, rec, nrec, z, true);
 }
 
 // Binned raster: one workgroup per (tile, map); overflowed maps are left to
@@ -1684,27 +1730,27 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
 // holding only the ground) arrive in runs that pile onto a few CUs while the
 // rest idle.  Tile-major order spreads each costly tile's maps over the XCDs
 // and CUs.
-template <int TS, bool kVis, bool kBig>
-__global__ __launch_bounds__(kRasterThreads, kVis || kBig ? 1 : 8) void k_raster(MeshView mesh, MvpSource mvps,
-                                                                                 RasterCfg cfg, BinBufs b, void* out,
-                                                                                 int map_base, int map_count,
-                                                                                 bool spread) {
+template <int TS, bool kVis>
+__global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 8) void k_raster(MeshView mesh, MvpSource mvps, RasterCfg cfg,
+                                                                         BinBufs b, void* out, int map_base,
+                                                                         int map_count, bool spread) {
     __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec;
     const int map = map_base + (int)(blockIdx.x % (unsigned)map_count);
     const int tile_id = (int)(blockIdx.x / (unsigned)map_count);
     if (b.overflow[map]) return;
-    raster_tile<TS, kVis, false, kBig>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, spread);
+    raster_tile<TS, kVis, false>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, spread);
 }
 
 // k_raster for launches that split long lists: the first workgroups take a
 // (tile, map) each, and of a split tile its first region; kSplitWorkers more
 // take the other regions in turn.
 constexpr int kSplitWorkers = 1024;
-template <int TS, bool kVis, bool kBig>
-__global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, MvpSource mvps, RasterCfg cfg,
-                                                                 BinBufs b, void* out, int map_base, int map_count) {
+template <int TS, bool kVis>
+__global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 6) void k_raster_split(MeshView mesh, MvpSource mvps,
+                                                                               RasterCfg cfg, BinBufs b, void* out,
+                                                                               int map_base, int map_count) {
     __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec, nlist;
@@ -1719,7 +1765,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, 
         if (b.overflow[map]) return;
         const uint32_t* o = b.offsets + (size_t)map * (ntiles + 1) + tile_id;
         if (o[1] - o[0] <= split_tiles(b, map)[1]) {
-            raster_tile<TS, kVis, false, kBig>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, true);
+            raster_tile<TS, kVis, false>(mesh, mvps, cfg, b, out, map, tile_id, tile, rec, nrec, true);
             return;
         }
     } else {
@@ -1741,7 +1787,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, 
             part = 1 + t % (kSplitRegions - 1);
             t += kSplitWorkers;
         }
-        raster_region<TS, kVis, kBig>(mesh, mvps, cfg, b, out, map, tile_id, part, tile, rec, nrec, nlist);
+        raster_region<TS, kVis>(mesh, mvps, cfg, b, out, map, tile_id, part, tile, rec, nrec, nlist);
         if (bid >= 0) return;
         __syncthreads();  // the region's LDS is used again
     }
@@ -1761,7 +1807,7 @@ __global__ __launch_bounds__(kRasterThreads) void k_raster_fallback(MeshView mes
     if (!__syncthreads_or(any)) return;
     for (int map = 0; map < nmaps; ++map) {
         if (!b.overflow[map]) continue;
-        raster_tile<TS, kVis, true, true>(mesh, mvps, cfg, b, out, map, blockIdx.x, tile, rec, nrec, true);
+        raster_tile<TS, kVis, true>(mesh, mvps, cfg, b, out, map, blockIdx.x, tile, rec, nrec, true);
         __syncthreads();
     }
 }

@@ -4,7 +4,7 @@ one fixed FP32 expression, so no tolerance is due)."""
 import numpy as np
 import pytest
 
-from helpers import bits_equal, clip_heavy_mesh, clipped_count, mismatch_report
+from helpers import bits_equal, clip_heavy_mesh, clipped_count, horizon_scene, mismatch_report
 
 pytestmark = pytest.mark.gpu
 
@@ -153,3 +153,49 @@ def test_long_lists_by_launch(gi, oracle_lib, cuda, w, h, n):
     pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
     assert bits_equal(g.position.cpu().numpy(), pos_o)
     assert bits_equal(g.normal.cpu().numpy(), nrm_o)
+
+
+@pytest.mark.parametrize("w,extent,n_long,n_small", [(8191, 1e7, 1, 0), (8191, 1e7, 3, 400), (8191, 1e8, 40, 400),
+                                                     (8170, 1e8, 2, 400)])
+def test_long_edges_of_clipped_triangles(gi, oracle_lib, cuda, w, extent, n_long, n_small):
+    """Clipped vertices rounded to outside the guard band, so that views below
+    8,192 pixels have edges past the 24-bit factors of the 32-bit edge tests:
+    one map and the G-buffer (lists in regions), 65 maps (tiles only); 40 are
+    more than a tile's queue holds."""
+    h = 64
+    mesh, mvp = horizon_scene(n_long, n_small, w, h, extent)
+    dm = gi.DeviceMesh.from_mesh(mesh)
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp, w, h)
+    assert (want < 1.0).mean() > 0.3
+    for maps in (1, 65):
+        got = gi.render_shadow_map(dm, np.tile(mvp.reshape(1, 16), (maps, 1)), w, h).cpu().numpy()
+        for k in range(maps):
+            assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k} of {maps}")
+    g = gi.render_gbuffer(dm, mvp, w, h)
+    pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
+    assert bits_equal(g.position.cpu().numpy(), pos_o), mismatch_report(g.position.cpu().numpy(), pos_o, "position")
+    assert bits_equal(g.normal.cpu().numpy(), nrm_o)
+
+
+@pytest.mark.parametrize("tile", [32, 64])
+@pytest.mark.parametrize("w,extent,n_long", [(8191, 1e7, 3), (8191, 1e8, 40), (8192, 1e8, 3)])
+def test_batch_of_long_edges(gi, oracle_lib, cuda, w, extent, n_long, tile):
+    """The same in a batch, beside a map without long edges."""
+    import torch
+    from globalillumination_amd.batch import Batch, BatchInstance
+
+    insts, want = [], []
+    for width, long in ((w, n_long), (512, 0)):
+        mesh, mvp = horizon_scene(long, 300, width, 64, extent)
+        dm = gi.DeviceMesh.from_mesh(mesh)
+        g = gi.render_gbuffer(dm, mvp, 32, 16)
+        insts.append(BatchInstance(dm, np.stack([mvp, mvp]), width, 64, g, gi.passes.SoftParams()))
+        want.append(oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp, width, 64))
+    b = Batch(insts)
+    b.set_tuning(tile, 4, 3, 4)
+    b.run()
+    torch.cuda.synchronize()
+    for k, (i, d) in enumerate(zip(insts, want)):
+        for m in i.maps.cpu().numpy():
+            assert bits_equal(m, d), mismatch_report(m, d, f"instance {k}")
+    b.close()
