@@ -497,15 +497,18 @@ struct BinBufs {
 // bits 16-17 the box width in tiles minus 1, bits 18-21 which of the box's
 // (at most 4) tiles it overlaps.  Bits 18-21 zero: none (rejected, clipped,
 // wide or empty); bit 31 then marks a clipped triangle, whose place in the
-// clip list fills the other bits (0-17, then 22-30).
+// clip list fills the other bits (0-17, then 22-30).  The counter that gives
+// the places runs past the list's capacity, up to the mesh's triangles; all
+// places past the list are one, the capacity, which fits these 27 bits.
 constexpr uint32_t kClipCode = 0x80000000u;
 __device__ __forceinline__ uint32_t tiles_code(int base, int ntx, uint32_t mask) {
     return mask ? ((uint32_t)base | ((uint32_t)(ntx - 1) << 16) | (mask << 18)) : 0u;
 }
-__device__ __forceinline__ uint32_t clip_code(uint32_t c) {  // c < 2^27 (wide_cap of 2^28 triangles is below 2^25)
+__host__ __device__ constexpr uint32_t clip_code(uint32_t c, uint32_t ccap) {
+    c = c < ccap ? c : ccap;
     return kClipCode | (c & 0x3FFFFu) | ((c >> 18) << 22);
 }
-__device__ __forceinline__ uint32_t clip_place(uint32_t code) {
+__host__ __device__ constexpr uint32_t clip_place(uint32_t code) {
     return (code & 0x3FFFFu) | (((code & ~kClipCode) >> 22) << 18);
 }
 
@@ -596,7 +599,7 @@ __device__ __forceinline__ void bin_body(const MeshView& mesh, const MvpSource& 
                 uint32_t c = atomicAdd(&b.nclip[map], 1u);
                 if (c < b.ccap) b.clip[(size_t)map * b.ccap + c] = (uint32_t)tri;
                 else b.wide_over[map] = 1;
-                code = clip_code(c);
+                code = clip_code(c, b.ccap);
             }
         } else if (ok) {
             int tx0 = t.px0 / TS, tx1 = t.px1 / TS, ty0 = t.py0 / TS, ty1 = t.py1 / TS;
@@ -1958,7 +1961,7 @@ inline uint32_t entry_cap(int ntris, int ntiles, int ts = kTile) {
 // resolve (14 MiB); the resolve clips those past it again.
 constexpr uint32_t kAttrTriangles = 16384u;
 
-inline uint32_t wide_cap(int ntris) { return 1024u + (uint32_t)ntris / 16u; }
+constexpr uint32_t wide_cap(int ntris) { return 1024u + (uint32_t)ntris / 16u; }
 
 inline size_t layout(int ntris, int nmaps, int w, int h, bool vis, Workspace* ws, char* base, int ts = kTile) {
     int tx = (w + ts - 1) / ts, ty = (h + ts - 1) / ts;
