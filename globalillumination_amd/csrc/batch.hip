@@ -142,6 +142,7 @@ __device__ __forceinline__ BinBufs bufs_in_ws(char* ws, const BinBufs& b) {
     g.entries = in_ws(ws, b.entries);
     g.tiles = in_ws(ws, b.tiles);
     g.setups = in_ws(ws, b.setups);
+    g.fars = in_ws(ws, b.fars);
     return g;
 }
 

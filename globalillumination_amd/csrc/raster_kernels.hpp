@@ -346,8 +346,9 @@ __device__ __forceinline__ Setup to_setup(const Tri<NA>& t, uint32_t id) {
 
 // The count pass's record of a directly binned triangle, 32 bytes: the list
 // entry supplies the id, the tie bits and the pixel box follow from the
-// vertices, and vertices 1 and 2 are kept as 16-bit offsets from vertex 0
-// (rec_fits; a triangle with a longer edge becomes a wide record).  The
+// vertices, and vertices 1 and 2 are kept as 16-bit offsets from vertex 0.  A
+// triangle with a vertex 128 pixels or more from vertex 0 (a thin one, or one
+// that leaves the view) keeps them in a FarRec beside the record.  The
 // records are the raster's and the count pass's largest traffic after the
 // maps themselves; with 48 bytes (32-bit coordinates, packed box) 289 maps of
 // a 50,002-triangle mesh took 206 us in the count pass and 450 us in the
@@ -359,9 +360,10 @@ struct alignas(16) SetupRec {
     float z0, A, B, zoff;
 };
 static_assert(sizeof(SetupRec) == 32, "two 16-byte loads");
-// Workspace bytes reserved per directly binned triangle and map.
-constexpr size_t kRecStride = 48;
-static_assert(sizeof(SetupRec) <= kRecStride, "the workspace's record area");
+struct alignas(16) FarRec {
+    int X1, Y1, X2, Y2;
+};
+constexpr uint32_t kFar = 0x80008000u;  // SetupRec::d1 of a record with a FarRec: no 16-bit offsets are these
 
 // Every vertex within 127 pixels of vertex 0.
 __device__ __forceinline__ bool rec_fits(const Tri<0>& t) {
@@ -369,37 +371,53 @@ __device__ __forceinline__ bool rec_fits(const Tri<0>& t) {
     return max(max(abs(dx1), abs(dx2)), max(abs(dy1), abs(dy2))) < 32768;
 }
 
-__device__ __forceinline__ SetupRec to_rec(const Tri<0>& t) {
+__device__ __forceinline__ void store_rec(SetupRec* recs, FarRec* fars, size_t at, const Tri<0>& t) {
     SetupRec r;
     r.X0 = t.X[0];
     r.Y0 = t.Y[0];
     r.d1 = ((uint32_t)(t.X[1] - t.X[0]) & 0xFFFFu) | ((uint32_t)(t.Y[1] - t.Y[0]) << 16);
     r.d2 = ((uint32_t)(t.X[2] - t.X[0]) & 0xFFFFu) | ((uint32_t)(t.Y[2] - t.Y[0]) << 16);
     r.z0 = t.z0; r.A = t.A; r.B = t.B; r.zoff = t.zoff;
-    return r;
+    if (!rec_fits(t)) {
+        r.d1 = kFar;
+        fars[at] = FarRec{t.X[1], t.Y[1], t.X[2], t.Y[2]};
+    }
+    recs[at] = r;
+}
+
+// A record's vertices, from its first 16 bytes.
+__device__ __forceinline__ void rec_vertices(int X0, int Y0, uint32_t d1, uint32_t d2, const FarRec& far, int X[3],
+                                             int Y[3]) {
+    X[0] = X0;
+    Y[0] = Y0;
+    X[1] = X0 + (int)(int16_t)(d1 & 0xFFFFu);
+    Y[1] = Y0 + ((int)d1 >> 16);
+    X[2] = X0 + (int)(int16_t)(d2 & 0xFFFFu);
+    Y[2] = Y0 + ((int)d2 >> 16);
+    if (d1 == kFar) {
+        const FarRec f = far;
+        X[1] = f.X1;
+        Y[1] = f.Y1;
+        X[2] = f.X2;
+        Y[2] = f.Y2;
+    }
 }
 
 // Pixel-centre box of a record's vertices, not yet clamped to the view.
-__device__ __forceinline__ void rec_box(int X0, int Y0, uint32_t d1, uint32_t d2, int& px0, int& px1, int& py0,
-                                        int& py1) {
-    const int x1 = (int)(int16_t)(d1 & 0xFFFFu), x2 = (int)(int16_t)(d2 & 0xFFFFu);
-    const int y1 = (int)d1 >> 16, y2 = (int)d2 >> 16;
-    px0 = (X0 + min(0, min(x1, x2)) + 127) >> 8;
-    px1 = (X0 + max(0, max(x1, x2)) - 128) >> 8;
-    py0 = (Y0 + min(0, min(y1, y2)) + 127) >> 8;
-    py1 = (Y0 + max(0, max(y1, y2)) - 128) >> 8;
+__device__ __forceinline__ void rec_box(const int X[3], const int Y[3], int& px0, int& px1, int& py0, int& py1) {
+    px0 = (min(X[0], min(X[1], X[2])) + 127) >> 8;
+    px1 = (max(X[0], max(X[1], X[2])) - 128) >> 8;
+    py0 = (min(Y[0], min(Y[1], Y[2])) + 127) >> 8;
+    py1 = (max(Y[0], max(Y[1], Y[2])) - 128) >> 8;
 }
 
-// Same box and tie rules as setup_piece, on the same 24.8 coordinates.
-__device__ __forceinline__ Setup from_rec(const SetupRec& r, uint32_t id, const RasterCfg& cfg) {
+// Same box and tie rules as setup_piece, on the same 24.8 coordinates.  Never a
+// long edge: the triangle was not clipped, so it reaches at most 1.5 views past
+// the view (24,576 pixels), and at most four tiles into it.
+__device__ __forceinline__ Setup from_rec(const SetupRec& r, const FarRec& far, uint32_t id, const RasterCfg& cfg) {
     Setup s;
-    s.X[0] = r.X0;
-    s.Y[0] = r.Y0;
-    s.X[1] = r.X0 + (int)(int16_t)(r.d1 & 0xFFFFu);
-    s.Y[1] = r.Y0 + ((int)r.d1 >> 16);
-    s.X[2] = r.X0 + (int)(int16_t)(r.d2 & 0xFFFFu);
-    s.Y[2] = r.Y0 + ((int)r.d2 >> 16);
-    rec_box(r.X0, r.Y0, r.d1, r.d2, s.px0, s.px1, s.py0, s.py1);
+    rec_vertices(r.X0, r.Y0, r.d1, r.d2, far, s.X, s.Y);
+    rec_box(s.X, s.Y, s.px0, s.px1, s.py0, s.py1);
     s.px0 = max(s.px0, 0);
     s.px1 = min(s.px1, cfg.w - 1);
     s.py0 = max(s.py0, 0);
@@ -488,6 +506,7 @@ struct BinBufs {
     uint32_t* entries;   // nmaps x cap
     uint32_t* tiles;     // nmaps x tstride: the count pass's tiles of each directly binned triangle
     SetupRec* setups;    // nmaps x tstride: its setup record (64-texel tiles only)
+    FarRec* fars;        // nmaps x tstride: and its vertices 1 and 2, where the record cannot hold them
     ResolveRec* attrs;   // G-buffer pass only (one map): acap x kMaxPieces, the clipped pieces' attributes
     uint32_t cap, wcap, ccap, tstride, acap;
 };
@@ -605,7 +624,7 @@ __device__ __forceinline__ void bin_body(const MeshView& mesh, const MvpSource& 
             int tx0 = t.px0 / TS, tx1 = t.px1 / TS, ty0 = t.py0 / TS, ty1 = t.py1 / TS;
             int ntx = tx1 - tx0 + 1;
             int span = ntx * (ty1 - ty0 + 1);
-            if (span > kWideSpan || (kCache && !rec_fits(t))) {
+            if (span > kWideSpan) {
                 if (!kScatter) push_record(b, map, t, entry);
             } else {
                 uint32_t mask = 0;
@@ -622,7 +641,7 @@ __device__ __forceinline__ void bin_body(const MeshView& mesh, const MvpSource& 
                     mask |= 1u << k;
                 }
                 code = tiles_code(ty0 * cfg.tiles_x + tx0, ntx, mask);
-                if (!kScatter && kCache && mask) b.setups[(size_t)map * b.tstride + tri] = to_rec(t);
+                if (!kScatter && kCache && mask) store_rec(b.setups, b.fars, (size_t)map * b.tstride + tri, t);
             }
         }
         if (!kScatter && kCache) b.tiles[(size_t)map * b.tstride + tri] = code;
@@ -1397,7 +1416,8 @@ __device__ __forceinline__ void load_setup(const MeshView& mesh, const MvpSource
         s = b.wide[(size_t)map * b.wcap + (entry & ~kWideBit)];
     } else if constexpr (!kFallback && wide_span<TS>() <= 4) {
         // a directly binned triangle: the count pass stored its setup
-        s = from_rec(b.setups[(size_t)map * b.tstride + (entry >> 3)], entry, cfg);
+        const size_t at = (size_t)map * b.tstride + (entry >> 3);
+        s = from_rec(b.setups[at], b.fars[at], entry, cfg);
     } else {
         float mvp[16];
         mvps.load(map, mvp);
@@ -1704,8 +1724,11 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
                 py0 = w.py0;
                 py1 = w.py1;
             } else {
-                const SetupRec& r = b.setups[(size_t)map * b.tstride + (e[q] >> 3)];
-                rec_box(r.X0, r.Y0, r.d1, r.d2, px0, px1, py0, py1);
+                const size_t at = (size_t)map * b.tstride + (e[q] >> 3);
+                const SetupRec& r = b.setups[at];
+                int X[3], Y[3];
+                rec_vertices(r.X0, r.Y0, r.d1, r.d2, b.fars[at], X, Y);
+                rec_box(X, Y, px0, px1, py0, py1);
             }
             hit[q] = px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0;
         }
@@ -1983,8 +2006,10 @@ inline size_t layout(int ntris, int nmaps, int w, int h, bool vis, Workspace* ws
     size_t o_entries = off; off = align256(off + sizeof(uint32_t) * (size_t)cap * nmaps);
     size_t o_tiles = off; off = align256(off + sizeof(uint32_t) * (size_t)(ntris > 0 ? ntris : 0) * nmaps);
     const bool records = 4 * (64 / ts) * (64 / ts) <= 4;  // the tile code's span (wide_span<ts>() <= 4)
+    const size_t nrecs = records ? (size_t)(ntris > 0 ? ntris : 0) * nmaps : 0;
     size_t o_setups = off;
-    if (records) off = align256(off + kRecStride * (size_t)(ntris > 0 ? ntris : 0) * nmaps);
+    size_t o_fars = off + sizeof(SetupRec) * nrecs;
+    off = align256(o_fars + sizeof(FarRec) * nrecs);
     // the G-buffer pass (one map): visibility keys and the clipped pieces' attributes
     const uint32_t acap = vis ? std::min(ccap, kAttrTriangles) : 0u;
     size_t o_vis = off;
@@ -2004,6 +2029,7 @@ inline size_t layout(int ntris, int nmaps, int w, int h, bool vis, Workspace* ws
         b.entries = reinterpret_cast<uint32_t*>(base + o_entries);
         b.tiles = reinterpret_cast<uint32_t*>(base + o_tiles);
         b.setups = records ? reinterpret_cast<SetupRec*>(base + o_setups) : nullptr;
+        b.fars = records ? reinterpret_cast<FarRec*>(base + o_fars) : nullptr;
         b.tstride = (uint32_t)(ntris > 0 ? ntris : 0);
         b.cap = cap;
         b.wcap = wcap;

@@ -4,7 +4,7 @@ one fixed FP32 expression, so no tolerance is due)."""
 import numpy as np
 import pytest
 
-from helpers import bits_equal, clip_heavy_mesh, clipped_count, horizon_scene, mismatch_report
+from helpers import bits_equal, clip_heavy_mesh, clipped_count, fence_mesh, horizon_scene, mismatch_report
 
 pytestmark = pytest.mark.gpu
 
@@ -199,3 +199,40 @@ def test_batch_of_long_edges(gi, oracle_lib, cuda, w, extent, n_long, tile):
         for m in i.maps.cpu().numpy():
             assert bits_equal(m, d), mismatch_report(m, d, f"instance {k}")
     b.close()
+
+
+def binning_counters(ws, w, h, maps):
+    """(wide records, whether they were too many) of every map, from the
+    workspace: the tile counts, then both, each area a multiple of 256 bytes."""
+    words = ws.view(np.int32) if isinstance(ws, np.ndarray) else ws.cpu().numpy().view(np.int32)
+    step = lambda n: (4 * n + 255) // 256 * 64
+    at = step(((w + 63) // 64) * ((h + 63) // 64) * maps)
+    return words[at:at + maps], words[at + step(maps):at + step(maps) + maps]
+
+
+@pytest.mark.parametrize("w,h,n,length,thick,maps", [(512, 512, 4000, 150.0, 2.0, 1), (640, 384, 3000, 185.0, 1.0, 20),
+                                                     (1024, 768, 6000, 129.0, 6.0, 1), (128, 128, 4000, 230.0, 3.0, 1),
+                                                     (65, 64, 3000, 140.0, 20.0, 70), (4096, 64, 4000, 140.0, 2.0, 1)])
+def test_many_long_thin_triangles(gi, oracle_lib, cuda, w, h, n, length, thick, maps):
+    """Triangles with a vertex more than 127 pixels from their first one, in at
+    most four tiles, more of them than the wide records' 1,024 + n / 16: they
+    are binned directly, whatever their length.  Small views, which every such
+    triangle leaves, included."""
+    mesh = fence_mesh(n, w, h, length, thick)
+    assert clipped_count(mesh, np.eye(4)) < 100  # fan pieces of clipped triangles are wide records
+    mvps = np.tile(np.eye(4, dtype=np.float32).reshape(1, 16), (maps, 1))
+    dm = gi.DeviceMesh.from_mesh(mesh)
+    p = gi.passes.SplitDepthPass(dm, mvps, w, h)
+    p.bin()
+    nwide, over = binning_counters(p.ws, w, h, maps)
+    assert not over.any() and nwide.max() <= 1024 + n // 16, (nwide, over)
+    p.raster(0, maps)
+    got = p.out.cpu().numpy()
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvps[0], w, h)
+    for k in range(maps):
+        assert bits_equal(got[k], want), mismatch_report(got[k], want, f"map {k}")
+    assert (want < 1.0).mean() > 0.15
+    g = gi.render_gbuffer(dm, mvps[0], w, h)
+    pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvps[0], w, h)
+    assert bits_equal(g.position.cpu().numpy(), pos_o)
+    assert bits_equal(g.normal.cpu().numpy(), nrm_o)
