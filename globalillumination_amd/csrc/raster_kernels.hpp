@@ -1432,9 +1432,10 @@ __device__ __forceinline__ void load_setup(const MeshView& mesh, const MvpSource
 
 // One round of list entries, one per lane (`has`: the lane has one).  Small
 // records are rasterized by their lane, larger ones by the wave in 8x8
-// blocks, those of more than `aside` blocks are put aside in `rec`; one with a
-// long edge leaves its flag in nrec (raster_long).
-constexpr int kHasLong = (int)0x80000000u;
+// blocks, those of more than `aside` blocks and those with a long edge are put
+// aside in `rec`; a long one that finds it full leaves a flag in nrec
+// (raster_long).
+constexpr int kMoreLong = (int)0x80000000u;
 template <int TS, int RS, bool kVis, bool kFallback>
 __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                              const BinBufs& b, int map, const Region& g, uint32_t entry, bool has,
@@ -1458,13 +1459,13 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
         t = tile_edges(s, g.x0, g.y0);
         blocks = block_mask<RS>(rx0 - g.x0, rx1 - g.x0, ry0 - g.y0, ry1 - g.y0);
         area = (rx1 - rx0 + 1) * (ry1 - ry0 + 1);
-        if (s.tl & kLongEdge) {
-            atomicOr(&nrec, kHasLong);
-            has = false;
-        } else if (__popcll(blocks) > aside) {
-            const int slot = atomicAdd(&nrec, 1) & ~kHasLong;
+        if ((s.tl & kLongEdge) || __popcll(blocks) > aside) {
+            const int slot = atomicAdd(&nrec, 1) & ~kMoreLong;
             if (slot < kRecQueue) {
                 rec[slot] = s;
+                has = false;
+            } else if (s.tl & kLongEdge) {
+                atomicOr(&nrec, kMoreLong);
                 has = false;
             }
         }
@@ -1475,9 +1476,22 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
     if (self) raster_rect_self<RS, kVis>(s, t, g.x0, g.y0, rx0, rx1, ry0, ry1, tile);
 }
 
-// The records with a long edge among entries [begin, end), every record by the
-// whole workgroup with the 64-bit edge functions.  Walking the list again here
-// keeps those functions' registers out of raster_round.
+// The records with a long edge among the n of the queue, each by the whole
+// workgroup with the 64-bit edge functions.
+template <int RS, bool kVis>
+__device__ __forceinline__ void raster_queued_long(const Region& g, const Setup* rec, int n,
+                                                   typename KeyOf<kVis>::T* tile) {
+    for (int q = 0; q < n; ++q) {
+        if (!(rec[q].tl & kLongEdge)) continue;  // uniform
+        const Setup r = rec[q];
+        raster_rect_slow<RS, kVis>(r, g.x0, g.y0, max(g.x0, r.px0), min(g.x1, r.px1), max(g.y0, r.py0),
+                                   min(g.y1, r.py1), (int)threadIdx.x, kRasterThreads, tile);
+    }
+}
+
+// All records with a long edge among entries [begin, end), where the queue
+// could not hold them.  Walking the list again keeps the 64-bit edge functions'
+// registers out of raster_round.
 template <int TS, int RS, bool kVis, bool kFallback>
 __device__ __forceinline__ void raster_long(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
                                             const BinBufs& b, int map, const Region& g, uint32_t begin, uint32_t end,
@@ -1503,11 +1517,7 @@ __device__ __forceinline__ void raster_long(const MeshView& mesh, const MvpSourc
             }
             __syncthreads();
             n = nrec;
-            for (int q = 0; q < min(n, kRecQueue); ++q) {
-                const Setup& r = rec[q];
-                raster_rect_slow<RS, kVis>(r, g.x0, g.y0, max(g.x0, r.px0), min(g.x1, r.px1), max(g.y0, r.py0),
-                                           min(g.y1, r.py1), tid, kRasterThreads, tile);
-            }
+            raster_queued_long<RS, kVis>(g, rec, min(n, kRecQueue), tile);
         }
     }
     __syncthreads();
@@ -1530,8 +1540,8 @@ __device__ __forceinline__ void finish_region(const MeshView& mesh, const MvpSou
     constexpr int kWaves = kRasterThreads / 64;
     const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
     __syncthreads();
-    const bool has_long = (nrec & kHasLong) != 0;
-    const int nq = min(nrec & ~kHasLong, kRecQueue);
+    const bool more_long = (nrec & kMoreLong) != 0;
+    const int nq = min(nrec & ~kMoreLong, kRecQueue);
     if (nq > 0) {  // uniform
         Setup s;
         TileEdges t = {};
@@ -1550,10 +1560,11 @@ __device__ __forceinline__ void finish_region(const MeshView& mesh, const MvpSou
             blocks = rows & block_mask<RS>(max(g.x0, s.px0) - g.x0, min(g.x1, s.px1) - g.x0,
                                            max(g.y0, s.py0) - g.y0, min(g.y1, s.py1) - g.y0);
         }
-        raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks, g.x0, g.y0, lane, z.zmax, z.age, tile);
+        raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks && !(s.tl & kLongEdge), g.x0, g.y0, lane, z.zmax, z.age, tile);
+        raster_queued_long<RS, kVis>(g, rec, nq, tile);
         __syncthreads();
     }
-    if (has_long) raster_long<TS, RS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, begin, end, tile, rec, nrec);  // uniform
+    if (more_long) raster_long<TS, RS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, begin, end, tile, rec, nrec);  // uniform
     constexpr int kPx = RS * RS;
     const size_t plane = (size_t)cfg.w * cfg.h;
     if constexpr (!kVis) {

@@ -156,12 +156,13 @@ def test_long_lists_by_launch(gi, oracle_lib, cuda, w, h, n):
 
 
 @pytest.mark.parametrize("w,extent,n_long,n_small", [(8191, 1e7, 1, 0), (8191, 1e7, 3, 400), (8191, 1e8, 40, 400),
-                                                     (8170, 1e8, 2, 400)])
+                                                     (8191, 1e8, 40, 4000), (8170, 1e8, 2, 400)])
 def test_long_edges_of_clipped_triangles(gi, oracle_lib, cuda, w, extent, n_long, n_small):
     """Clipped vertices rounded to outside the guard band, so that views below
     8,192 pixels have edges past the 24-bit factors of the 32-bit edge tests:
-    one map and the G-buffer (lists in regions), 65 maps (tiles only); 40 are
-    more than a tile's queue holds."""
+    one map and the G-buffer (lists in regions), 65 maps (tiles only).  40 are
+    more than a tile's queue holds; with few other triangles their lists exceed
+    the workspace, too, and the fallback rasterizes them."""
     h = 64
     mesh, mvp = horizon_scene(n_long, n_small, w, h, extent)
     dm = gi.DeviceMesh.from_mesh(mesh)
