@@ -1407,6 +1407,30 @@ struct ZBound {
     int age;
 };
 
+// Walk of the fallback, which has no list: the first pieces of 256 triangles,
+// then their second ones, and so on, so that a round's lanes have work together
+// (a piece per lane of triangles in turn leaves seven lanes of eight idle).
+__device__ __forceinline__ uint32_t fallback_length(const MeshView& mesh) {
+    return (uint32_t)(mesh.nt + 255) / 256u * 2048u;
+}
+__device__ __forceinline__ uint32_t fallback_entry(uint32_t k) {
+    return ((k / 2048u * 256u + k % 256u) << 3) | (k / 256u % 8u);
+}
+
+// Entry k of a tile's list; `has` is false past its end.
+template <bool kFallback>
+__device__ __forceinline__ uint32_t list_entry(const MeshView& mesh, const BinBufs& b, int map, uint32_t k,
+                                               uint32_t end, bool& has) {
+    has = k < end;
+    if constexpr (kFallback) {
+        const uint32_t e = fallback_entry(k);
+        has = has && (e >> 3) < (uint32_t)mesh.nt;
+        return e;
+    } else {
+        return has ? b.entries[(size_t)map * b.cap + k] : 0u;
+    }
+}
+
 // The setup record of a list entry; `has` becomes false for an empty piece.
 template <int TS, bool kFallback>
 __device__ __forceinline__ void load_setup(const MeshView& mesh, const MvpSource& mvps, const RasterCfg& cfg,
@@ -1498,10 +1522,9 @@ __device__ __forceinline__ void raster_long(const MeshView& mesh, const MvpSourc
                                             typename KeyOf<kVis>::T* tile, Setup* rec, int& nrec) {
     const int tid = (int)threadIdx.x;
     for (uint32_t base = begin; base < end; base += kRasterThreads) {
-        const uint32_t k = base + (uint32_t)tid;
-        bool mine = k < end;
+        bool mine;
         Setup s;
-        const uint32_t entry = kFallback ? k : (mine ? b.entries[(size_t)map * b.cap + k] : 0u);
+        const uint32_t entry = list_entry<kFallback>(mesh, b, map, base + (uint32_t)tid, end, mine);
         load_setup<TS, kFallback>(mesh, mvps, cfg, b, map, entry, mine, s);
         mine = mine && (s.tl & kLongEdge) && s.px0 <= g.x1 && s.px1 >= g.x0 && s.py0 <= g.y1 && s.py1 >= g.y0;
         for (int n = kRecQueue + 1; n > kRecQueue;) {  // until the queue held all that were left
@@ -1627,7 +1650,7 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
         begin = b.offsets[(size_t)map * (ntiles + 1) + tile_id];
         end = b.offsets[(size_t)map * (ntiles + 1) + tile_id + 1];
     } else {
-        end = (uint32_t)mesh.nt * 8u;
+        end = fallback_length(mesh);
     }
     if constexpr (!kFallback && !kVis) {
         // A whole tile whose list is one wide record covering every pixel
@@ -1663,9 +1686,9 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
     const int aside = end - begin <= (uint32_t)kShareList ? kShareBlocks : kShareBlocksLong;
     ZBound z{0xFFFFFFFFu, 0};
     for (uint32_t base = begin; base < end; base += kRasterThreads) {
-        const uint32_t k = base + (uint32_t)(spread ? lane * kWaves + wave : tid);
-        const bool has = k < end;
-        const uint32_t entry = kFallback ? k : (has ? b.entries[(size_t)map * b.cap + k] : 0u);
+        bool has;
+        const uint32_t entry =
+            list_entry<kFallback>(mesh, b, map, base + (uint32_t)(spread ? lane * kWaves + wave : tid), end, has);
         raster_round<TS, TS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, entry, has, aside, tile, rec, nrec, z);
     }
     finish_region<TS, TS, kVis, kFallback>(mesh, mvps, cfg, b, g, out, map, begin, end, tile, rec, nrec, z, spread);

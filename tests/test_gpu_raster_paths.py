@@ -203,12 +203,12 @@ def test_batch_of_long_edges(gi, oracle_lib, cuda, w, extent, n_long, tile):
 
 
 def binning_counters(ws, w, h, maps):
-    """(wide records, whether they were too many) of every map, from the
-    workspace: the tile counts, then both, each area a multiple of 256 bytes."""
-    words = ws.view(np.int32) if isinstance(ws, np.ndarray) else ws.cpu().numpy().view(np.int32)
-    step = lambda n: (4 * n + 255) // 256 * 64
-    at = step(((w + 63) // 64) * ((h + 63) // 64) * maps)
-    return words[at:at + maps], words[at + step(maps):at + step(maps) + maps]
+    """(wide records, whether the lists or records were too many) of every map,
+    from the workspace: tile counts, wide records, wide records too many, clipped
+    triangles, list offsets, too many; each area a multiple of 256 bytes."""
+    words, tiles = ws.cpu().numpy().view(np.int32), ((w + 63) // 64) * ((h + 63) // 64)
+    at = np.cumsum([(4 * n + 255) // 256 * 64 for n in (tiles * maps, maps, maps, maps, (tiles + 1) * maps)])
+    return words[at[0]:at[0] + maps], words[at[4]:at[4] + maps]
 
 
 @pytest.mark.parametrize("w,h,n,length,thick,maps", [(512, 512, 4000, 150.0, 2.0, 1), (640, 384, 3000, 185.0, 1.0, 20),
@@ -235,5 +235,32 @@ def test_many_long_thin_triangles(gi, oracle_lib, cuda, w, h, n, length, thick, 
     assert (want < 1.0).mean() > 0.15
     g = gi.render_gbuffer(dm, mvps[0], w, h)
     pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvps[0], w, h)
+    assert bits_equal(g.position.cpu().numpy(), pos_o)
+    assert bits_equal(g.normal.cpu().numpy(), nrm_o)
+
+
+@pytest.mark.parametrize("n", [130, 255, 256, 257, 600, 2049])
+def test_fallback_by_triangle_count(gi, oracle_lib, cuda, n):
+    """Maps whose lists exceed the workspace, with triangles cut into several
+    pieces, around the 256 triangles whose pieces the fallback walks together."""
+    rng = np.random.default_rng(300 + n)
+    w, h = 1000, 800
+    pos = rng.uniform(-30, 30, size=(n, 3, 3)).astype(np.float32)
+    pos[:, :, 1] = rng.uniform(0.0, 60.0, size=(n, 3))
+    pos[-1] = [[-40, 30, -40], [40, 30, -40], [0, 47, 60]]
+    nrm = rng.normal(size=(3 * n, 3)).astype(np.float32)
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3), nrm, np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    view = gi.scenes.View((0.0, 50.0, 0.1), (0.0, 0.0, 0.0), w, h, fov=90.0)
+    mvp = gi.passes.view_matrices(view)[2]
+    assert clipped_count(mesh, mvp) > n // 4
+    dm = gi.DeviceMesh.from_mesh(mesh)
+    p = gi.passes.SplitDepthPass(dm, mvp.reshape(1, 16), w, h)
+    p.bin()
+    assert binning_counters(p.ws, w, h, 1)[1][0] == 1
+    got = p.out.cpu().numpy()[0]  # bin rasterizes the maps that fell back
+    want = oracle_lib.depth_raster(mesh.positions, mesh.indices, mvp, w, h)
+    assert bits_equal(got, want), mismatch_report(got, want, "depth")
+    g = gi.render_gbuffer(dm, mvp, w, h)
+    pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
     assert bits_equal(g.position.cpu().numpy(), pos_o)
     assert bits_equal(g.normal.cpu().numpy(), nrm_o)
