@@ -55,13 +55,20 @@ def _upload(arr: np.ndarray, device, stream=None) -> torch.Tensor:
     copy from pageable memory does: a frame that uploads its light matrix
     began only when the frame before it had ended; a 1080p PCSS frame took
     190 us so and takes 173 us).
-    The copy is ordered on torch's current stream: a pass on another stream or
-    device, and a capture, take the waiting copy."""
+    A pass on another stream than torch's current one has its copy allocated
+    and made on that stream: the tensor is dropped when the call returns, and
+    its memory then goes only to work behind the pass.  A capture and a pass on
+    another device take the waiting copy."""
     t = torch.from_numpy(arr)
     dev = torch.device(device)
-    if dev.type != "cuda" or (dev.index is not None and dev.index != torch.cuda.current_device()) or \
-            (stream is not None and stream != torch.cuda.current_stream()) or \
-            torch.cuda.is_current_stream_capturing():
+    if dev.type != "cuda":
+        return t.to(device)
+    if stream is not None and stream != torch.cuda.current_stream():
+        with torch.cuda.stream(stream):
+            if not torch.cuda.is_current_stream_capturing():
+                return _upload(arr, device)
+        return t.to(device)
+    if dev.index not in (None, torch.cuda.current_device()) or torch.cuda.is_current_stream_capturing():
         return t.to(device)
     pinned = torch.empty(t.shape, dtype=t.dtype, pin_memory=True)  # torch reuses it once the copy is done
     pinned.copy_(t)

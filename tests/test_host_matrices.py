@@ -76,3 +76,38 @@ def test_host_matrices_may_change_after_the_call(gi, cuda, side_stream):
     torch.cuda.synchronize()
     for o in outs:
         assert torch.equal(o.view(torch.int32), want.view(torch.int32))
+
+
+@pytest.mark.gpu
+def test_uploads_of_calls_on_another_stream(gi, cuda):
+    """Passes on a stream that is not torch's current one, several in a row
+    with other matrices each, behind work that is still running there: each
+    reads its own, though the tensors of the calls before have been dropped."""
+    import torch
+
+    wl = gi.scenes.config3(nsamples=4, view_w=64, view_h=64, sm=256, freq=20)
+    dm = gi.DeviceMesh.from_mesh(wl.mesh)
+    mvps = np.stack([passes.view_matrices(v)[2] for v in wl.lights])
+    frames = [np.roll(mvps, k, axis=0) * np.float32(1.0 + 0.05 * k) for k in range(4)]
+    g = gi.render_gbuffer(dm, passes.view_matrices(wl.camera)[2], 64, 64)
+    soft = passes.SoftParams()
+    want = []
+    for k, m in enumerate(frames):
+        maps = gi.render_shadow_map(dm, torch.from_numpy(m).cuda(), 256, 256)
+        trans = torch.from_numpy(passes.soft_uniforms(m, 0.01 * k)[1]).cuda()
+        want.append((maps, gi.render_monte_carlo(g, maps, m, soft, zbias=0.01 * k, trans_dev=trans)))
+    assert not torch.equal(want[0][0], want[1][0])
+    outs = [(torch.empty_like(m), torch.empty_like(s)) for m, s in want]
+    a = torch.randn(4096, 4096, device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for _ in range(20):
+            a = a @ a * 1e-3
+    for k, (m, (maps, out)) in enumerate(zip(frames, outs)):
+        gi.render_shadow_map(dm, m, 256, 256, out=maps, stream=stream)
+        gi.render_monte_carlo(g, maps, m, soft, zbias=0.01 * k, out=out, stream=stream)
+    stream.synchronize()
+    for (maps, out), (wm, wo) in zip(outs, want):
+        assert torch.equal(maps.view(torch.int32), wm.view(torch.int32))
+        assert torch.equal(out.view(torch.int32), wo.view(torch.int32))
