@@ -3,7 +3,7 @@ import numpy as np
 import pytest
 
 from globalillumination_amd import camera, passes
-from globalillumination_amd.diff import AreaLight, _dot, _normalize, perspective64
+from globalillumination_amd.diff import AreaLight, _dot, _normalize, lookat64, perspective64
 
 
 @pytest.mark.parametrize("n,zbias", [(1, 0.0), (2, 0.005), (64, -0.25), (289, 0.0)])
@@ -111,3 +111,31 @@ def test_uploads_of_calls_on_another_stream(gi, cuda):
     for (maps, out), (wm, wo) in zip(outs, want):
         assert torch.equal(maps.view(torch.int32), wm.view(torch.int32))
         assert torch.equal(out.view(torch.int32), wo.view(torch.int32))
+
+
+@pytest.mark.parametrize("r", [0.25, np.float32(0.25), np.array(0.25), np.array([0.25]), np.array([0.25, 0.5, 2.0])])
+def test_area_light_radius_forms(r):
+    """The radius may be one number or one per axis, as an array too: (N, 4, 4)
+    matrices, each that of the light moved by r * (ox, oy, 0)."""
+    light = AreaLight((0.1, -0.2, 0.3), np.array([[0.5, -0.25], [-1.0, 0.75]]), 64)
+    L = np.array([3.0, 7.0, 2.0])
+    got = light.matrices(L, r)
+    assert got.shape == (2, 4, 4)
+    for m, (ox, oy) in zip(got, light.offsets):
+        d = r * np.array([ox, oy, 0.0])
+        still = AreaLight(tuple(np.asarray(light.at) + d), np.zeros((1, 2)), 64)
+        assert (m == still.matrices(L + d, 0.0)[0]).all()
+
+
+@pytest.mark.parametrize("L,r", [(np.ones(3), np.ones(2)), (np.ones(3), np.ones((2, 3))), (np.ones(3), np.ones((2, 1))),
+                                 (np.ones((1, 3)), 0.5), (np.ones(2), 0.5)])
+def test_area_light_refuses_other_shapes(L, r):
+    with pytest.raises(ValueError):
+        AreaLight((0.1, -0.2, 0.3), np.array([[0.5, -0.25], [-1.0, 0.75]]), 64).matrices(L, r)
+
+
+def test_area_light_and_views_refuse_other_counts():
+    with pytest.raises(ValueError):
+        AreaLight((0.1, -0.2, 0.3), np.zeros((0, 2)), 64).matrices(np.ones(3), 0.5)
+    with pytest.raises(ValueError):
+        lookat64(np.ones((2, 3)), np.zeros((2, 3)), (0.0, 0.0, 1.0))
