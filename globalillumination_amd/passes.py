@@ -477,6 +477,8 @@ def soft_uniforms(light_mvps: np.ndarray, zbias: float = 0.0):
     (SoftShadowMapping/src/Viewers/MyGLGeometryViewer.cpp:168-195): columns 0-2
     of the LAST sample's biased matrix, column 3 of every sample's."""
     m = np.ascontiguousarray(light_mvps, dtype=np.float32).reshape(-1, 16)
+    if len(m) == 0:
+        raise ValueError("at least one light matrix is required")
     b = biased_samples(m, zbias)
     return b[-1].copy(), camera.soft_light_trans(b)
 

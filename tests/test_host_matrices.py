@@ -139,3 +139,9 @@ def test_area_light_and_views_refuse_other_counts():
         AreaLight((0.1, -0.2, 0.3), np.zeros((0, 2)), 64).matrices(np.ones(3), 0.5)
     with pytest.raises(ValueError):
         lookat64(np.ones((2, 3)), np.zeros((2, 3)), (0.0, 0.0, 1.0))
+
+
+def test_no_light_matrices_are_refused():
+    for f in (passes.soft_uniforms, lambda m: passes.adaptive_trans(m, [])):
+        with pytest.raises(ValueError):
+            f(np.zeros((0, 16), np.float32))
