@@ -264,3 +264,32 @@ def test_fallback_by_triangle_count(gi, oracle_lib, cuda, n):
     pos_o, nrm_o, _ = oracle_lib.gbuffer(mesh.positions, mesh.normals, mesh.indices, mvp, w, h)
     assert bits_equal(g.position.cpu().numpy(), pos_o)
     assert bits_equal(g.normal.cpu().numpy(), nrm_o)
+
+
+@pytest.mark.parametrize("w,h,maps,ranges", [(512, 512, 5, [(0, 2), (2, 2), (4, 1)]), (2048, 128, 64, [(63, 1), (0, 40), (40, 23)]),
+                                             (512, 512, 66, [(0, 1), (1, 64), (65, 1)])])
+def test_ranges_of_maps_with_long_lists(gi, oracle_lib, cuda, w, h, maps, ranges):
+    """The raster of a range of maps at a time, of launches that split long
+    lists (up to 64 maps) and that do not; every map has crowded tiles of its
+    own, and what a range does not cover is left as it was."""
+    rng = np.random.default_rng(maps)
+    n = 4000
+    cen = rng.uniform(-1.0, 1.0, size=(n, 1, 3)) * [100.0 / w, 50.0 / h, 0.9]
+    pos = (cen + rng.uniform(-1.0, 1.0, size=(n, 3, 3)) * [12.0 / w, 12.0 / h, 0.05]).astype(np.float32)
+    mesh = gi.scenes.Mesh(pos.reshape(-1, 3), np.zeros((3 * n, 3), np.float32), np.arange(3 * n, dtype=np.int32).reshape(n, 3))
+    mvps = np.tile(np.eye(4, dtype=np.float32).reshape(1, 16), (maps, 1))
+    mvps[:, 12] = np.arange(maps) % 3 * 0.25 - 0.3  # the crowd's place differs between maps
+    p = gi.passes.SplitDepthPass(gi.DeviceMesh.from_mesh(mesh), mvps, w, h)
+    p.bin()
+    p.out.fill_(-1.0)
+    want = [oracle_lib.depth_raster(mesh.positions, mesh.indices, mvps[k], w, h) for k in range(3)]
+    done = np.zeros(maps, bool)
+    for first, count in ranges:
+        p.raster(first, count)
+        done[first:first + count] = True
+        got = p.out.cpu().numpy()
+        for k in range(maps):
+            if done[k]:
+                assert bits_equal(got[k], want[k % 3]), mismatch_report(got[k], want[k % 3], f"map {k}")
+            else:
+                assert (got[k] == -1.0).all(), k
