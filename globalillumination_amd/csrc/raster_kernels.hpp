@@ -27,7 +27,7 @@ constexpr int kMaxPoly = 9;
 // 28 setup records (64 B each) beside the 18 KiB tile and the record count
 // keep a workgroup's LDS at 20,228 bytes, so 8 workgroups fit in a CU's
 // 160 KiB (7 of 20,484 bytes ran 3% slower).
-constexpr int kRecQueue = 28;  // LDS setup records that a workgroup puts aside
+constexpr int kRecQueue = 28;  // at most 31; LDS setup records that a workgroup puts aside
 constexpr int kShareList = 128;   // entries up to which a tile's list counts as short
 constexpr int kShareBlocks = 4;       // blocks over which a record of a short list is put aside
 constexpr int kShareBlocksLong = 44;  // and of a long one
@@ -1500,14 +1500,14 @@ __device__ __forceinline__ void raster_round(const MeshView& mesh, const MvpSour
     if (self) raster_rect_self<RS, kVis>(s, t, g.x0, g.y0, rx0, rx1, ry0, ry1, tile);
 }
 
-// The records with a long edge among the n of the queue, each by the whole
-// workgroup with the 64-bit edge functions.
+// The records of the queue whose bit is set in `which` (wave-uniform, the same
+// in all waves), each by the whole workgroup with the 64-bit edge functions.
 template <int RS, bool kVis>
-__device__ __forceinline__ void raster_queued_long(const Region& g, const Setup* rec, int n,
+__device__ __forceinline__ void raster_queued_long(const Region& g, const Setup* rec, unsigned which,
                                                    typename KeyOf<kVis>::T* tile) {
-    for (int q = 0; q < n; ++q) {
-        if (!(rec[q].tl & kLongEdge)) continue;  // uniform
-        const Setup r = rec[q];
+    while (which) {
+        const Setup r = rec[__ffs((int)which) - 1];
+        which &= which - 1;
         raster_rect_slow<RS, kVis>(r, g.x0, g.y0, max(g.x0, r.px0), min(g.x1, r.px1), max(g.y0, r.py0),
                                    min(g.y1, r.py1), (int)threadIdx.x, kRasterThreads, tile);
     }
@@ -1540,7 +1540,7 @@ __device__ __forceinline__ void raster_long(const MeshView& mesh, const MvpSourc
             }
             __syncthreads();
             n = nrec;
-            raster_queued_long<RS, kVis>(g, rec, min(n, kRecQueue), tile);
+            raster_queued_long<RS, kVis>(g, rec, (1u << min(n, kRecQueue)) - 1u, tile);
         }
     }
     __syncthreads();
@@ -1584,7 +1584,7 @@ __device__ __forceinline__ void finish_region(const MeshView& mesh, const MvpSou
                                            max(g.y0, s.py0) - g.y0, min(g.y1, s.py1) - g.y0);
         }
         raster_lanes<RS, kVis, true>(s, t, blocks, has && blocks && !(s.tl & kLongEdge), g.x0, g.y0, lane, z.zmax, z.age, tile);
-        raster_queued_long<RS, kVis>(g, rec, nq, tile);
+        raster_queued_long<RS, kVis>(g, rec, (unsigned)__ballot(has && (s.tl & kLongEdge)), tile);
         __syncthreads();
     }
     if (more_long) raster_long<TS, RS, kVis, kFallback>(mesh, mvps, cfg, b, map, g, begin, end, tile, rec, nrec);  // uniform
