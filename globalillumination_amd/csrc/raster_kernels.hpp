@@ -1701,15 +1701,17 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
 // are long beside the launch's average (split_bound); each is rasterized in 16
 // regions of 16x16 pixels by workgroups of their own.  A region's workgroup
 // goes through the tile's whole list, but reads only each record's box (its
-// first 16 bytes, kSplitLoads in flight per thread), and rasterizes the
-// entries that touch the region from a list in LDS.  Raster of one map, tiles
-// only and with split lists: 200k soup, 2048^2: 130 and 47 us (its G-buffer at
-// 1920x1080: 232 and 67 us); 100,822 triangles seen from 315 units, 2048^2: 98
-// and 43 us; a 3,970-triangle scene, 1024^2: 43 and 17 us, 256^2: 26 and 13 us.
+// first 16 bytes, kBoxes in flight per thread), and rasterizes the entries that
+// touch the region from a list in LDS.  Raster of one map, tiles only and with
+// split lists: 200k soup, 2048^2: 130 and 46 us (its G-buffer at 1920x1080: 232
+// and 67 us); 100,822 triangles seen from 315 units, 2048^2: 98 and 32 us (42
+// with a box at a time); a 3,970-triangle scene, 1024^2: 43 and 17 us, 256^2: 26
+// and 13 us.  Eight boxes at a time spill registers (the soup 50 us).
 // ---------------------------------------------------------------------------
 constexpr int kSplitEdge = 16;
 constexpr int kSplitRegions = (kTile / kSplitEdge) * (kTile / kSplitEdge);
 constexpr int kSplitLoads = 8;                              // entries per thread and pass over the list
+constexpr int kBoxes = 4;                                   // of them whose boxes are read together
 constexpr int kSplitPass = kSplitLoads * kRasterThreads;    // entries a pass looks at, and its LDS list's size
 
 // The region list in LDS, behind the region's pixels in the tile's memory.
@@ -1733,6 +1735,8 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
     const uint32_t begin = b.offsets[(size_t)map * (ntiles + 1) + tile_id];
     const uint32_t end = b.offsets[(size_t)map * (ntiles + 1) + tile_id + 1];
     const uint32_t* entries = b.entries + (size_t)map * b.cap;
+    const char* boxes = reinterpret_cast<const char*>(b.wide + (size_t)map * b.wcap) + offsetof(Setup, px0);
+    const char* recs = reinterpret_cast<const char*>(b.setups + (size_t)map * b.tstride);
     uint32_t* list = split_list<TS, kVis>(tile);
     clear_region<RS, kVis>(tile, nrec);
     ZBound z{0xFFFFFFFFu, 0};
@@ -1745,26 +1749,35 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
             const uint32_t k = base + (uint32_t)(q * kRasterThreads + tid);
             e[q] = k < end ? entries[k] : ~0u;
         }
+        // a wide record's box, or the first 16 bytes of a direct one: one load
+        // from either address (behind a branch each would wait for the one
+        // before it), kBoxes in flight together
+        typedef int quad __attribute__((ext_vector_type(4), aligned(8)));
+        static_assert(kSplitLoads % kBoxes == 0, "whole groups");
         bool hit[kSplitLoads];
 #pragma unroll
-        for (int q = 0; q < kSplitLoads; ++q) {
-            hit[q] = false;
-            if (e[q] == ~0u) continue;
-            int px0, px1, py0, py1;
-            if (e[q] & kWideBit) {
-                const Setup& w = b.wide[(size_t)map * b.wcap + (e[q] & ~kWideBit)];
-                px0 = w.px0;
-                px1 = w.px1;
-                py0 = w.py0;
-                py1 = w.py1;
-            } else {
-                const size_t at = (size_t)map * b.tstride + (e[q] >> 3);
-                const SetupRec& r = b.setups[at];
-                int X[3], Y[3];
-                rec_vertices(r.X0, r.Y0, r.d1, r.d2, b.fars[at], X, Y);
-                rec_box(X, Y, px0, px1, py0, py1);
+        for (int q0 = 0; q0 < kSplitLoads; q0 += kBoxes) {
+            quad v[kBoxes];
+#pragma unroll
+            for (int i = 0; i < kBoxes; ++i) {
+                const uint32_t en = e[q0 + i];
+                const bool wide = (en & kWideBit) != 0;
+                const uint32_t idx = en == ~0u ? 0u : wide ? en & ~kWideBit : en >> 3;
+                const uint32_t size = wide ? (uint32_t)sizeof(Setup) : (uint32_t)sizeof(SetupRec);
+                v[i] = *reinterpret_cast<const quad*>((wide ? boxes : recs) + (size_t)idx * size);
             }
-            hit[q] = px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0;
+#pragma unroll
+            for (int i = 0; i < kBoxes; ++i) {
+                const uint32_t en = e[q0 + i];
+                int px0 = v[i].x, px1 = v[i].y, py0 = v[i].z, py1 = v[i].w;
+                if (!(en & kWideBit)) {
+                    int X[3], Y[3];
+                    rec_vertices(v[i].x, v[i].y, (uint32_t)v[i].z, (uint32_t)v[i].w,
+                                 b.fars[(size_t)map * b.tstride + (en >> 3)], X, Y);
+                    rec_box(X, Y, px0, px1, py0, py1);
+                }
+                hit[q0 + i] = en != ~0u && px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0;
+            }
         }
 #pragma unroll
         for (int q = 0; q < kSplitLoads; ++q)
@@ -1808,9 +1821,8 @@ __global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 8) void k_raster(MeshVie
 // take the other regions in turn.
 constexpr int kSplitWorkers = 1024;
 template <int TS, bool kVis>
-__global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 6) void k_raster_split(MeshView mesh, MvpSource mvps,
-                                                                               RasterCfg cfg, BinBufs b, void* out,
-                                                                               int map_base, int map_count) {
+__global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, MvpSource mvps, RasterCfg cfg,
+                                                                 BinBufs b, void* out, int map_base, int map_count) {
     __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec, nlist;
