@@ -1704,14 +1704,15 @@ __device__ __forceinline__ void raster_tile(const MeshView& mesh, const MvpSourc
 // first 16 bytes, kBoxes in flight per thread), and rasterizes the entries that
 // touch the region from a list in LDS.  Raster of one map, tiles only and with
 // split lists: 200k soup, 2048^2: 130 and 46 us (its G-buffer at 1920x1080: 232
-// and 67 us); 100,822 triangles seen from 315 units, 2048^2: 98 and 32 us (42
+// and 67 us); 100,822 triangles seen from 315 units, 2048^2: 98 and 34 us (42
 // with a box at a time); a 3,970-triangle scene, 1024^2: 43 and 17 us, 256^2: 26
-// and 13 us.  Eight boxes at a time spill registers (the soup 50 us).
+// and 13 us.
 // ---------------------------------------------------------------------------
 constexpr int kSplitEdge = 16;
 constexpr int kSplitRegions = (kTile / kSplitEdge) * (kTile / kSplitEdge);
 constexpr int kSplitLoads = 8;                              // entries per thread and pass over the list
 constexpr int kBoxes = 4;                                   // of them whose boxes are read together
+static_assert(kSplitLoads % kBoxes == 0, "a pass is whole groups of boxes");
 constexpr int kSplitPass = kSplitLoads * kRasterThreads;    // entries a pass looks at, and its LDS list's size
 
 // The region list in LDS, behind the region's pixels in the tile's memory.
@@ -1743,45 +1744,40 @@ __device__ __forceinline__ void raster_region(const MeshView& mesh, const MvpSou
     for (uint32_t base = begin; base < end; base += kSplitPass) {
         if (tid == 0) nlist = 0;
         __syncthreads();  // also: the region is cleared, the last pass's list is done with
-        uint32_t e[kSplitLoads];
-#pragma unroll
-        for (int q = 0; q < kSplitLoads; ++q) {
-            const uint32_t k = base + (uint32_t)(q * kRasterThreads + tid);
-            e[q] = k < end ? entries[k] : ~0u;
-        }
         // a wide record's box, or the first 16 bytes of a direct one: one load
         // from either address (behind a branch each would wait for the one
-        // before it), kBoxes in flight together
+        // before it), kBoxes in flight together.  Holding all of a pass takes 95
+        // registers, so 5 workgroups per CU instead of 6: the far map above 32
+        // us, but a soup over the whole of a 2048^2 map 121 us instead of 116.
         typedef int quad __attribute__((ext_vector_type(4), aligned(8)));
-        static_assert(kSplitLoads % kBoxes == 0, "whole groups");
-        bool hit[kSplitLoads];
-#pragma unroll
-        for (int q0 = 0; q0 < kSplitLoads; q0 += kBoxes) {
+        for (uint32_t b0 = base; b0 < min(base + kSplitPass, end); b0 += kBoxes * kRasterThreads) {  // uniform
+            uint32_t e[kBoxes];
             quad v[kBoxes];
 #pragma unroll
-            for (int i = 0; i < kBoxes; ++i) {
-                const uint32_t en = e[q0 + i];
-                const bool wide = (en & kWideBit) != 0;
-                const uint32_t idx = en == ~0u ? 0u : wide ? en & ~kWideBit : en >> 3;
-                const uint32_t size = wide ? (uint32_t)sizeof(Setup) : (uint32_t)sizeof(SetupRec);
-                v[i] = *reinterpret_cast<const quad*>((wide ? boxes : recs) + (size_t)idx * size);
+            for (int q = 0; q < kBoxes; ++q) {
+                const uint32_t k = b0 + (uint32_t)(q * kRasterThreads + tid);
+                e[q] = k < end ? entries[k] : ~0u;
             }
 #pragma unroll
-            for (int i = 0; i < kBoxes; ++i) {
-                const uint32_t en = e[q0 + i];
-                int px0 = v[i].x, px1 = v[i].y, py0 = v[i].z, py1 = v[i].w;
-                if (!(en & kWideBit)) {
+            for (int q = 0; q < kBoxes; ++q) {
+                const bool wide = (e[q] & kWideBit) != 0;
+                const uint32_t idx = e[q] == ~0u ? 0u : wide ? e[q] & ~kWideBit : e[q] >> 3;
+                const uint32_t size = wide ? (uint32_t)sizeof(Setup) : (uint32_t)sizeof(SetupRec);
+                v[q] = *reinterpret_cast<const quad*>((wide ? boxes : recs) + (size_t)idx * size);
+            }
+#pragma unroll
+            for (int q = 0; q < kBoxes; ++q) {
+                int px0 = v[q].x, px1 = v[q].y, py0 = v[q].z, py1 = v[q].w;
+                if (!(e[q] & kWideBit)) {
                     int X[3], Y[3];
-                    rec_vertices(v[i].x, v[i].y, (uint32_t)v[i].z, (uint32_t)v[i].w,
-                                 b.fars[(size_t)map * b.tstride + (en >> 3)], X, Y);
+                    rec_vertices(v[q].x, v[q].y, (uint32_t)v[q].z, (uint32_t)v[q].w,
+                                 b.fars[(size_t)map * b.tstride + (e[q] >> 3)], X, Y);
                     rec_box(X, Y, px0, px1, py0, py1);
                 }
-                hit[q0 + i] = en != ~0u && px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0;
+                if (e[q] != ~0u && px0 <= g.x1 && px1 >= g.x0 && py0 <= g.y1 && py1 >= g.y0)
+                    list[atomicAdd(&nlist, 1)] = e[q];
             }
         }
-#pragma unroll
-        for (int q = 0; q < kSplitLoads; ++q)
-            if (hit[q]) list[atomicAdd(&nlist, 1)] = e[q];
         __syncthreads();
         const int n = nlist;
         for (int k0 = 0; k0 < n; k0 += kRasterThreads) {
@@ -1821,8 +1817,9 @@ __global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 8) void k_raster(MeshVie
 // take the other regions in turn.
 constexpr int kSplitWorkers = 1024;
 template <int TS, bool kVis>
-__global__ __launch_bounds__(kRasterThreads) void k_raster_split(MeshView mesh, MvpSource mvps, RasterCfg cfg,
-                                                                 BinBufs b, void* out, int map_base, int map_count) {
+__global__ __launch_bounds__(kRasterThreads, kVis ? 1 : 6) void k_raster_split(MeshView mesh, MvpSource mvps,
+                                                                               RasterCfg cfg, BinBufs b, void* out,
+                                                                               int map_base, int map_count) {
     __shared__ __align__(16) typename KeyOf<kVis>::T tile[TS * tile_pitch<TS>()];
     __shared__ Setup rec[kRecQueue];
     __shared__ int nrec, nlist;
