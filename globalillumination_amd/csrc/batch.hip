@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kScanThreads) void kb_scan(RasterTable t) {
         const int j = find_job(pre, t.njobs, item);
         const RasterJob& J = t.jobs[j];
         const int map = (int)(item - pre[j]);
-        scan_body(J.b, J.ntiles, map, 0);
+        scan_body(J.b, J.ntiles, map, 0, 1u);
         // the thread that decided the map's overflow raises the batch's flag
         // (kb_raster_fallback does nothing without it)
         if (threadIdx.x == kScanThreads - 1 && J.b.overflow[map]) t.counter[0] = 1u;

@@ -54,13 +54,53 @@ namespace {
 constexpr size_t kSpreadTiles = 2048;
 
 // Whether a depth pass of nmaps maps splits long tile lists (k_raster_split):
-// while its tiles are few enough (six per resident workgroup) that a long list
-// can outlast the rest: nine 2048^2 maps of a far mesh took 118 us without and
-// 98 us with, while with 64 maps of 2048^2 every CU has 250 tiles to draw from.
+// where its long lists are few beside what the GPU holds.  The maps of a pass
+// show one mesh, so each brings long lists of its own, and from some number of
+// maps on they fill the GPU without being split, while k_raster_split keeps 6
+// workgroups per CU where k_raster keeps 8, and its regions read each list 16
+// times.  Depth passes with and without splitting, us (a 32,002- and a
+// 98,002-triangle body, soups of 50,000 and 200,000):
+//   maps            tiles     body        body        soup        soup
+//   1 of 512^2         64   48   77     69  126     54   97    105  259
+//   4 of 512^2        256   55   79     79  136     99  104    203  279
+//   8 of 350^2        288   69  108     99  159    107  119    288  354
+//   9 of 512^2        576   64   88    101  145    115  113    303  297
+//   16 of 256^2       256   74   87    114  106    131  132    533  406
+//   16 of 512^2     1,024   84   94    161  158    120  117    336  327
+//   25 of 512^2     1,600  106   98    241  168    148  143    414  389
+//   9 of 1024^2     2,304   77   73    112  103    152  144    331  343
+//   64 of 256^2     1,024  153  110    282  166    178  169    580  568
+//   64 of 512^2     4,096  148  132    274  249    284  273    860  808
+// Five to eight maps of 900^2 to 1800^2 take 1% more to 8% less without, in the
+// mean of seven meshes (19% more to 21% less with one), and stay split.
+// Few maps split, some more while their tiles are few, and large ones, whose one
+// long list stands against 1,024 tiles: nine 2048^2 maps of a far mesh take 118
+// us without and 98 with, of the first body over the whole map 93 and 98.
 constexpr size_t kSplitTiles = 12288;
-constexpr int kSplitMaps = 64;  // its workers hold a map's task count per lane
+constexpr int kSplitFew = 8;
+constexpr int kSplitSome = 16;
+constexpr size_t kSplitSomeTiles = 1024;
+constexpr int kSplitLarge = 1024;  // tiles of a map
+static_assert(kSplitTiles / kSplitLarge <= 64 && kSplitSome <= 64, "the workers hold a map's task count per lane");
 bool splits_lists(int ntiles, int nmaps) {
-    return nmaps <= kSplitMaps && (size_t)ntiles * nmaps <= kSplitTiles;
+    const size_t tiles = (size_t)ntiles * nmaps;
+    return tiles <= kSplitTiles &&
+           (nmaps <= kSplitFew || (nmaps <= kSplitSome && tiles <= kSplitSomeTiles) || ntiles >= kSplitLarge);
+}
+
+// Into how many shares a launch of `tiles` tiles is thought to be cut, a list
+// longer than one being split (split_bound): a share per CU, or smaller ones
+// while the tiles leave the GPU room.  Depth passes with 1,024, 512 and 256, us:
+// one 512^2 map (64 tiles) of a 50,000-triangle soup 55, -, 80, of a 200,000-
+// triangle soup 105, -, 148; one 2048^2 map (1,024 tiles) of these 113, 96, 96
+// and 228, 189, 186; three of 900^2 (675) of a 4,830-triangle scene 55, 55, 63.
+// More tiles: one 4096^2 map of 100,822 triangles 58 with 1,024, 48 with 256.  A
+// CU holds 4 workgroups of a visibility pass: 510 tiles of a 200,000-triangle
+// soup's G-buffer 67 us with 1,024, 83 with 256 (the raster alone); 4,096 tiles of
+// 16 maps of 50,002 triangles 235 and 138.
+template <bool kVis>
+uint32_t split_shares(size_t tiles) {
+    return tiles <= 256 ? 1024u : tiles <= 1024 ? (kVis ? 1024u : 512u) : 256u;
 }
 
 // Binning of every map (count, clip, scan, scatter) and the raster of the
@@ -85,7 +125,8 @@ int bin_stage(const MeshView& mesh, const MvpSource& mvps, int nmaps, const Rast
         hipLaunchKernelGGL((k_bin_wide<kTile, false>), gw, dim3(256), 0, s, cfg, b);
     }
     hipLaunchKernelGGL(k_scan, dim3(nmaps), dim3(kScanThreads), 0, s, b, ntiles,
-                       splits_lists(ntiles, nmaps) ? nmaps : 0);
+                       splits_lists(ntiles, nmaps) ? nmaps : 0,
+                       split_shares<kVis>((size_t)ntiles * nmaps));
     if (mesh.nt > 0) {
         if constexpr (wide_span<kTile>() <= 4) {
             // triangles' appends and the wide records' appends in one launch

@@ -969,18 +969,11 @@ __device__ __forceinline__ uint32_t* split_tiles(const BinBufs& b, int map) {
 }
 
 // Entries from which a tile's list is split, for a launch of `nmaps` maps like
-// one with `total` entries in `ntiles` tiles: a CU's even share of the launch,
-// and no less than kSplitMin, below which the 16 passes over the list cost more
-// than they spread.  A quarter of that share splits lists whose tiles fill the
-// GPU anyway: 16 visibility maps of 1024^2 (50,002 triangles, 4,096 tiles) 235 us
-// against 138 us, one 4096^2 map (100,822 triangles) 58 against 48 us.  Launches
-// of at most 1,024 tiles, four a CU, do not fill it, and take the quarter: the
-// 510 tiles of a 200k-triangle soup's G-buffer 67 us, 83 with the whole share;
-// single maps of 16 to 1,024 tiles with few long lists are the same with both.
+// one with `total` entries: one of `shares` even shares of the launch
+// (split_shares), and no less than kSplitMin, below which the 16 passes over the
+// list cost more than they spread.
 constexpr uint32_t kSplitMin = 48;
-constexpr int kSplitRoomy = 1024;
-__device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nmaps, int ntiles) {
-    const unsigned long long shares = (long long)ntiles * nmaps <= kSplitRoomy ? 1024ull : 256ull;
+__device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nmaps, uint32_t shares) {
     const unsigned long long even = total * (unsigned)nmaps / shares;
     return even > kSplitMin ? (uint32_t)min(even, 0x7FFFFFFFull) : kSplitMin;
 }
@@ -990,7 +983,7 @@ __device__ __forceinline__ uint32_t split_bound(unsigned long long total, int nm
 // launches that split long lists (split_maps > 0), lists those.  A chain of loads
 // and sums in one workgroup: 2.9 us for 256 tiles with the sums by lane
 // exchanges and 16 wave totals, 3.6 with ten rounds of LDS between barriers.
-__device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map, int split_maps) {
+__device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map, int split_maps, uint32_t shares) {
     __shared__ unsigned long long wave_sum[kScanThreads / 64];
     __shared__ uint32_t nsplit;
     uint32_t* c = b.counts + (size_t)map * ntiles;
@@ -1016,7 +1009,7 @@ __device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map,
         run += k < wave ? wave_sum[k] : 0ull;
         total += wave_sum[k];
     }
-    const uint32_t bound = split_maps > 0 ? split_bound(total, split_maps, ntiles) : 0u;
+    const uint32_t bound = split_maps > 0 ? split_bound(total, split_maps, shares) : 0u;
     uint32_t* split = split_tiles(b, map);
     for (int i = lo; i < hi; ++i) {
         o[i] = (uint32_t)run;
@@ -1043,8 +1036,8 @@ __device__ __forceinline__ void scan_body(const BinBufs& b, int ntiles, int map,
     }
 }
 
-__global__ __launch_bounds__(kScanThreads) void k_scan(BinBufs b, int ntiles, int split_maps) {
-    scan_body(b, ntiles, blockIdx.x, split_maps);
+__global__ __launch_bounds__(kScanThreads) void k_scan(BinBufs b, int ntiles, int split_maps, uint32_t shares) {
+    scan_body(b, ntiles, blockIdx.x, split_maps, shares);
 }
 
 // ---------------------------------------------------------------------------
