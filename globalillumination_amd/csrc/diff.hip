@@ -264,26 +264,32 @@ __device__ __forceinline__ double texel_depth(const TexelPlane* __restrict__ pl,
     return p.d0 + (p.A * (double)(a - p.x0) + p.B * (double)(b - p.y0));
 }
 
-// A pixel's mean over the maps.  Bound by the gathers of keys and records: 16
-// maps of 1024^2 under a 512^2 view 60 us (132 us with a pass that stored every
-// texel's depth before it; fetching the next map's keys ahead changes nothing).
+// A pixel's mean over the maps.  Bound by the gathers of keys and records, a
+// chain of two per map: 16 maps of 1024^2 under a 512^2 view 60 us with a thread
+// per pixel (132 us with a pass that stored every texel's depth before it;
+// fetching the next map's keys ahead changes nothing).  Walking all the maps, a
+// thread of a small view has few other waves to hide them: 64 maps of 128^2
+// under 128x96 pixels 185 us (86 us with stored depths), so kParts threads share
+// a pixel's maps.  The forward pass with 64 maps of 256^2 (2,882 triangles): 126
+// against 264 us under 128x96 pixels, 145 against 262 under 400x300, 387 against
+// 446 under 1280x720.
+template <int kParts>
 __global__ __launch_bounds__(kThreads) void k_diff_shade(const float* __restrict__ gpos,
                                                          const double* __restrict__ biased,
                                                          const unsigned long long* __restrict__ vis,
                                                          const TexelPlane* __restrict__ planes, int ntris, DiffCfg c,
                                                          float* __restrict__ out) {
+    constexpr int kPixels = kThreads / kParts;
+    static_assert(kPixels % 64 == 0, "a wave's lanes walk the same maps");
     const size_t plane = (size_t)c.gw * c.gh;
-    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= plane) return;
-    const float xf = gpos[k];
-    if (xf == 0.0f) {
-        out[k] = 0.0f;
-        return;
-    }
-    const double x = xf, y = gpos[plane + k], z = gpos[2 * plane + k];
+    const size_t k = (size_t)blockIdx.x * kPixels + threadIdx.x % kPixels;
+    const int part = (int)threadIdx.x / kPixels;
+    const float xf = k < plane ? gpos[k] : 0.0f;
+    const bool lit = xf != 0.0f;
+    const double x = xf, y = lit ? gpos[plane + k] : 0.0, z = lit ? gpos[2 * plane + k] : 0.0;
     const size_t msz = (size_t)c.smw * c.smh;
     double acc = 0.0;
-    for (int i = 0; i < c.S; ++i) {
+    for (int i = lit ? part : c.S; i < c.S; i += kParts) {
         double m[16];
         load_m(biased + 16 * i, m);
         const Tap t = project(m, x, y, z, c);
@@ -301,7 +307,23 @@ __global__ __launch_bounds__(kThreads) void k_diff_shade(const float* __restrict
                      sigmoid_d((texel_depth(pl, tri[2 * db + da], t.a0 + da, t.b0 + db) - t.z + c.bias) / c.tau);
         acc += c.si + (1.0 - c.si) * q;
     }
-    out[k] = (float)(acc / (double)c.S);
+    if constexpr (kParts > 1) {
+        __shared__ double sums[kParts][kPixels];
+        sums[part][threadIdx.x % kPixels] = acc;
+        __syncthreads();
+        acc = 0.0;
+        for (int p = 0; p < kParts; ++p) acc += sums[p][threadIdx.x % kPixels];
+    }
+    if (part == 0 && k < plane) out[k] = lit ? (float)(acc / (double)c.S) : 0.0f;
+}
+
+// Threads per pixel: four from eight maps on, and from four on while the pixels
+// do not fill the GPU by themselves (the forward pass with four maps of 256^2: 51
+// us with, 57 without under 256x256 pixels, 62 and 63 under 800x600, 72 and 70
+// under 1280x720).
+constexpr int kShadeParts = 4;
+inline int shade_parts(int px_blocks, int S) {
+    return S >= 2 * kShadeParts || (S >= kShadeParts && px_blocks <= 2048) ? kShadeParts : 1;
 }
 
 // x + y with the halves of the wave transposed: lanes 0-31 get x's sum over
@@ -865,8 +887,14 @@ int gi_diff_soft_forward(const float* positions_dev, int nverts, const int32_t* 
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     rc = recompute(positions_dev, nverts, indices_dev, ntris, mvps_dev, c, w, s, false);
     if (rc != GI_OK) return rc;
-    hipLaunchKernelGGL(k_diff_shade, dim3(w.px_blocks), dim3(kThreads), 0, s, gbuffer->position_dev, biased_mvps_dev,
-                       w.vis, w.texels, ntris, c, out_dev);
+    const size_t pixels = (size_t)c.gw * c.gh;
+    if (shade_parts(w.px_blocks, nsamples) > 1)
+        hipLaunchKernelGGL(k_diff_shade<kShadeParts>, dim3((unsigned)((pixels * kShadeParts + kThreads - 1) / kThreads)),
+                           dim3(kThreads), 0, s, gbuffer->position_dev, biased_mvps_dev, w.vis, w.texels, ntris, c,
+                           out_dev);
+    else
+        hipLaunchKernelGGL(k_diff_shade<1>, dim3(w.px_blocks), dim3(kThreads), 0, s, gbuffer->position_dev,
+                           biased_mvps_dev, w.vis, w.texels, ntris, c, out_dev);
     return hipGetLastError() == hipSuccess ? GI_OK : GI_EDEVICE;
 }
 

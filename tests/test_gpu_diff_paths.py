@@ -49,6 +49,16 @@ def test_two_maps_a_thread(gi, oracle_lib, cuda):
     _check(_Sized(gi, oracle_lib, 97, (40, 30), 54, samples=9), 9)
 
 
+@pytest.mark.parametrize("samples,view", [(1, (65, 3)), (4, (1, 1)), (4, (64, 2)), (9, (65, 3)), (16, (33, 17)),
+                                          (25, (130, 5))])
+def test_pixels_shared_by_threads(gi, oracle_lib, cuda, samples, view):
+    """A pixel's maps walked by one thread and by four, in equal and unequal
+    shares, in views of one, of whole and of odd blocks of 64 pixels.  The FP64
+    sums differ in their order only: the forward pass's bar."""
+    st = _Sized(gi, oracle_lib, 65, view, 4, samples=samples)
+    assert np.abs(st.gpu_forward(st.L, st.r) - st.oracle_forward(st.L, st.r)).max() <= 1e-6
+
+
 def _check(st, seed):
     got, want = st.gpu_forward(st.L, st.r), st.oracle_forward(st.L, st.r)
     assert np.abs(got - want).max() <= 1e-6
