@@ -64,6 +64,8 @@ def _upload(arr: np.ndarray, device, stream=None) -> torch.Tensor:
     if dev.type != "cuda":
         return t.to(device)
     if stream is not None and stream != torch.cuda.current_stream():
+        if not isinstance(stream, torch.cuda.Stream):  # whatever has a cuda_stream, as the passes take it
+            stream = torch.cuda.ExternalStream(stream.cuda_stream, device=dev)
         with torch.cuda.stream(stream):
             if not torch.cuda.is_current_stream_capturing():
                 return _upload(arr, device)

@@ -79,10 +79,14 @@ def test_host_matrices_may_change_after_the_call(gi, cuda, side_stream):
 
 
 @pytest.mark.gpu
-def test_uploads_of_calls_on_another_stream(gi, cuda):
+@pytest.mark.parametrize("wrapped", [False, True])
+def test_uploads_of_calls_on_another_stream(gi, cuda, wrapped):
     """Passes on a stream that is not torch's current one, several in a row
     with other matrices each, behind work that is still running there: each
-    reads its own, though the tensors of the calls before have been dropped."""
+    reads its own, though the tensors of the calls before have been dropped.
+    Also with an object that only names the stream's handle."""
+    import types
+
     import torch
 
     wl = gi.scenes.config3(nsamples=4, view_w=64, view_h=64, sm=256, freq=20)
@@ -105,8 +109,9 @@ def test_uploads_of_calls_on_another_stream(gi, cuda):
         for _ in range(20):
             a = a @ a * 1e-3
     for k, (m, (maps, out)) in enumerate(zip(frames, outs)):
-        gi.render_shadow_map(dm, m, 256, 256, out=maps, stream=stream)
-        gi.render_monte_carlo(g, maps, m, soft, zbias=0.01 * k, out=out, stream=stream)
+        handle = types.SimpleNamespace(cuda_stream=stream.cuda_stream) if wrapped else stream
+        gi.render_shadow_map(dm, m, 256, 256, out=maps, stream=handle)
+        gi.render_monte_carlo(g, maps, m, soft, zbias=0.01 * k, out=out, stream=handle)
     stream.synchronize()
     for (maps, out), (wm, wo) in zip(outs, want):
         assert torch.equal(maps.view(torch.int32), wm.view(torch.int32))
