@@ -72,12 +72,13 @@ constexpr size_t kSpreadTiles = 2048;
 //   64 of 256^2     1,024  153  110    282  166    178  169    580  568
 //   64 of 512^2     4,096  148  132    274  249    284  273    860  808
 // Five to eight maps of 900^2 to 1800^2 take 1% more to 8% less without, in the
-// mean of seven meshes (19% more to 21% less with one), and stay split.
+// mean of seven meshes (19% more to 21% less with one), and stay split, and so do
+// the nine corner maps of an adaptive frame, whose light stands further away (maps
+// of 1721^2, 38,722 triangles, the whole frame: 391 us with, 426 without).
 // Few maps split, some more while their tiles are few, and large ones, whose one
-// long list stands against 1,024 tiles: nine 2048^2 maps of a far mesh take 118
-// us without and 98 with, of the first body over the whole map 93 and 98.
+// long list stands against 1,024 tiles or more.
 constexpr size_t kSplitTiles = 12288;
-constexpr int kSplitFew = 8;
+constexpr int kSplitFew = 9;
 constexpr int kSplitSome = 16;
 constexpr size_t kSplitSomeTiles = 1024;
 constexpr int kSplitLarge = 1024;  // tiles of a map

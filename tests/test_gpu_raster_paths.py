@@ -268,7 +268,7 @@ def test_fallback_by_triangle_count(gi, oracle_lib, cuda, n):
 
 @pytest.mark.parametrize("w,h,maps,ranges", [(512, 512, 5, [(0, 2), (2, 2), (4, 1)]), (2048, 128, 64, [(63, 1), (0, 40), (40, 23)]),
                                              (512, 512, 66, [(0, 1), (1, 64), (65, 1)]), (256, 256, 16, [(0, 16)]),
-                                             (256, 256, 17, [(0, 9), (9, 8)]), (576, 512, 8, [(0, 8)]), (576, 512, 15, [(0, 15)])])
+                                             (256, 256, 17, [(0, 9), (9, 8)]), (576, 512, 9, [(0, 9)]), (576, 512, 10, [(0, 10)]), (576, 512, 15, [(0, 15)])])
 def test_ranges_of_maps_with_long_lists(gi, oracle_lib, cuda, w, h, maps, ranges):
     """The raster of a range of maps at a time, of launches that split long
     lists and that do not, around the numbers of maps and tiles up to which they
